@@ -10,14 +10,15 @@
 // written a plan record for this batch shape. The optional lse output is the base-2 log-sum-exp of the scaled scores,
 // log2(sum_j 2^(s_j * log2 e)), which is the convention of the FlashInfer kernels the reference wraps.
 //
-// Decode (mode DECODE) -- HBM bound (DecodeKernel, DecodeMergeKernel):
+// Decode (mode DECODE) -- HBM bound (DecodeMfmaKernel in bf16, DecodeF32Kernel, DecodeMergeKernel):
 //   * plan() deals the batch's 16-token groups out evenly to one range per resident workgroup slot and cuts sequences
 //     at range boundaries (so the variant is DETERMINISTIC but not BATCH_INVARIANT); a workgroup serves the KV heads
 //     of its range, its wavefronts take alternate groups;
-//   * K and V rows are loaded branch-free into a register double buffer (the next group in flight while the current
-//     one is computed), each K/V byte once, shared by the query heads of the GQA group;
-//   * bf16: q.k on v_mfma_f32_16x16x32_bf16 (tokens on M, the group's query heads on N), P.V on v_dot2 with P rounded
-//     to bf16; f32: q.k as VALU products reduce-scattered across the lanes of a row;
+//   * bf16: a wavefront serves all the query heads of a KV head (up to 16), each K/V byte requested once; K and V rows are
+//     loaded branch-free into one register buffer each, the next group's K in flight from the moment the scores have
+//     read this one's; q.k on v_mfma_f32_16x16x32_bf16 (tokens on M, heads on N), P.V on v_mfma_f32_16x16x16_bf16 with P
+//     rounded to bf16 and fp32 accumulation;
+//   * f32: groups of 4 heads, a register double buffer, q.k as VALU products reduce-scattered across the lanes of a row;
 //   * the wavefronts merge through LDS; a sequence cut into pieces writes fp32 partials (o, m, l) that
 //     DecodeMergeKernel combines in key order.
 // Prefill (mode PREFILL) -- MFMA bound (PrefillTileKernel + PrefillMergeKernel for page sizes that are powers of two
@@ -28,8 +29,8 @@
 //     query live in one lane pair; P is rounded to bf16 before the P.V product (as FlashAttention-2 does);
 //   * plan() cuts items longer than the average CU load into pieces (bf16 partials merged in key order) and orders the
 //     work longest-first so the ragged causal tail does not set the makespan;
-//   * single-token sequences of a prefill call run on the decode kernels, beside the tile kernel on the context's
-//     second stream when plan() finds that cheaper (ChooseOverlap); an f32 prefill runs every query token as a row of
+//   * single-token sequences of a prefill call run on the decode kernels, in one launch with the tile kernel when plan()
+//     finds that cheaper (ChooseOverlap); an f32 prefill runs every query token as a row of
 //     the f32 decode kernel.
 // Output gate (roost_amd_paged_attention_gated_run): Qwen3.5's SigmoidMul on the attention output, applied by every
 // kernel that stores an output element (decode, both prefill kernels, both merges) to the element already rounded to
@@ -179,14 +180,22 @@ struct Layout {
 
 // ---- Admission ---------------------------------------------------------------------------------------------------
 
-// Query heads per KV head the kernels serve: groups of kGroup = 4, or 8, 16 and 32 as 2, 4 and 8 groups of 4 that read
-// the same KV rows (the reference builds 4 only).
+// Query heads per KV head the kernels serve: 4, 8, 16 and 32 (the reference builds 4 only). The prefill and f32 kernels
+// take larger groups as 2, 4 and 8 groups of kGroup = 4 that read the same KV rows.
 bool GroupBuilt(uint32_t g) { return g == 4 || g == 8 || g == 16 || g == 32; }
 // Groups of kGroup query heads ("virtual" KV heads) and the log2 of how many of them share one real KV head.
 uint32_t VirtualHeads(const RoostPagedAttentionParams& p) { return p.q_heads / kGroup; }
 uint32_t HeadShift(const RoostPagedAttentionParams& p) {
   return static_cast<uint32_t>(__builtin_ctz(p.q_heads / (p.kv_heads * kGroup)));
 }
+
+// Query heads one wavefront of the decode kernels serves: 4 in f32, the whole group of 4, 8 or 16 in bf16 (groups of 32
+// as two of 16), so that a K/V row is requested once for up to 16 heads.
+uint32_t DecodeGroupOf(const RoostPagedAttentionParams& p) {
+  return p.q.dtype == ROOST_DTYPE_F32 ? kGroup : std::min(p.q_heads / p.kv_heads, 16u);
+}
+// Groups of DecodeGroupOf query heads.
+uint32_t DecodeHeads(const RoostPagedAttentionParams& p) { return p.q_heads / DecodeGroupOf(p); }
 
 // Shapes with a kernel here, per mode: head dims 64/128/256 decode; prefill on the tile kernel at 64, 128 and 256
 // (64 and 128 need page sizes that are powers of two and multiples of 16), on the general kernel at 256.
@@ -328,8 +337,16 @@ int64_t DecodeFirstKey(int64_t kv, int32_t window) { return window < 0 ? 0 : std
 // partial slots and one DecodeMerge entry (merged by DecodeMergeKernel); a sequence without keys is one empty piece
 // that writes its zero rows.
 // The split depends on the batch, so the variant is deterministic but not batch invariant.
-// KV heads one decode workgroup serves: 4, 2 or 1, whichever divides kv_heads first.
-uint32_t HeadsPerWorkgroup(uint32_t kv_heads) { return kv_heads % 4 == 0 ? 4 : (kv_heads % 2 == 0 ? 2 : 1); }
+// (Virtual) KV heads one decode workgroup serves: the largest of 4, 2 and 1 that divides their number, up to about 1 KB
+// of an NHD token's row, which the workgroup's wavefronts then read side by side, and up to 2 where the heads lie in
+// other places (HND). Measured at 4 / 2 / 1 heads (us): 32 heads over 8 at head dim 128, NHD 107 / 112 / 123; 16 over 4 at
+// 256 109 / 105 / 105; 32 over 4 at 128, HND 110 / 107 / 105. With 8 or 16 heads per wavefront at head dim 256 one head per
+// workgroup halves the partials: 67 against 70 us at 16 heads over 2, 74 against 79 at 32 over 2 (324 MB each).
+uint32_t HeadsPerWorkgroup(const RoostPagedAttentionParams& p) {
+  const uint32_t heads = DecodeHeads(p);
+  const uint32_t most = p.head_dim == 256 ? (DecodeGroupOf(p) > kGroup ? 1 : 2) : p.kv_layout == ROOST_LAYOUT_PAGED_HND ? 2 : 4;
+  return heads % 4 == 0 && most == 4 ? 4 : (heads % 2 == 0 && most >= 2 ? 2 : 1);
+}
 
 struct DecodePlan {
   std::vector<DecodeWork> items;
@@ -363,7 +380,7 @@ DecodePlan BuildDecodeRows(const RoostPagedAttentionParams& p, uint32_t cus, con
     total += groups[r];
   }
   const uint64_t slots_wanted = std::max<uint64_t>(
-      1, static_cast<uint64_t>(cus) * kDecodeWgsPerCu / (VirtualHeads(p) / HeadsPerWorkgroup(VirtualHeads(p))));
+      1, static_cast<uint64_t>(cus) * kDecodeWgsPerCu / (DecodeHeads(p) / HeadsPerWorkgroup(p)));
   const uint64_t ranges = std::max<uint64_t>(1, std::min<uint64_t>(slots_wanted, total));
   uint64_t per_range = std::max<uint64_t>(1, roost::CeilDiv(total, ranges));
   // A row spans at most ceil(groups / per_range) + 1 pieces; keep that within what the merge kernel combines.
@@ -597,7 +614,7 @@ OverlapChoice ChooseOverlap(const RoostPagedAttentionParams& p, const Items& ite
   OverlapChoice best;
   double dec_bytes = 0.0;
   for (uint32_t b = 0; b < p.batch; ++b) {
-    if (single(b)) dec_bytes += static_cast<double>(KvLenHost(p, b)) * VirtualHeads(p) * p.head_dim * 2.0 * 2.0;
+    if (single(b)) dec_bytes += static_cast<double>(KvLenHost(p, b)) * DecodeHeads(p) * p.head_dim * 2.0 * 2.0;
   }
   if (dec_bytes == 0.0 || items.empty() || cus < 2 || p.page_size % 16 != 0) return best;
   int64_t longest = 0;
@@ -783,28 +800,11 @@ __device__ __forceinline__ uint64_t KeyRowSafe(const KvView& kv, int32_t p0, int
   return good ? row * D : 0;
 }
 
+// A float as the output type stores it.
 template <typename T>
-struct Vec;  // 16-byte vector of T, widened to float
-template <>
-struct Vec<uint16_t> {  // bf16
-  static constexpr int N = 8;
-  __device__ static void Widen(const uint4& r, float* f) {
-    f[0] = Bf16LoToF32(r.x); f[1] = Bf16HiToF32(r.x);
-    f[2] = Bf16LoToF32(r.y); f[3] = Bf16HiToF32(r.y);
-    f[4] = Bf16LoToF32(r.z); f[5] = Bf16HiToF32(r.z);
-    f[6] = Bf16LoToF32(r.w); f[7] = Bf16HiToF32(r.w);
-  }
-  __device__ static uint16_t Narrow(float x) { return F32ToBf16(x); }
-};
-template <>
-struct Vec<float> {
-  static constexpr int N = 4;
-  __device__ static void Widen(const uint4& r, float* f) {
-    f[0] = __uint_as_float(r.x); f[1] = __uint_as_float(r.y);
-    f[2] = __uint_as_float(r.z); f[3] = __uint_as_float(r.w);
-  }
-  __device__ static float Narrow(float x) { return x; }
-};
+__device__ __forceinline__ T Narrow(float x) {
+  if constexpr (sizeof(T) == 2) return F32ToBf16(x); else return x;
+}
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
@@ -839,24 +839,13 @@ __device__ __forceinline__ T GateApply(const void* gate, T g, T v) {
   return gate == nullptr ? v : GateMul(v, g);
 }
 
-// 16-byte load with the non-temporal hint, for data read exactly once in whole cache lines per instruction (decode V:
-// 2 tokens x 512 contiguous bytes per wavefront load). Keeping such a stream out of the caches raises the rate of a
-// random-16 KB-page read on the MI355X from about 5.9 to 6.8 TB/s (measured). Decode K is read 64 bytes per token per
-// instruction (the MFMA operand layout), so the other half of each 128-byte line is read by the next instruction: K
-// stays on plain loads, where that second half hits in L2.
+// 16-byte load with the non-temporal hint, for data read exactly once in whole cache lines per instruction (f32 K and V).
 __device__ __forceinline__ uint4 LoadStream16(const void* p) {
   const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
-// Partial dot product of a 16-byte K vector with the matching 16 bytes of q (both bf16; q kept as packed pairs).
-__device__ __forceinline__ float Dot16(const uint4& k, const uint32_t* q, float acc) {
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, k.x), __builtin_bit_cast(bf16x2_t, q[0]), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, k.y), __builtin_bit_cast(bf16x2_t, q[1]), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, k.z), __builtin_bit_cast(bf16x2_t, q[2]), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, k.w), __builtin_bit_cast(bf16x2_t, q[3]), acc, false);
-  return acc;
-}
+// Partial dot product of a 16-byte f32 K vector with the matching 16 bytes of q.
 __device__ __forceinline__ float Dot16(const uint4& k, const float* q, float acc) {
   acc = fmaf(__uint_as_float(k.x), q[0], acc);
   acc = fmaf(__uint_as_float(k.y), q[1], acc);
@@ -883,24 +872,23 @@ __device__ __forceinline__ float Pick4(const float* x, int i) {
   return i == 0 ? x[0] : (i == 1 ? x[1] : (i == 2 ? x[2] : x[3]));
 }
 
-// ---- Decode kernel ---------------------------------------------------------------------------------------------------
+// ---- f32 decode kernel -----------------------------------------------------------------------------------------------
 
-template <typename T, int D>
+template <int D>
 struct DecodeCfg {
-  static constexpr int kVec = Vec<T>::N;            // elements per 16-byte vector
+  static constexpr int kVec = 4;                     // floats per 16-byte vector
   static constexpr int kLpr = D / kVec;              // lanes per K/V row
   static constexpr int kTpi = 64 / kLpr;             // rows (tokens) per wave-wide load
   static constexpr int kNi = 16 / kTpi;              // loads per 16-token group per lane
-  static constexpr int kQWords = sizeof(T) == 2 ? kVec / 2 : kVec;  // q registers per head
   static_assert(kLpr <= 64 && 64 % kLpr == 0 && 16 % kTpi == 0, "shape");
   static_assert(kNi * kGroup == kLpr, "each lane must end the reduce-scatter with one (token, head) score");
 };
 
 // One wavefront's running state: acc[h][e] is this lane's slice of sum_j p_j v_j for query head h, m[h] the running
 // max of the head (wave-uniform), l_lane this lane's share of the head-(r % 4) denominator.
-template <typename T, int D>
+template <int D>
 struct DecodeState {
-  float acc[kGroup][DecodeCfg<T, D>::kVec];
+  float acc[kGroup][DecodeCfg<D>::kVec];
   float m[kGroup];
   float l_lane;
 };
@@ -913,11 +901,11 @@ struct DecodeState {
 // logical index as this lane's register j, so s[j] += partner.s[j + mk]; afterwards register 0 holds the complete score
 // of index r (slot r / 4, head r % 4). V register i holds slot i in natural order.
 // valid: bit s set when token slot s of this lane's row group is a real key.
-template <typename T, int D, typename QW>
-__device__ __forceinline__ void DecodeGroup(DecodeState<T, D>& st, const uint4* kr, const uint4* vr, uint32_t valid,
-                                            const QW (*qr)[DecodeCfg<T, D>::kQWords], float* x_row, int r, int ri,
-                                            int lane, float scale_log2, SoftCap cap) {
-  using C = DecodeCfg<T, D>;
+template <int D>
+__device__ __forceinline__ void DecodeGroup(DecodeState<D>& st, const uint4* kr, const uint4* vr, uint32_t valid,
+                                            const float (*qr)[DecodeCfg<D>::kVec], float* x_row, int r, int ri, int lane,
+                                            float scale_log2, SoftCap cap) {
+  using C = DecodeCfg<D>;
   constexpr int kVec = C::kVec, kLpr = C::kLpr, kNi = C::kNi;
   float s[kLpr];
 #pragma unroll
@@ -957,163 +945,31 @@ __device__ __forceinline__ void DecodeGroup(DecodeState<T, D>& st, const uint4* 
 #pragma unroll
       for (int e = 0; e < kVec; ++e) st.acc[h][e] *= corr[h];
   }
-  if constexpr (sizeof(T) == 2) {
-    // bf16: the weights of slots 2a and 2a+1 (lanes r and r ^ 4) travel as one packed bf16 pair per head, and P.V runs
-    // on v_dot2 over token pairs (P rounded to bf16 before the product, fp32 accumulation).
-    const float po = ShflXor(pw, 4);
-    auto* xw = reinterpret_cast<uint32_t*>(x_row);
-    if ((r & 4) == 0) xw[ri * (kLpr / 2) + (r >> 3) * kGroup + my_head] = PackBf16(pw, po);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    uint32_t pp[kNi / 2][kGroup];
+  x_row[lane] = pw;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  float pv[kLpr];
 #pragma unroll
-    for (int a = 0; a < kNi / 2; ++a) {
-      const uint4 t4 = *reinterpret_cast<const uint4*>(&xw[ri * (kLpr / 2) + a * kGroup]);
-      pp[a][0] = t4.x; pp[a][1] = t4.y; pp[a][2] = t4.z; pp[a][3] = t4.w;
-    }
-    __builtin_amdgcn_wave_barrier();
+  for (int i = 0; i < kLpr; i += 4) {
+    const float4 t4 = *reinterpret_cast<const float4*>(&x_row[ri * kLpr + i]);
+    pv[i] = t4.x; pv[i + 1] = t4.y; pv[i + 2] = t4.z; pv[i + 3] = t4.w;
+  }
+  __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int a = 0; a < kNi / 2; ++a) {
-      const uint32_t* v0 = reinterpret_cast<const uint32_t*>(&vr[2 * a]);
-      const uint32_t* v1 = reinterpret_cast<const uint32_t*>(&vr[2 * a + 1]);
+  for (int i = 0; i < kNi; ++i) {
+    const float vf[kVec] = {__uint_as_float(vr[i].x), __uint_as_float(vr[i].y), __uint_as_float(vr[i].z),
+                            __uint_as_float(vr[i].w)};
 #pragma unroll
-      for (int w = 0; w < kVec / 2; ++w) {
-        const uint32_t lo = __builtin_amdgcn_perm(v1[w], v0[w], 0x05040100u);  // (v[2a][2w], v[2a+1][2w])
-        const uint32_t hi = __builtin_amdgcn_perm(v1[w], v0[w], 0x07060302u);  // (v[2a][2w+1], v[2a+1][2w+1])
+    for (int h = 0; h < (int)kGroup; ++h) {
+      const float w = pv[i * kGroup + h];
 #pragma unroll
-        for (int h = 0; h < (int)kGroup; ++h) {
-          const bf16x2_t ph = __builtin_bit_cast(bf16x2_t, pp[a][h]);
-          st.acc[h][2 * w] = __builtin_amdgcn_fdot2_f32_bf16(ph, __builtin_bit_cast(bf16x2_t, lo), st.acc[h][2 * w], false);
-          st.acc[h][2 * w + 1] =
-              __builtin_amdgcn_fdot2_f32_bf16(ph, __builtin_bit_cast(bf16x2_t, hi), st.acc[h][2 * w + 1], false);
-        }
-      }
-    }
-  } else {
-    x_row[lane] = pw;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    float pv[kLpr];
-#pragma unroll
-    for (int i = 0; i < kLpr; i += 4) {
-      const float4 t4 = *reinterpret_cast<const float4*>(&x_row[ri * kLpr + i]);
-      pv[i] = t4.x; pv[i + 1] = t4.y; pv[i + 2] = t4.z; pv[i + 3] = t4.w;
-    }
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int i = 0; i < kNi; ++i) {
-      float vf[kVec];
-      Vec<T>::Widen(vr[i], vf);
-#pragma unroll
-      for (int h = 0; h < (int)kGroup; ++h) {
-        const float w = pv[i * kGroup + h];
-#pragma unroll
-        for (int e = 0; e < kVec; ++e) st.acc[h][e] = fmaf(w, vf[e], st.acc[h][e]);
-      }
+      for (int e = 0; e < kVec; ++e) st.acc[h][e] = fmaf(w, vf[e], st.acc[h][e]);
     }
   }
 }
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
-// bf16 form of one 16-token group. q.k runs on v_mfma_f32_16x16x32_bf16 with the 16 tokens on M and the 4 query heads
-// (padded to 16 with zero columns) on N: K register kc of lane l holds token l % 16, dims 32*kc + 8*(l / 16) .. +8,
-// q register kc the same dims of head l % 16 (zero for l % 16 >= 4), and the result lane l holds the scores of tokens
-// 4*(l / 16) + j, j = 0..3, for head l % 16. No cross-lane reduction is needed for the scores; the per-head maximum is
-// two exchanges and four readlanes, so the running maxima are wave-uniform scalars. The weights go through 256 bytes of
-// LDS into the P.V layout (lane (ri, r): V register i = token kTpi*i + ri, 16-byte slice r), where P.V runs on v_dot2
-// over token pairs with P rounded to bf16 and fp32 accumulation.
-template <int D>
-__device__ __forceinline__ void DecodeGroupMfma(DecodeState<uint16_t, D>& st, const uint4* kr, const uint4* vr,
-                                                uint32_t validmask, const u32x4_t* qb, float* x_row, int r, int ri,
-                                                int lane, float scale_log2, SoftCap cap) {
-  using C = DecodeCfg<uint16_t, D>;
-  constexpr int kVec = C::kVec, kTpi = C::kTpi, kNi = C::kNi, kChunks = D / 32;
-  f32x4_t acc4 = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int kc = 0; kc < kChunks; ++kc) {
-    acc4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kr[kc]),
-                                                    __builtin_bit_cast(bf16x8_t, qb[kc]), acc4, 0, 0, 0);
-  }
-  const int col = lane & 15;
-  const int tok0 = (lane >> 4) * 4;
-  float sc[4];
-  float mx = -INFINITY;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const bool ok = col < (int)kGroup && ((validmask >> (tok0 + j)) & 1u);
-    float y = acc4[j] * scale_log2;
-    if (cap.capl != 0.0f) y = Capped(y, cap);
-    sc[j] = ok ? y : -INFINITY;
-    mx = fmaxf(mx, sc[j]);
-  }
-  mx = fmaxf(mx, ShflXor(mx, 16));
-  mx = MaxXor32(mx);
-  float corr[kGroup];
-  bool rescale = false;
-#pragma unroll
-  for (int h = 0; h < (int)kGroup; ++h) {
-    const float hm = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx), h));  // lane h holds head h
-    const float mn = fmaxf(st.m[h], hm);
-    corr[h] = mn == -INFINITY ? 1.0f : exp2f(st.m[h] - mn);
-    rescale |= mn != st.m[h];
-    st.m[h] = mn;
-  }
-  const float mine = Pick4(st.m, col & 3);
-  float pf[4];
-  float psum = 0.0f;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    pf[j] = sc[j] == -INFINITY ? 0.0f : exp2f(sc[j] - mine);
-    psum += pf[j];
-  }
-  st.l_lane = st.l_lane * Pick4(corr, col & 3) + psum;
-  if (rescale) {
-#pragma unroll
-    for (int h = 0; h < (int)kGroup; ++h)
-#pragma unroll
-      for (int e = 0; e < kVec; ++e) st.acc[h][e] *= corr[h];
-  }
-  // Weights to LDS as [token][head] floats, then each P.V lane packs the bf16 pairs it needs.
-  if (col < (int)kGroup) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) x_row[(tok0 + j) * kGroup + col] = pf[j];
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  uint32_t pp[kNi / 2][kGroup];
-#pragma unroll
-  for (int a = 0; a < kNi / 2; ++a) {
-    const float4 p0 = *reinterpret_cast<const float4*>(&x_row[(kTpi * (2 * a) + ri) * kGroup]);
-    const float4 p1 = *reinterpret_cast<const float4*>(&x_row[(kTpi * (2 * a + 1) + ri) * kGroup]);
-    pp[a][0] = PackRne(p0.x, p1.x);
-    pp[a][1] = PackRne(p0.y, p1.y);
-    pp[a][2] = PackRne(p0.z, p1.z);
-    pp[a][3] = PackRne(p0.w, p1.w);
-  }
-  __builtin_amdgcn_wave_barrier();
-#pragma unroll
-  for (int a = 0; a < kNi / 2; ++a) {
-    const uint32_t* v0 = reinterpret_cast<const uint32_t*>(&vr[2 * a]);
-    const uint32_t* v1 = reinterpret_cast<const uint32_t*>(&vr[2 * a + 1]);
-#pragma unroll
-    for (int w = 0; w < kVec / 2; ++w) {
-      const uint32_t lo = __builtin_amdgcn_perm(v1[w], v0[w], 0x05040100u);
-      const uint32_t hi = __builtin_amdgcn_perm(v1[w], v0[w], 0x07060302u);
-#pragma unroll
-      for (int h = 0; h < (int)kGroup; ++h) {
-        const bf16x2_t ph = __builtin_bit_cast(bf16x2_t, pp[a][h]);
-        st.acc[h][2 * w] = __builtin_amdgcn_fdot2_f32_bf16(ph, __builtin_bit_cast(bf16x2_t, lo), st.acc[h][2 * w], false);
-        st.acc[h][2 * w + 1] =
-            __builtin_amdgcn_fdot2_f32_bf16(ph, __builtin_bit_cast(bf16x2_t, hi), st.acc[h][2 * w + 1], false);
-      }
-    }
-  }
-  (void)r;
-}
 
 // A workgroup barrier that orders LDS only: the wavefront's LDS operations complete, global loads and stores stay in
 // flight. `__syncthreads()` also waits for every outstanding global access (`vmcnt(0)`); at a piece's end that is the
@@ -1124,41 +980,43 @@ __device__ __forceinline__ void LdsBarrier() {
   asm volatile("s_barrier" ::: "memory");
 }
 
-// Split-K paged decode. kFastPage: page_size is a multiple of 16, so a 16-token group (16-aligned within its
+// Split-K paged decode of f32 caches. kFastPage: page_size is a multiple of 16, so a 16-token group (16-aligned within its
 // sequence) lies in one page and its page id is one wave-uniform scalar load; otherwise each lane looks its own
 // token's page up. Loads are branch-free (an absent key reads a valid address and is masked) and the next group's
 // K/V is fetched into a second register buffer while the current group is computed. Workgroup (range, KV head)
 // processes the pieces of its range in turn; a piece that is not a whole sequence writes fp32 partials that
 // DecodeMergeKernel combines in key order.
-template <typename T, int D, bool kFastPage, int kWaves>
-__device__ __forceinline__ void DecodeBody(const T* __restrict__ q, T* __restrict__ out, float* __restrict__ lse,
-                                           KvView kv, const int32_t* __restrict__ kv_indices,
-                                           const DecodeWork* __restrict__ work, const int32_t* __restrict__ range_ptr,
-                                           float* __restrict__ part_o, float* __restrict__ part_ml,
-                                           const int32_t* __restrict__ q_rows, uint32_t q_heads, uint32_t heads_per_wg,
-                                           float scale_log2, int32_t window, uint32_t causal, SoftCap cap,
-                                           uint32_t block, float* x_lds, float* m_lds, float* l_lds, float* o_lds) {
-  // LDS (the caller's): x_lds [kWaves][64], m_lds and l_lds [kWaves][kGroup], o_lds [kWaves][kGroup][D] floats.
-  using C = DecodeCfg<T, D>;
+template <int D, bool kFastPage>
+__global__ void __launch_bounds__(256, kDecodeWgsPerCu)
+    DecodeF32Kernel(const float* __restrict__ q, float* __restrict__ out, float* __restrict__ lse, KvView kv,
+                    const int32_t* __restrict__ kv_indices, const DecodeWork* __restrict__ work,
+                    const int32_t* __restrict__ range_ptr, float* __restrict__ part_o, float* __restrict__ part_ml,
+                    const int32_t* __restrict__ q_rows, uint32_t q_heads, uint32_t heads_per_wg, float scale_log2,
+                    int32_t window, uint32_t causal, SoftCap cap) {
+  using C = DecodeCfg<D>;
   constexpr int kVec = C::kVec, kLpr = C::kLpr, kTpi = C::kTpi, kNi = C::kNi;
-  constexpr bool kMfma = sizeof(T) == 2;  // bf16: q.k on MFMA; f32: the VALU reduce-scatter path
+  constexpr int kWaves = 4;
+  __shared__ float x_lds[kWaves][64];
+  __shared__ float m_lds[kWaves * kGroup];
+  __shared__ float l_lds[kWaves * kGroup];
+  __shared__ float o_lds[kWaves * kGroup * D];
 
   // Both KV heads of a range are adjacent in launch order, so the two halves of each NHD page row are read together.
   // A workgroup serves heads_per_wg (1, 2 or 4) KV heads of one range, 4 / heads_per_wg wavefronts per head, so the
   // KV heads of each page row (adjacent in an NHD pool) are read by one CU at the same time.
   const uint32_t hblocks = kv.vheads / heads_per_wg;
-  const uint32_t range = block / hblocks;
+  const uint32_t range = blockIdx.x / hblocks;
   const int lane = threadIdx.x & 63;
   // The wavefront index is uniform within a wavefront; saying so lets the group's page id be a scalar load.
   const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t kvh = (block % hblocks) * heads_per_wg + wave_id % heads_per_wg;
+  const uint32_t kvh = (blockIdx.x % hblocks) * heads_per_wg + wave_id % heads_per_wg;
   const int wave = wave_id / static_cast<int>(heads_per_wg);           // index among this head's wavefronts
   const int waves_per_head = kWaves / static_cast<int>(heads_per_wg);
   const int r = lane % kLpr;   // which 16-byte slice of a row
   const int ri = lane / kLpr;  // which row of a wave-wide load
   const int kperm = r / static_cast<int>(kGroup);  // this lane's token-slot permutation for K
-  const T* kbase = static_cast<const T*>(kv.k);
-  const T* vbase = static_cast<const T*>(kv.v);
+  const float* kbase = static_cast<const float*>(kv.k);
+  const float* vbase = static_cast<const float*>(kv.v);
 
   const int32_t it_end = range_ptr[range + 1];
   for (int32_t it = range_ptr[range]; it < it_end; ++it) {
@@ -1179,29 +1037,17 @@ __device__ __forceinline__ void DecodeBody(const T* __restrict__ q, T* __restric
   // The sliding window's first visible key; the piece may start up to 15 keys before it, which are masked.
   const uint32_t lo = window < 0 || kv_len == 0 ? 0u : static_cast<uint32_t>(max(0, qpos - window));
 
-  using QW = typename std::conditional<sizeof(T) == 2, uint32_t, float>::type;
-  QW qr[kGroup][C::kQWords];   // VALU path (f32)
-  u32x4_t qb[kMfma ? D / 32 : 1];  // MFMA path (bf16): B operand of q.k
-  if constexpr (kMfma) {
-    const int col = lane & 15;
-    const T* qrow = q + (tok * q_heads + kvh * kGroup + (col & 3)) * D + (lane >> 4) * 8;
-#pragma unroll
-    for (int kc = 0; kc < D / 32; ++kc) {
-      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(qrow + kc * 32);
-      qb[kc] = col < (int)kGroup ? v : u32x4_t{0, 0, 0, 0};
-    }
-  } else {
-    const T* qrow = q + (tok * q_heads + kvh * kGroup) * D + r * kVec;
+  float qr[kGroup][kVec];
+  {
+    const float* qrow = q + (tok * q_heads + kvh * kGroup) * D + r * kVec;
 #pragma unroll
     for (int h = 0; h < (int)kGroup; ++h) {
-      const uint4 v = *reinterpret_cast<const uint4*>(qrow + (h ^ (r & 3)) * D);
-      const QW* w = reinterpret_cast<const QW*>(&v);
-#pragma unroll
-      for (int i = 0; i < C::kQWords; ++i) qr[h][i] = w[i];
+      const float4 v = *reinterpret_cast<const float4*>(qrow + (h ^ (r & 3)) * D);
+      qr[h][0] = v.x; qr[h][1] = v.y; qr[h][2] = v.z; qr[h][3] = v.w;
     }
   }
 
-  DecodeState<T, D> st;
+  DecodeState<D> st;
 #pragma unroll
   for (int h = 0; h < (int)kGroup; ++h) {
     st.m[h] = -INFINITY;
@@ -1211,7 +1057,7 @@ __device__ __forceinline__ void DecodeBody(const T* __restrict__ q, T* __restric
   st.l_lane = 0.0f;
 
   // Byte stride between the rows of consecutive tokens of one KV head inside a page.
-  const uint32_t tok_bytes = (kv.hnd ? D : kv.kv_heads * D) * static_cast<uint32_t>(sizeof(T));
+  const uint32_t tok_bytes = (kv.hnd ? D : kv.kv_heads * D) * 4;
   // Group gi (0-based, 16 tokens) of this wavefront: key g = t_begin + 16 * (wave + waves_per_head * gi).
   const uint32_t ngroups = (t_end > t_begin) ? (t_end - t_begin + 15) / 16 : 0;
   const uint32_t nw = ngroups > static_cast<uint32_t>(wave)
@@ -1239,42 +1085,23 @@ __device__ __forceinline__ void DecodeBody(const T* __restrict__ q, T* __restric
         const uint32_t tv = i * kTpi + ri;  // V register i: slot i
         const bool okv = live && page_ok && g0 + tv < t_end && g0 + tv >= lo;
         vr[i] = LoadStream16(vg + ((okv ? tv : 0) * tok_bytes + r * 16));
-        if constexpr (kMfma) {
-          const uint32_t tk = lane & 15;  // K register i: dims 32 i + 8 (lane / 16) of token lane % 16
-          const bool okk = page_ok && g0 + tk < t_end;
-          kr[i] = *reinterpret_cast<const uint4*>(kg + ((okk ? tk : 0) * tok_bytes + i * 64 + (lane >> 4) * 16));
-        } else {
-          const uint32_t tk = (i ^ kperm) * kTpi + ri;  // K register i: slot i ^ kperm
-          const bool okk = page_ok && g0 + tk < t_end;
-          kr[i] = LoadStream16(kg + ((okk ? tk : 0) * tok_bytes + r * 16));
-          valid |= static_cast<uint32_t>(okv) << i;
-        }
-      }
-      if constexpr (kMfma) {
-        const uint32_t n = live && page_ok ? min(16u, t_end - g0) : 0u;
-        valid = (1u << n) - 1u;  // bit t: token t of the group is a real key
-        if (g0 < lo) valid &= ~((1u << min(16u, lo - g0)) - 1u);  // before the window
+        const uint32_t tk = (i ^ kperm) * kTpi + ri;  // K register i: slot i ^ kperm
+        const bool okk = page_ok && g0 + tk < t_end;
+        kr[i] = LoadStream16(kg + ((okk ? tk : 0) * tok_bytes + r * 16));
+        valid |= static_cast<uint32_t>(okv) << i;
       }
     } else {
-      bool kok = false;
 #pragma unroll
       for (int i = 0; i < kNi; ++i) {
         bool okk, okv;
-        const int32_t tk = kMfma ? static_cast<int32_t>(g0 + (lane & 15))
-                                 : static_cast<int32_t>(g0 + (i ^ kperm) * kTpi + ri);
+        const int32_t tk = static_cast<int32_t>(g0 + (i ^ kperm) * kTpi + ri);
         const uint64_t rowk = KeyRowSafe<D>(kv, p0, tk, static_cast<int32_t>(t_end), kvh, &okk);
         const uint64_t rowv = KeyRowSafe<D>(kv, p0, static_cast<int32_t>(g0 + i * kTpi + ri),
                                             static_cast<int32_t>(t_end), kvh, &okv);
-        okk = okk && tk >= static_cast<int32_t>(lo);
         okv = okv && g0 + i * kTpi + ri >= lo;
-        kr[i] = *reinterpret_cast<const uint4*>(kMfma ? kbase + rowk + i * 32 + (lane >> 4) * 8 : kbase + rowk + r * kVec);
+        kr[i] = *reinterpret_cast<const uint4*>(kbase + rowk + r * kVec);
         vr[i] = LoadStream16(vbase + rowv + r * kVec);
-        if constexpr (!kMfma) valid |= static_cast<uint32_t>(okv && live) << i;
-        kok = okk;
-      }
-      if constexpr (kMfma) {
-        // Lanes 0..15 hold tokens 0..15 of the group: their K validity is the key mask.
-        valid = static_cast<uint32_t>(__ballot(kok && live)) & 0xFFFFu;
+        valid |= static_cast<uint32_t>(okv && live) << i;
       }
     }
   };
@@ -1293,11 +1120,7 @@ __device__ __forceinline__ void DecodeBody(const T* __restrict__ q, T* __restric
         const int nxt = (s + kLast) % kDecodeRing;
         load(gi + s + kLast, kbuf[nxt], vbuf[nxt], valid[nxt]);
         if (gi + s < nw) {
-          if constexpr (kMfma) {
-            DecodeGroupMfma<D>(st, kbuf[s], vbuf[s], valid[s], qb, x_lds + 64 * wave_id, r, ri, lane, scale_log2, cap);
-          } else {
-            DecodeGroup<T, D, QW>(st, kbuf[s], vbuf[s], valid[s], qr, x_lds + 64 * wave_id, r, ri, lane, scale_log2, cap);
-          }
+          DecodeGroup<D>(st, kbuf[s], vbuf[s], valid[s], qr, x_lds[wave_id], r, ri, lane, scale_log2, cap);
         }
       }
     }
@@ -1310,10 +1133,10 @@ __device__ __forceinline__ void DecodeBody(const T* __restrict__ q, T* __restric
     for (int h = 0; h < (int)kGroup; ++h)
 #pragma unroll
       for (int e = 0; e < kVec; ++e) st.acc[h][e] += ShflXor(st.acc[h][e], mk);
-  // Per-lane denominators: VALU path, lanes with r % 4 == h hold head h; MFMA path, lanes with lane % 16 == h.
+  // Per-lane denominators: lanes with r % 4 == h hold head h.
   float lsum = st.l_lane;
 #pragma unroll
-  for (int mk = kMfma ? 16 : 4; mk < 64; mk <<= 1) lsum += ShflXor(lsum, mk);
+  for (int mk = 4; mk < 64; mk <<= 1) lsum += ShflXor(lsum, mk);
   if (lane < (int)kGroup) {
     m_lds[wave_id * kGroup + lane] = Pick4(st.m, lane);
     l_lds[wave_id * kGroup + lane] = lsum;  // lane h holds the total of head h
@@ -1340,10 +1163,10 @@ __device__ __forceinline__ void DecodeBody(const T* __restrict__ q, T* __restric
       o += o_lds[(w * kGroup + h) * D + d] * f;
       L += l_lds[w * kGroup + h] * f;
     }
-    const uint32_t qh = ((block % hblocks) * heads_per_wg + hk) * kGroup + h;
+    const uint32_t qh = ((blockIdx.x % hblocks) * heads_per_wg + hk) * kGroup + h;
     if (split < 0) {
       const uint64_t row = tok * q_heads + qh;
-      out[row * D + d] = GateOut<T>(kv.out_gate, row * D + d, Vec<T>::Narrow(L > 0.0f ? o / L : 0.0f));
+      out[row * D + d] = GateOut<float>(kv.out_gate, row * D + d, L > 0.0f ? o / L : 0.0f);
       if (lse != nullptr && d == 0) lse[row] = L > 0.0f ? M + log2f(L) : -INFINITY;
     } else {
       const uint64_t prow = static_cast<uint64_t>(split) * q_heads + qh;
@@ -1359,23 +1182,297 @@ __device__ __forceinline__ void DecodeBody(const T* __restrict__ q, T* __restric
 }
 
 
-// Split-K paged decode, one workgroup of 4 wavefronts per (range, head block): DecodeBody with LDS of its own.
-template <typename T, int D, bool kFastPage>
-__global__ void __launch_bounds__(256, kDecodeWgsPerCu) DecodeKernel(const T* __restrict__ q, T* __restrict__ out, float* __restrict__ lse,
-                                                    KvView kv, const int32_t* __restrict__ kv_indices,
-                                                    const DecodeWork* __restrict__ work,
-                                                    const int32_t* __restrict__ range_ptr,
-                                                    float* __restrict__ part_o, float* __restrict__ part_ml,
-                                                    const int32_t* __restrict__ q_rows,
-                                                    uint32_t q_heads, uint32_t heads_per_wg, float scale_log2,
-                                                    int32_t window, uint32_t causal, SoftCap cap) {
-  __shared__ float x_lds[4][64];
-  __shared__ float m_lds[4][kGroup];
-  __shared__ float l_lds[4][kGroup];
-  __shared__ float o_lds[4][kGroup][D];
-  DecodeBody<T, D, kFastPage, 4>(q, out, lse, kv, kv_indices, work, range_ptr, part_o, part_ml, q_rows, q_heads,
-                                 heads_per_wg, scale_log2, window, causal, cap, blockIdx.x, &x_lds[0][0], &m_lds[0][0],
-                                 &l_lds[0][0], &o_lds[0][0][0]);
+// ---- bf16 decode kernel ----------------------------------------------------------------------------------------------
+//
+// A wavefront serves all NH = 4, 8 or 16 query heads of a KV head (padded to 16) and both products run on matrix
+// instructions, with no exchange of the weights between lanes. Per group of 16 tokens, lane (c = lane % 16, g = lane / 16):
+//   * q.k on v_mfma_f32_16x16x32_bf16 (tokens on M, heads on N): the lane gets the scores of tokens 4g .. 4g + 3 for head c;
+//   * its four weights, packed, are the A operand (heads on M, tokens 4g + i in k-slots 4g + i) of
+//     v_mfma_f32_16x16x16_bf16;
+//   * it loads the D / 16 dims of slice c of tokens 4g .. 4g + 3 (whole rows per 16 lanes), and pairs of those rows
+//     interleaved with v_perm are the B operands: one multiply per dim e of the slice gives heads 4g + j, dim (c, e).
+// The running maximum moves only when a score exceeds it by more than 2^8 (as in the prefill kernels: weights stay below
+// 256), so the exchange that brings a head's rescale factor to the lanes holding its sums is rare.
+//
+// Bound by HBM. One register buffer each for a group's K and V rows: the next group's K rows are requested once the
+// scores have read these, its V rows once P.V has, so one of the two is in flight at all times. Two buffers of each
+// (the next group requested before this one is computed) were slower: 73 against 67 us at 16 heads over 2, head dim
+// 256, 324 MB (they spill there), 113 against 112 at 32 over 4, head dim 128. V, read in whole rows, and K at head dims
+// 64 and 128 take the non-temporal hint (V plain: 110 against 101 us at 8 over 2, head dim 256, 579 MB); K at 256, where
+// an instruction reads half of each 128-byte line, is faster without (101 against 102.4).
+// Measured against groups of 4 heads on v_dot2 with a double buffer, whose larger groups requested the rows again for
+// every 4 heads (contexts cold): 8 over 2, 256: 107 -> 101 us (5.7 TB/s); 32 over 8, 128: 115 -> 107; 16 over 4, 64:
+// 82 -> 72; 32 over 4, 128 (642 MB): 168 -> 112; 32 over 2, 128: 134 -> 64; 32 over 2, 256: 155 -> 74.
+typedef short i16x4v_t __attribute__((ext_vector_type(4)));
+
+template <int D, int NH, bool kFastPage, int kWaves>
+__device__ __forceinline__ void DecodeMfmaBody(const uint16_t* __restrict__ q, uint16_t* __restrict__ out,
+                                               float* __restrict__ lse, KvView kv,
+                                               const int32_t* __restrict__ kv_indices,
+                                               const DecodeWork* __restrict__ work,
+                                               const int32_t* __restrict__ range_ptr, float* __restrict__ part_o,
+                                               float* __restrict__ part_ml, const int32_t* __restrict__ q_rows,
+                                               uint32_t q_heads, uint32_t heads_per_wg, float scale_log2,
+                                               int32_t window, uint32_t causal, SoftCap cap, uint32_t block,
+                                               float* m_lds, float* l_lds, float* o_lds) {
+  // LDS (the caller's): m_lds and l_lds [kWaves][NH], o_lds [kWaves][NH][D] floats. kv.vheads and kv.head_shift count
+  // groups of NH query heads.
+  constexpr int kKc = D / 32;                // K operands (16 bytes per lane) of a group
+  constexpr int kSlice = D >= 128 ? 8 : 4;   // dims of one V load per lane
+  constexpr int kVh = D / 16 / kSlice;       // V loads per token: the row in kVh parts of 16 slices
+  constexpr bool kQLds = D == 256 && NH > 4;
+  static_assert(!kQLds || NH * D * 4 >= 64 * 16 * kKc, "q fits in the wavefront's share of o_lds");
+  typedef uint32_t vword_t __attribute__((ext_vector_type(kSlice / 2)));
+
+  const uint32_t hblocks = kv.vheads / heads_per_wg;
+  const uint32_t range = block / hblocks;
+  const int lane = threadIdx.x & 63;
+  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t kvh = (block % hblocks) * heads_per_wg + wave_id % heads_per_wg;
+  const int wave = wave_id / static_cast<int>(heads_per_wg);
+  const int waves_per_head = kWaves / static_cast<int>(heads_per_wg);
+  const int c = lane & 15, g = lane >> 4;
+  const uint16_t* kbase = static_cast<const uint16_t*>(kv.k);
+  const uint16_t* vbase = static_cast<const uint16_t*>(kv.v);
+
+  const int32_t it_end = range_ptr[range + 1];
+  for (int32_t it = range_ptr[range]; it < it_end; ++it) {
+    const DecodeWork wk = work[it];
+    int32_t p0 = 0;
+    const uint32_t kv_len = SeqKvLen(kv, wk.seq, &p0);
+    // The row's query token and the keys it sees, as in DecodeF32Kernel.
+    const uint64_t tok = q_rows != nullptr
+                             ? static_cast<uint64_t>(max(q_rows[wk.seq], q_rows[wk.seq + 1] - 1 - wk.q_back))
+                             : static_cast<uint64_t>(wk.seq);
+    const int32_t qpos = static_cast<int32_t>(kv_len) - 1 - wk.q_back;
+    const uint32_t t_begin = static_cast<uint32_t>(wk.token_begin);
+    uint32_t t_end = min(kv_len, static_cast<uint32_t>(wk.token_end));
+    if (causal) t_end = min(t_end, static_cast<uint32_t>(max(0, qpos + 1)));
+    const uint32_t lo = window < 0 || kv_len == 0 ? 0u : static_cast<uint32_t>(max(0, qpos - window));
+
+    // B operand of q.k: head c's dims 32 kc + 8 g .. +8 (columns past NH repeat the heads; their results are not used).
+    // At head dim 256 it is kept in this wavefront's share of o_lds and read per group: in registers it spilled 48.
+    u32x4_t qb[kQLds ? 1 : kKc];
+    auto* q_lds = reinterpret_cast<u32x4_t*>(o_lds + wave_id * NH * D) + lane;
+    {
+      const uint16_t* qrow = q + (tok * q_heads + kvh * NH + c % NH) * D + g * 8;
+#pragma unroll
+      for (int kc = 0; kc < kKc; ++kc) {
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(qrow + kc * 32);
+        if constexpr (kQLds) q_lds[64 * kc] = v; else qb[kc] = v;
+      }
+    }
+    f32x4_t acc[D / 16];  // acc[kSlice * h + e][j]: head 4g + j, dim 16 kSlice h + kSlice c + e
+#pragma unroll
+    for (int e = 0; e < D / 16; ++e) acc[e] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    float m_run = -INFINITY;  // head c's running maximum (the same in the four lanes of a head)
+    float l_lane = 0.0f;      // this lane's share of head c's denominator
+
+    const uint32_t tok_bytes = (kv.hnd ? D : kv.kv_heads * D) * 2;
+    const uint32_t ngroups = (t_end > t_begin) ? (t_end - t_begin + 15) / 16 : 0;
+    const uint32_t nw = ngroups > static_cast<uint32_t>(wave)
+                            ? (ngroups - wave + waves_per_head - 1) / waves_per_head : 0;
+    // Where group gi (16 tokens) of this wavefront lies: key g0 = t_begin + 16 (wave + waves_per_head gi). A group past
+    // the end is the last one again with no valid key, so that every load is unconditional.
+    struct Place {
+      uint64_t row;    // element offset of its first token's row; of token c's row when the group may cross pages
+      uint32_t g0;
+      uint32_t valid;  // bit t: token t is a real key of the window
+      bool page_ok;    // its page id lies in the pool (a group in one page)
+    };
+    auto place = [&](uint32_t gi) {
+      Place a;
+      a.g0 = t_begin + 16u * (wave + waves_per_head * min(gi, nw - 1));
+      if constexpr (kFastPage) {
+        const uint32_t pi = a.g0 / kv.page_size;
+        const uint32_t off0 = a.g0 - pi * kv.page_size;
+        const int32_t page = kv_indices[p0 + pi];  // uniform address: a scalar load
+        a.page_ok = page >= 0 && static_cast<uint64_t>(page) < kv.pool_pages;
+        const uint64_t pg = a.page_ok ? static_cast<uint64_t>(page) : 0;
+        const uint32_t kvr = kvh >> kv.head_shift;
+        a.row = (kv.hnd ? (pg * kv.kv_heads + kvr) * kv.page_size + off0
+                        : (pg * kv.page_size + off0) * kv.kv_heads + kvr) * D;
+        const uint32_t n = gi < nw && a.page_ok ? min(16u, t_end - a.g0) : 0u;
+        a.valid = (1u << n) - 1u;
+      } else {
+        bool ok;
+        a.row = KeyRowSafe<D>(kv, p0, static_cast<int32_t>(a.g0 + c), static_cast<int32_t>(t_end), kvh, &ok);
+        a.page_ok = true;
+        a.valid = static_cast<uint32_t>(__ballot(ok && gi < nw)) & 0xFFFFu;  // lanes 0..15 hold tokens 0..15
+      }
+      if (a.g0 < lo) a.valid &= ~((1u << min(16u, lo - a.g0)) - 1u);  // before the window
+      return a;
+    };
+    // Rows of absent tokens are read as the group's first (general pages: as the pool's first).
+    auto load_k = [&](const Place& a, u32x4_t* kr) {
+      const char* kg = reinterpret_cast<const char*>(kbase + a.row);
+      const uint32_t ko = (kFastPage && a.page_ok && a.g0 + c < t_end ? c : 0) * tok_bytes + g * 16;
+#pragma unroll
+      for (int i = 0; i < kKc; ++i) {
+        const auto* kp = reinterpret_cast<const u32x4_t*>(kg + (ko + i * 64));
+        kr[i] = D <= 128 ? __builtin_nontemporal_load(kp) : *kp;
+      }
+    };
+    auto load_v = [&](const Place& a, vword_t (*vr)[4]) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t tv = 4 * g + i;
+        uint64_t row = a.row;
+        uint32_t vo = c * (2 * kSlice);
+        if constexpr (kFastPage) {
+          vo += (((a.valid >> tv) & 1u) ? tv : 0) * tok_bytes;
+        } else {
+          bool ok;
+          row = KeyRowSafe<D>(kv, p0, static_cast<int32_t>(a.g0 + tv), static_cast<int32_t>(t_end), kvh, &ok);
+        }
+        const char* vg = reinterpret_cast<const char*>(vbase + row);
+#pragma unroll
+        for (int h = 0; h < kVh; ++h) {
+          vr[h][i] = __builtin_nontemporal_load(reinterpret_cast<const vword_t*>(vg + (vo + h * 32 * kSlice)));
+        }
+      }
+    };
+    auto scores = [&](const u32x4_t* kr) {
+      f32x4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
+      int again = 0;
+      if constexpr (kQLds) asm volatile("" : "+v"(again));  // keeps the reads in the loop
+#pragma unroll
+      for (int kc = 0; kc < kKc; ++kc) {
+        u32x4_t qv;
+        if constexpr (kQLds) qv = q_lds[64 * kc + again]; else qv = qb[kc];
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kr[kc]),
+                                                    __builtin_bit_cast(bf16x8_t, qv), s, 0, 0, 0);
+      }
+      return s;
+    };
+    auto fold = [&](f32x4_t s, const vword_t (*vr)[4], uint32_t valid) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float y = s[j] * scale_log2;
+        if (cap.capl != 0.0f) y = Capped(y, cap);
+        s[j] = ((valid >> (4 * g + j)) & 1u) ? y : -INFINITY;
+        mx = fmaxf(mx, s[j]);
+      }
+      mx = fmaxf(mx, ShflXor(mx, 16));
+      mx = MaxXor32(mx);
+      const bool grow = mx > m_run + 8.0f;
+      if (__any(grow)) {
+        const float m_new = grow ? mx : m_run;
+        const float corr = m_run == -INFINITY ? 0.0f : exp2f(m_run - m_new);
+        l_lane *= corr;
+        m_run = m_new;
+        float cj[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) cj[j] = __shfl(corr, 4 * g + j, 64);  // lane h holds head h
+#pragma unroll
+        for (int e = 0; e < D / 16; ++e)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[e][j] *= cj[j];
+      }
+      const float m_use = m_run == -INFINITY ? 0.0f : m_run;  // a head with no visible key yet keeps p = 0
+      float p[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(s[j] - m_use);
+      l_lane += (p[0] + p[1]) + (p[2] + p[3]);
+      const i16x4v_t pa = __builtin_bit_cast(i16x4v_t, u32x2_t{PackRne(p[0], p[1]), PackRne(p[2], p[3])});
+#pragma unroll
+      for (int h = 0; h < kVh; ++h)
+#pragma unroll
+        for (int w = 0; w < kSlice / 2; ++w) {
+          const u32x2_t b0{__builtin_amdgcn_perm(vr[h][1][w], vr[h][0][w], 0x05040100u),
+                           __builtin_amdgcn_perm(vr[h][3][w], vr[h][2][w], 0x05040100u)};
+          const u32x2_t b1{__builtin_amdgcn_perm(vr[h][1][w], vr[h][0][w], 0x07060302u),
+                           __builtin_amdgcn_perm(vr[h][3][w], vr[h][2][w], 0x07060302u)};
+          const int e = kSlice * h + 2 * w;
+          acc[e] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa, __builtin_bit_cast(i16x4v_t, b0), acc[e], 0, 0, 0);
+          acc[e + 1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa, __builtin_bit_cast(i16x4v_t, b1), acc[e + 1], 0, 0, 0);
+        }
+    };
+
+    if (nw > 0) {
+      u32x4_t kr[kKc];
+      vword_t vr[kVh][4];
+      Place cur = place(0);
+      load_k(cur, kr);
+      load_v(cur, vr);
+      for (uint32_t gi = 0; gi < nw; ++gi) {
+        const Place nxt = place(gi + 1);
+        const f32x4_t s = scores(kr);
+        __builtin_amdgcn_sched_barrier(0);  // the next K rows are requested as soon as the scores have read these
+        load_k(nxt, kr);
+        fold(s, vr, cur.valid);
+        __builtin_amdgcn_sched_barrier(0);
+        load_v(nxt, vr);
+        cur = nxt;
+      }
+    }
+
+    float lsum = l_lane + ShflXor(l_lane, 16);
+    lsum = SumXor32(lsum);
+    if (lane < NH) {
+      m_lds[wave_id * NH + lane] = m_run;
+      l_lds[wave_id * NH + lane] = lsum;
+    }
+    if (4 * g < NH) {
+#pragma unroll
+      for (int h = 0; h < kVh; ++h)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int e = 0; e < kSlice; ++e)
+            o_lds[(wave_id * NH + 4 * g + j) * D + 16 * kSlice * h + kSlice * c + e] = acc[kSlice * h + e][j];
+    }
+    LdsBarrier();
+
+    // Workgroup: merge the wavefronts of each KV head, then write the final row or this piece's partial (four dims per
+    // thread: a head's weights are formed once for the four).
+    const int split = wk.slot;
+    for (int idx = threadIdx.x; idx < (int)(heads_per_wg * NH * D / 4); idx += 64 * kWaves) {
+      const int hk = idx / (NH * D / 4);
+      const int h = (idx / (D / 4)) % NH;
+      const int d = 4 * (idx % (D / 4));
+      float M = -INFINITY;
+      for (int w = hk; w < kWaves; w += heads_per_wg) M = fmaxf(M, m_lds[w * NH + h]);
+      f32x4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+      float L = 0.0f;
+      for (int w = hk; w < kWaves; w += heads_per_wg) {
+        const float f = m_lds[w * NH + h] == -INFINITY ? 0.0f : exp2f(m_lds[w * NH + h] - M);
+        o += *reinterpret_cast<const f32x4_t*>(&o_lds[(w * NH + h) * D + d]) * f;
+        L += l_lds[w * NH + h] * f;
+      }
+      const uint32_t qh = ((block % hblocks) * heads_per_wg + hk) * NH + h;
+      if (split < 0) {
+        const uint64_t row = tok * q_heads + qh;
+        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+        const u32x2_t v{PackBf16(o[0] * inv, o[1] * inv), PackBf16(o[2] * inv, o[3] * inv)};
+        *reinterpret_cast<u32x2_t*>(out + row * D + d) = GateOut2(kv.out_gate, row * D + d, v);
+        if (lse != nullptr && d == 0) lse[row] = L > 0.0f ? M + log2f(L) : -INFINITY;
+      } else {
+        const uint64_t prow = static_cast<uint64_t>(split) * q_heads + qh;
+        *reinterpret_cast<f32x4_t*>(part_o + prow * D + d) = o;
+        if (d == 0) {
+          part_ml[prow * 2] = M;
+          part_ml[prow * 2 + 1] = L;
+        }
+      }
+    }
+    LdsBarrier();  // the next piece reuses the LDS merge buffers
+  }
+}
+
+template <int D, int NH, bool kFastPage>
+__global__ void __launch_bounds__(256, kDecodeWgsPerCu)
+    DecodeMfmaKernel(const uint16_t* __restrict__ q, uint16_t* __restrict__ out, float* __restrict__ lse, KvView kv,
+                     const int32_t* __restrict__ kv_indices, const DecodeWork* __restrict__ work,
+                     const int32_t* __restrict__ range_ptr, float* __restrict__ part_o, float* __restrict__ part_ml,
+                     const int32_t* __restrict__ q_rows, uint32_t q_heads, uint32_t heads_per_wg, float scale_log2,
+                     int32_t window, uint32_t causal, SoftCap cap) {
+  __shared__ float m_lds[4][NH];
+  __shared__ float l_lds[4][NH];
+  __shared__ __attribute__((aligned(16))) float o_lds[4][NH][D];
+  DecodeMfmaBody<D, NH, kFastPage, 4>(q, out, lse, kv, kv_indices, work, range_ptr, part_o, part_ml, q_rows, q_heads, heads_per_wg,
+                           scale_log2, window, causal, cap, blockIdx.x, &m_lds[0][0], &l_lds[0][0], &o_lds[0][0][0]);
 }
 
 // Combines the pieces of each split sequence in key order: one workgroup per (sequence, query head), D threads, one
@@ -1450,7 +1547,7 @@ __device__ __forceinline__ void DecodeMergeBody(T* __restrict__ out, float* __re
   }
   for (int c = kPre; c < n; ++c) acc[c & 3] = fmaf(po[c * step], f_lds[c], acc[c & 3]);
   const float o0 = acc[0], o1 = acc[1], o2 = acc[2], o3 = acc[3];
-  out[e] = GateApply<T>(out_gate, gv, Vec<T>::Narrow(((o0 + o1) + (o2 + o3)) * inv_lds));
+  out[e] = GateApply<T>(out_gate, gv, Narrow<T>(((o0 + o1) + (o2 + o3)) * inv_lds));
 }
 
 template <typename T, int D>
@@ -2068,11 +2165,11 @@ __global__ void __launch_bounds__(512, 1)
 // wavefronts each (one range of one KV-head block per CU, 8 / heads_per_wg wavefronts per head). Tile workgroups come
 // first in launch order, so they take their CUs before the decode ranges fill the others. Both kinds use the one LDS
 // buffer in their own layout (a decode workgroup needs far less than a tile one, and neither shares its CU).
-template <int D>
-constexpr int kMixedDecodeLds = 4 * (kMixedDecodeWaves * 64 + 2 * kMixedDecodeWaves * kGroup +
-                                     kMixedDecodeWaves * kGroup * D);
+// NH: query heads of a decode wavefront (DecodeGroupOf); dec_vheads and dec_shift are the decode side's KvView fields.
+template <int D, int NH>
+constexpr int kMixedDecodeLds = 4 * (2 * kMixedDecodeWaves * NH + kMixedDecodeWaves * NH * D);
 
-template <int D, bool kCap>
+template <int D, bool kCap, int NH>
 __global__ void __launch_bounds__(512, 1)
     MixedAttentionKernel(const uint16_t* __restrict__ q, uint16_t* __restrict__ out, float* __restrict__ lse,
                          KvView kv, const int32_t* __restrict__ kv_indices, const int32_t* __restrict__ q_indptr,
@@ -2081,9 +2178,9 @@ __global__ void __launch_bounds__(512, 1)
                          float scale_log2, int32_t window, SoftCap raw_cap, uint32_t items,
                          const DecodeWork* __restrict__ dec_work, const int32_t* __restrict__ dec_range_ptr,
                          float* __restrict__ dec_part_o, float* __restrict__ dec_part_ml, uint32_t heads_per_wg,
-                         SoftCap cap) {
+                         uint32_t dec_vheads, uint32_t dec_shift, SoftCap cap) {
   constexpr int kTileLds = 2 * 2 * kPfTileBytes<D>;
-  constexpr int kLds = kTileLds > kMixedDecodeLds<D> ? kTileLds : kMixedDecodeLds<D>;
+  constexpr int kLds = kTileLds > kMixedDecodeLds<D, NH> ? kTileLds : kMixedDecodeLds<D, NH>;
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
   if (blockIdx.x < items) {
     PrefillTileBody<D, kCap>(q, out, lse, kv, kv_indices, q_indptr, work, part_o, part_ml, q_heads, causal, ps_shift,
@@ -2092,13 +2189,14 @@ __global__ void __launch_bounds__(512, 1)
     return;
   }
   constexpr int W = kMixedDecodeWaves;
-  float* x_lds = reinterpret_cast<float*>(lds);
-  float* m_lds = x_lds + W * 64;
-  float* l_lds = m_lds + W * kGroup;
-  float* o_lds = l_lds + W * kGroup;
-  DecodeBody<uint16_t, D, true, W>(q, out, lse, kv, kv_indices, dec_work, dec_range_ptr, dec_part_o, dec_part_ml,
-                                   q_indptr, q_heads, heads_per_wg, scale_log2, window, causal, cap,
-                                   blockIdx.x - items, x_lds, m_lds, l_lds, o_lds);
+  kv.vheads = dec_vheads;
+  kv.head_shift = dec_shift;
+  float* m_lds = reinterpret_cast<float*>(lds);
+  float* l_lds = m_lds + W * NH;
+  float* o_lds = l_lds + W * NH;
+  DecodeMfmaBody<D, NH, true, W>(q, out, lse, kv, kv_indices, dec_work, dec_range_ptr, dec_part_o, dec_part_ml, q_indptr,
+                                 q_heads, heads_per_wg, scale_log2, window, causal, cap, blockIdx.x - items, m_lds,
+                                 l_lds, o_lds);
 }
 
 // Combines the pieces of a split prefill item: block (merge, group of kRows tokens) of kGroup * D / 4 threads; thread t
@@ -2264,6 +2362,13 @@ RoostStatus LaunchDecodeMerge(const RoostPagedAttentionParams& p, const PlanReco
   return roost::HipStatus(hipGetLastError(), "paged_attention", "decode merge launch");
 }
 
+// The view of the decode kernels, whose virtual heads are groups of DecodeGroupOf query heads.
+KvView DecodeView(const RoostPagedAttentionParams& p, KvView kv) {
+  kv.vheads = DecodeHeads(p);
+  kv.head_shift = static_cast<uint32_t>(__builtin_ctz(kv.vheads / p.kv_heads));
+  return kv;
+}
+
 template <typename T, int D>
 RoostStatus LaunchDecode(const RoostPagedAttentionParams& p, const PlanRecord& rec, unsigned char* dev, const KvView& kv,
                          float scale_log2, hipStream_t stream) {
@@ -2277,16 +2382,26 @@ RoostStatus LaunchDecode(const RoostPagedAttentionParams& p, const PlanRecord& r
       p.mode == ROOST_ATTENTION_PREFILL ? static_cast<const int32_t*>(p.q_indptr.address) : nullptr;
   auto* out = static_cast<T*>(p.output.address);
   auto* lse = static_cast<float*>(p.lse.address);
-  const uint32_t hpw = HeadsPerWorkgroup(VirtualHeads(p));
-  const dim3 grid(static_cast<uint32_t>(rec.dec_ranges * (VirtualHeads(p) / hpw)));
-  if (p.page_size % 16 == 0) {
-    hipLaunchKernelGGL((DecodeKernel<T, D, true>), grid, dim3(256), 0, stream, static_cast<const T*>(p.q.address), out,
-                       lse, kv, kv.kv_indices, items, range_ptr, part_o, part_ml, q_rows, p.q_heads, hpw, scale_log2,
-                       WindowOf(p), p.causal, CapOf(p));
+  const uint32_t heads = DecodeHeads(p), hpw = HeadsPerWorkgroup(p);
+  const KvView dkv = DecodeView(p, kv);
+  const dim3 grid(static_cast<uint32_t>(rec.dec_ranges * (heads / hpw)));
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, static_cast<const T*>(p.q.address), out, lse, dkv,
+                       kv.kv_indices, items, range_ptr, part_o, part_ml, q_rows, p.q_heads, hpw, scale_log2, WindowOf(p),
+                       p.causal, CapOf(p));
+  };
+  const bool fast = p.page_size % 16 == 0;
+  if constexpr (sizeof(T) == 2) {
+    auto of_group = [&](auto nh) {
+      constexpr int kNh = decltype(nh)::value;
+      fast ? launch(DecodeMfmaKernel<D, kNh, true>) : launch(DecodeMfmaKernel<D, kNh, false>);
+    };
+    const uint32_t nh = DecodeGroupOf(p);
+    nh == 16  ? of_group(std::integral_constant<int, 16>{})
+    : nh == 8 ? of_group(std::integral_constant<int, 8>{})
+              : of_group(std::integral_constant<int, 4>{});
   } else {
-    hipLaunchKernelGGL((DecodeKernel<T, D, false>), grid, dim3(256), 0, stream, static_cast<const T*>(p.q.address), out,
-                       lse, kv, kv.kv_indices, items, range_ptr, part_o, part_ml, q_rows, p.q_heads, hpw, scale_log2,
-                       WindowOf(p), p.causal, CapOf(p));
+    fast ? launch(DecodeF32Kernel<D, true>) : launch(DecodeF32Kernel<D, false>);
   }
   ROOST_RETURN_IF_FAILED(roost::HipStatus(hipGetLastError(), "paged_attention", "decode launch"));
   return LaunchDecodeMerge<T, D>(p, rec, dev, kv, stream);
@@ -2341,9 +2456,10 @@ RoostStatus LaunchMixed(const RoostPagedAttentionParams& p, const PlanRecord& re
   const SoftCap cap = CapOf(p);
   const SoftCap raw{cap.capl / scale_log2, cap.k * scale_log2};
   const bool capped = cap.capl != 0.0f;
-  const uint32_t hpw = HeadsPerWorkgroup(VirtualHeads(p));
+  const KvView dkv = DecodeView(p, kv);
+  const uint32_t hpw = HeadsPerWorkgroup(p);
   const uint32_t n_items = static_cast<uint32_t>(rec.work_items);
-  const dim3 grid(n_items + static_cast<uint32_t>(rec.dec_ranges * (VirtualHeads(p) / hpw)));
+  const dim3 grid(n_items + static_cast<uint32_t>(rec.dec_ranges * (dkv.vheads / hpw)));
   const auto* dec_items = reinterpret_cast<const DecodeWork*>(dev + rec.dec_item_offset);
   const auto* dec_ranges = reinterpret_cast<const int32_t*>(dev + rec.dec_range_offset);
   auto* dec_o = reinterpret_cast<float*>(dev + rec.dec_float_offset);
@@ -2351,15 +2467,21 @@ RoostStatus LaunchMixed(const RoostPagedAttentionParams& p, const PlanRecord& re
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, q16, outp, lsep, kv, kv.kv_indices, q_indptr, items,
                        PrefillPartO(p, rec, dev), PrefillPartMl(p, rec, dev), p.q_heads, p.causal, ps_shift,
-                       scale_log2, WindowOf(p), raw, n_items, dec_items, dec_ranges, dec_o, dec_ml, hpw, cap);
+                       scale_log2, WindowOf(p), raw, n_items, dec_items, dec_ranges, dec_o, dec_ml, hpw, dkv.vheads,
+                       dkv.head_shift, cap);
   };
-  if (p.head_dim == 64) {
-    capped ? launch(MixedAttentionKernel<64, true>) : launch(MixedAttentionKernel<64, false>);
-  } else if (p.head_dim == 128) {
-    capped ? launch(MixedAttentionKernel<128, true>) : launch(MixedAttentionKernel<128, false>);
-  } else {
-    capped ? launch(MixedAttentionKernel<256, true>) : launch(MixedAttentionKernel<256, false>);
-  }
+  auto of_group = [&](auto d, auto capped_c) {
+    constexpr int kD = decltype(d)::value;
+    constexpr bool kC = decltype(capped_c)::value;
+    const uint32_t nh = DecodeGroupOf(p);
+    nh == 16  ? launch(MixedAttentionKernel<kD, kC, 16>)
+    : nh == 8 ? launch(MixedAttentionKernel<kD, kC, 8>)
+              : launch(MixedAttentionKernel<kD, kC, 4>);
+  };
+  auto of_dim = [&](auto d) { capped ? of_group(d, std::true_type{}) : of_group(d, std::false_type{}); };
+  p.head_dim == 64    ? of_dim(std::integral_constant<int, 64>{})
+  : p.head_dim == 128 ? of_dim(std::integral_constant<int, 128>{})
+                      : of_dim(std::integral_constant<int, 256>{});
   ROOST_RETURN_IF_FAILED(roost::HipStatus(hipGetLastError(), "paged_attention", "mixed attention launch"));
   const PrefillMergeArgs pm = rec.merges != 0 ? PrefillMergeArgsOf(p, rec, dev) : PrefillMergeArgs{};
   const DecodeMergeArgs dm = DecodeMergeArgsOf(p, rec, dev, p.head_dim);
