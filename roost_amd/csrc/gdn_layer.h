@@ -11,6 +11,9 @@ namespace roost_layer {
 // The rules of roost_causal_conv1d_run, reported under `op`.
 RoostStatus AdmitConv(const RoostCausalConv1dParams& p, const char* op);
 
+// The convolution of an admitted CausalConv1d call without its state update.
+RoostStatus RunConv(const RoostCausalConv1dParams& p, hipStream_t s, const char* op);
+
 // The state update of an admitted CausalConv1d call alone: each sequence's slot keeps the last width - 1 inputs of
 // [state, sequence]. Stream-ordered after everything that reads the old state.
 RoostStatus ConvStateUpdate(const RoostCausalConv1dParams& p, hipStream_t s, const char* op);
@@ -23,10 +26,10 @@ RoostStatus AdmitNorm(const RoostGatedRmsNormParams& p, const char* op, bool* ro
 // input and gate rows with the non-temporal hint (the chunk layer, whose norm input the scan stored past the caches).
 RoostStatus RunNorm(const RoostGatedRmsNormParams& p, hipStream_t s, bool stream_input, const char* op);
 
-// RunNorm (input read as cached), then ConvStateUpdate, in one launch where both take their vector forms (a bf16
-// single-pass norm over 128 columns; bf16 input with 2 to 4 taps and 16-byte aligned buffers), else as the two calls.
+// RunNorm, then ConvStateUpdate, in one launch where both take their vector forms (a bf16 single-pass norm over 128
+// columns; bf16 input with 2 to 4 taps and 16-byte aligned buffers), else as the two calls.
 RoostStatus RunNormAndConvState(const RoostGatedRmsNormParams& np, const RoostCausalConv1dParams& cp, hipStream_t s,
-                                const char* op);
+                                bool stream_input, const char* op);
 
 }  // namespace roost_layer
 

@@ -272,6 +272,23 @@ __device__ __forceinline__ int32_t SeqOfToken(const int32_t* cu, uint32_t batch,
   return static_cast<int32_t>(lo);
 }
 
+// SeqOfToken by a whole wavefront (every lane active, t uniform): where the guess fails, 64 entries are compared at a time,
+// one load round for up to 64 sequences and two for up to 4,096 instead of log2(batch) dependent ones.
+__device__ __forceinline__ int32_t SeqOfTokenWave(const int32_t* cu, uint32_t batch, int32_t t, uint32_t tokens) {
+  if (batch <= 1) return 0;
+  const uint32_t g = static_cast<uint32_t>(min<uint64_t>(uint64_t(t) * batch / tokens, batch - 1));
+  if (cu[g] <= t && t < cu[g + 1]) return static_cast<int32_t>(g);
+  uint32_t lo = 0, n = batch;  // the answer lies in [lo, lo + n)
+  while (n > 1) {
+    const uint32_t step = (n + 63) / 64, i = lo + (threadIdx.x & 63) * step;
+    const uint64_t at = __ballot(i < lo + n && cu[min(i, batch)] <= t);  // entries do not fall: a run of ones
+    const uint32_t k = max(__popcll(at), 1) - 1;
+    n = min(step, n - k * step);
+    lo += k * step;
+  }
+  return static_cast<int32_t>(__builtin_amdgcn_readfirstlane(lo));
+}
+
 // A run of kBytes / sizeof(T) consecutive channels: one 4-, 8- or 16-byte load or store.
 template <int kBytes>
 __device__ __forceinline__ void LoadWords(const void* p, uint32_t* w) {
@@ -309,44 +326,67 @@ __device__ __forceinline__ void PackWords(const float* v, uint32_t* w) {
   for (int q = 0; q < kWords; ++q) w[q] = sizeof(T) == 2 ? PackBf16Rne(v[2 * q], v[2 * q + 1]) : __float_as_uint(v[q]);
 }
 
-// Tiled form for a compile-time width and channel vectors of kBytes (kV channels per thread). Workgroup b serves token
-// tile b / cblocks (kConvTile tokens) and channel block b % cblocks (consecutive workgroups cover one row). A thread keeps
-// the last kW - 1 inputs of its channels in registers, so every input row is read once plus a kW - 1 row halo per tile,
-// and loads its kV x kW weights once. Narrow vectors (8 bytes for bf16) keep the register count low enough for eight
-// waves per SIMD, which with long tiles keeps the halo small while the grid still fills the chip several times over.
 // Zeros in device memory, read in place of an absent bias so that the request needs no branch.
 __device__ __align__(16) uint32_t kConvZeros[4] = {0u, 0u, 0u, 0u};
 
-constexpr int kConvTile = 32;
 constexpr int kConvChunk = 4;  // rows requested ahead of the arithmetic
+constexpr int kSub = 4;        // tokens of a boundary tile requested together
 
+// Tiled form for a compile-time width and channel vectors of kBytes (kV channels per thread). Workgroup b serves token
+// tile b / cblocks (`tile` tokens, a multiple of kConvChunk) and channel block b % cblocks (consecutive workgroups cover
+// one row). A thread keeps the last kW - 1 inputs of its channels in registers, so every input row is read once plus a
+// kW - 1 row halo per tile, and loads its kV x kW weights once. Narrow vectors (8 bytes for bf16) keep the register
+// count low enough for eight waves per SIMD. Weights, bias, halo and the first rows are requested before the tile's
+// sequence is looked up and unpacked after, as a request that waits for the lookup adds its round trip to the tile's.
+// A tile that crosses a sequence boundary takes its tokens kConvChunk at a time, every state entry they need requested
+// before any is used. (Taken token by token, each tap re-read, such a tile cost about 1.4 us a token, which set the time of
+// every batch with a length that is no multiple of the tile: at 32 tokens per tile 4 lengths around 3,940 took 136 us
+// against 79.5 now, 6 x 300 70 against 18, 4 x 40 46 against 9; 4 x 4,096 91 against 83. 6,144 channels, bf16.)
 template <typename T, int kW, int kBytes>
-__global__ void __launch_bounds__(256) ConvTileKernel(ConvArgs a, uint32_t cblocks) {
+__global__ void __launch_bounds__(256) ConvTileKernel(ConvArgs a, uint32_t cblocks, int32_t tile) {
   constexpr int kWords = kBytes / 4;
   constexpr int kV = kBytes / static_cast<int>(sizeof(T));
-  const uint32_t tile = blockIdx.x / cblocks;
-  const int32_t t_begin = static_cast<int32_t>(tile) * kConvTile;
-  const uint32_t c0 = ((blockIdx.x - tile * cblocks) * blockDim.x + threadIdx.x) * kV;
-  if (c0 >= a.channels) return;
-  const int32_t t_end = min(t_begin + kConvTile, static_cast<int32_t>(a.tokens));
-  const T* x = static_cast<const T*>(a.x);
-  auto row_at = [&](int32_t t, float* v) {
-    uint32_t q[kWords];
-    LoadWords<kBytes>(x + static_cast<uint64_t>(t) * a.channels + c0, q);
-    UnpackWords<T, kWords>(q, v);
+  constexpr int sl = kW - 1;
+  const uint32_t bt = blockIdx.x / cblocks;
+  const int32_t t_begin = static_cast<int32_t>(bt) * tile;
+  // Threads past the last channels repeat the last ones, so that every lane takes part in the sequence lookups.
+  const uint32_t c0 = min(((blockIdx.x - bt * cblocks) * blockDim.x + threadIdx.x) * kV, a.channels - kV);
+  const int32_t t_end = min(t_begin + tile, static_cast<int32_t>(a.tokens));
+  const T* x = static_cast<const T*>(a.x) + c0;
+  // Rows stream in with the non-temporal hint (Qwen3.5's [16384, 6144] projection: 74.6 against 86.0 us); the halo rows,
+  // which the tile before also reads, keep plain loads.
+  auto fetch = [&](int32_t t0, uint32_t (*r)[kWords]) {
+#pragma unroll
+    for (int i = 0; i < kConvChunk; ++i) {
+      LoadWordsNt<kBytes>(x + static_cast<uint64_t>(min(t0 + i, t_end - 1)) * a.channels, r[i]);
+    }
   };
   // Weights of channels c0 .. c0 + kV - 1: kV * kW consecutive elements, channel-major (kBytes-aligned: the launcher
-  // checks the base). Weights and bias are requested as words without a branch (no bias: zeros from kConvZeros) and
-  // unpacked after: a request inside a branch, used there, waited for everything before it.
+  // checks the base).
+  uint32_t rows[kConvChunk][kWords], next[kConvChunk][kWords], halo[sl][kWords], qw[kW][kWords], qb[kWords];
+  fetch(t_begin, rows);
+#pragma unroll
+  for (int j = 0; j < sl; ++j) {
+    LoadWords<kBytes>(x + static_cast<uint64_t>(max(t_begin - sl + j, 0)) * a.channels, halo[j]);
+  }
+  const T* wrow = static_cast<const T*>(a.w) + static_cast<uint64_t>(c0) * kW;
+#pragma unroll
+  for (int q = 0; q < kW; ++q) LoadWords<kBytes>(wrow + q * kV, qw[q]);
+  LoadWords<kBytes>(a.bias != nullptr ? static_cast<const T*>(a.bias) + c0 : reinterpret_cast<const T*>(kConvZeros), qb);
+  const int32_t seq0 = SeqOfTokenWave(a.cu, a.batch, t_begin, a.tokens);
+  const int32_t s0 = a.cu[seq0], s1 = a.cu[seq0 + 1];
+  const bool pairs = a.state_t == ROOST_DTYPE_BF16 && (reinterpret_cast<uintptr_t>(a.state) & 3) == 0;
+  auto slot_of = [&](int32_t seq) {
+    const int32_t slot = a.slots[seq];
+    return slot >= 0 && static_cast<uint64_t>(slot) < a.pool_slots ? slot : -1;
+  };
+  auto state_at = [&](int32_t slot, int e, int i) {  // a slot outside the pool reads zeros
+    return slot < 0 ? 0.0f
+                    : LoadF(a.state, a.state_t, (static_cast<uint64_t>(slot) * a.channels + c0 + e) * sl + i);
+  };
   float w[kV][kW];
   float bias[kV];
   {
-    uint32_t qw[kW][kWords], qb[kWords];
-    const T* wrow = static_cast<const T*>(a.w) + static_cast<uint64_t>(c0) * kW;
-#pragma unroll
-    for (int q = 0; q < kW; ++q) LoadWords<kBytes>(wrow + q * kV, qw[q]);
-    LoadWords<kBytes>(a.bias != nullptr ? static_cast<const T*>(a.bias) + c0 : reinterpret_cast<const T*>(kConvZeros),
-                      qb);
     float flat[kV * kW];
 #pragma unroll
     for (int q = 0; q < kW; ++q) UnpackWords<T, kWords>(qw[q], flat + q * kV);
@@ -356,52 +396,38 @@ __global__ void __launch_bounds__(256) ConvTileKernel(ConvArgs a, uint32_t cbloc
       for (int j = 0; j < kW; ++j) w[e][j] = flat[e * kW + j];
     UnpackWords<T, kWords>(qb, bias);
   }
-
-  const int32_t seq0 = SeqOfToken(a.cu, a.batch, t_begin, a.tokens);
-  const int32_t s0 = a.cu[seq0], s1 = a.cu[seq0 + 1];
-  // Entry i of [state (kW - 1), inputs] of sequence `seq` (first token `first`) for channels c0.., as floats.
-  auto history = [&](int32_t seq, int32_t first, int32_t i, float* v) {
-    if (i < kW - 1) {
-      const int32_t slot = a.slots[seq];
-      const bool ok = slot >= 0 && static_cast<uint64_t>(slot) < a.pool_slots;
-      const uint64_t so = static_cast<uint64_t>(ok ? slot : 0) * a.channels * (kW - 1);
-#pragma unroll
-      for (int e = 0; e < kV; ++e) v[e] = ok ? LoadF(a.state, a.state_t, so + (c0 + e) * (kW - 1) + i) : 0.0f;
-    } else {
-      row_at(first + i - (kW - 1), v);
-    }
-  };
   auto emit = [&](int32_t t, const float (*taps)[kV], const float* cur) {
     float y[kV];
 #pragma unroll
     for (int e = 0; e < kV; ++e) {
       float acc = bias[e];
 #pragma unroll
-      for (int j = 0; j < kW - 1; ++j) acc = fmaf(w[e][j], taps[j][e], acc);
-      acc = fmaf(w[e][kW - 1], cur[e], acc);
+      for (int j = 0; j < sl; ++j) acc = fmaf(w[e][j], taps[j][e], acc);
+      acc = fmaf(w[e][sl], cur[e], acc);
       y[e] = a.silu ? SiluF(acc) : acc;
     }
     uint32_t q[kWords];
     PackWords<T, kWords>(y, q);
     StoreWords<kBytes>(static_cast<T*>(a.y) + static_cast<uint64_t>(t) * a.channels + c0, q);
   };
-  float h[kW - 1][kV];  // the window: h[kW - 2] is the newest input
+  float h[sl][kV];  // the window: h[sl - 1] is the newest input
+#pragma unroll
+  for (int j = 0; j < sl; ++j) UnpackWords<T, kWords>(halo[j], h[j]);
 
   if (t_begin >= s0 && t_end <= s1) {
-    // The whole tile lies in one sequence (every tile but those at sequence boundaries): one window load, then a
-    // straight-line slide over the tile's rows, the next kConvChunk rows requested before the current ones are computed.
-    // The rows stream in with the non-temporal hint (Qwen3.5's [16384, 6144] projection: 74.6 against 86.0 us); the
-    // window's halo rows, which the tile before also reads, keep plain loads.
-    auto fetch = [&](int32_t t0, uint32_t (*r)[kWords]) {
+    // The whole tile lies in one sequence: a straight-line slide over the tile's rows, the next kConvChunk rows
+    // requested before the current ones are computed.
+    if (t_begin - s0 < sl) {  // the sequence's first tokens: the window reaches into the state
+      const int32_t slot = slot_of(seq0);
 #pragma unroll
-      for (int i = 0; i < kConvChunk; ++i) {
-        LoadWordsNt<kBytes>(x + static_cast<uint64_t>(min(t0 + i, t_end - 1)) * a.channels + c0, r[i]);
+      for (int j = 0; j < sl; ++j) {
+        const int32_t i = t_begin - s0 + j;  // entry of [state, inputs]
+        if (i < sl) {
+#pragma unroll
+          for (int e = 0; e < kV; ++e) h[j][e] = state_at(slot, e, i);
+        }
       }
-    };
-    uint32_t rows[kConvChunk][kWords], next[kConvChunk][kWords];
-    fetch(t_begin, rows);
-#pragma unroll
-    for (int j = 0; j < kW - 1; ++j) history(seq0, s0, t_begin - s0 + j, h[j]);
+    }
 #pragma unroll 1
     for (int32_t tc = t_begin; tc < t_end; tc += kConvChunk) {
       if (tc + kConvChunk < t_end) fetch(tc + kConvChunk, next);
@@ -413,11 +439,11 @@ __global__ void __launch_bounds__(256) ConvTileKernel(ConvArgs a, uint32_t cbloc
         UnpackWords<T, kWords>(rows[i], cur);
         emit(t, h, cur);
 #pragma unroll
-        for (int j = 0; j + 1 < kW - 1; ++j)
+        for (int j = 0; j + 1 < sl; ++j)
 #pragma unroll
           for (int e = 0; e < kV; ++e) h[j][e] = h[j + 1][e];
 #pragma unroll
-        for (int e = 0; e < kV; ++e) h[kW - 2][e] = cur[e];
+        for (int e = 0; e < kV; ++e) h[sl - 1][e] = cur[e];
       }
 #pragma unroll
       for (int i = 0; i < kConvChunk; ++i)
@@ -426,20 +452,81 @@ __global__ void __launch_bounds__(256) ConvTileKernel(ConvArgs a, uint32_t cbloc
     }
     return;
   }
-  // A tile that crosses a sequence boundary (or holds tokens outside every sequence): token by token, each tap read
-  // directly from the state or the inputs (the sequence is uniform across the workgroup: every thread shares the token).
-  int32_t seq = seq0;
-#pragma unroll 1
-  for (int32_t t = t_begin; t < t_end; ++t) {
-    while (seq + 1 < static_cast<int32_t>(a.batch) && a.cu[seq + 1] <= t) ++seq;
-    const int32_t first = a.cu[seq];
-    if (t < first || t >= a.cu[seq + 1]) continue;  // a token outside every sequence: no output
-    const int32_t rel = t - first;
+  // A tile that crosses a sequence boundary (or holds tokens outside every sequence). The window slides over the raw rows;
+  // at a sequence's first token it becomes the sequence's state. The sequence is uniform across the workgroup: every
+  // thread shares the token.
+  // Lane l holds the end of sequence sb + l and its slot, so that a token's sequence costs no load.
+  int32_t sb = seq0, base = s0;
+  int32_t ends, lane_slot;
+  auto window = [&]() {
+    const int32_t l = sb + static_cast<int32_t>(threadIdx.x & 63), last = static_cast<int32_t>(a.batch) - 1;
+    ends = a.cu[min(l, last) + 1];
+    lane_slot = a.slots[min(l, last)];
+  };
+  window();
+  if (t_begin > s0 && t_begin - s0 < sl && t_begin < s1) {  // the tile starts inside a sequence's first tokens
+    const int32_t slot = slot_of(seq0);
 #pragma unroll
-    for (int j = 0; j < kW - 1; ++j) history(seq, first, rel + j, h[j]);
-    float cur[kV];
-    row_at(t, cur);
-    emit(t, h, cur);
+    for (int j = 0; j < sl; ++j) {
+      if (t_begin - s0 + j < sl) {
+#pragma unroll
+        for (int e = 0; e < kV; ++e) h[j][e] = state_at(slot, e, t_begin - s0 + j);
+      }
+    }
+  }
+  constexpr int kSw = kV * sl / 2;  // state words of a token (bf16 pairs)
+#pragma unroll 1
+  for (int32_t tc = t_begin; tc < t_end; tc += kSub) {
+    int32_t live = 0, starts = 0;     // bit i: token tc + i lies in a sequence; is its first
+    int32_t slots[kSub];
+    uint32_t sw[kSub][kSw], cur_w[kSub][kWords];
+#pragma unroll
+    for (int i = 0; i < kSub; ++i) {
+      const int32_t t = min(tc + i, t_end - 1);
+      LoadWords<kBytes>(x + static_cast<uint64_t>(t) * a.channels, cur_w[i]);
+      int32_t k = __popcll(__ballot(ends <= t));  // sequences of the window that end at or before t
+      while (k == 64 && sb + 64 < static_cast<int32_t>(a.batch)) {
+        base = __builtin_amdgcn_readlane(ends, 63);
+        sb += 64;
+        window();
+        k = __popcll(__ballot(ends <= t));
+      }
+      const int32_t first = k == 0 ? base : __builtin_amdgcn_readlane(ends, k - 1);
+      const bool in = tc + i < t_end && k < 64 && t >= first;  // past the last sequence's end every lane counts
+      live |= static_cast<int32_t>(in) << i;
+      slots[i] = -1;
+      if (in && t == first) {
+        starts |= 1 << i;
+        const int32_t slot = __builtin_amdgcn_readlane(lane_slot, k);
+        slots[i] = slot >= 0 && static_cast<uint64_t>(slot) < a.pool_slots ? slot : -1;
+        if (pairs) {
+          const auto* sp = reinterpret_cast<const uint32_t*>(
+              static_cast<const uint16_t*>(a.state) + (static_cast<uint64_t>(max(slots[i], 0)) * a.channels + c0) * sl);
+#pragma unroll
+          for (int k = 0; k < kSw; ++k) sw[i][k] = sp[k];
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kSub; ++i) {
+      float cur[kV];
+      UnpackWords<T, kWords>(cur_w[i], cur);
+      if ((starts >> i) & 1) {
+#pragma unroll
+        for (int k = 0; k < kV * sl; ++k) {
+          const float f = pairs ? ((k & 1) ? Bf16HiToF32(sw[i][k / 2]) : Bf16LoToF32(sw[i][k / 2]))
+                                : state_at(slots[i], k / sl, k % sl);
+          h[k % sl][k / sl] = slots[i] < 0 ? 0.0f : f;
+        }
+      }
+      if ((live >> i) & 1) emit(tc + i, h, cur);
+#pragma unroll
+      for (int j = 0; j + 1 < sl; ++j)
+#pragma unroll
+        for (int e = 0; e < kV; ++e) h[j][e] = h[j + 1][e];
+#pragma unroll
+      for (int e = 0; e < kV; ++e) h[sl - 1][e] = cur[e];
+    }
   }
 }
 
@@ -1028,16 +1115,16 @@ ConvArgs MakeConvArgs(const RoostCausalConv1dParams& p) {
 }
 
 // A layer call's last two steps in one launch: workgroups [0, norm_blocks) run GatedRmsNormRowKernel's rows (bf16,
-// the input read as cached), the rest ConvStateVecKernel's (sequence, channel block) pairs, state_by blocks per
+// the input streamed or read as cached), the rest ConvStateVecKernel's (sequence, channel block) pairs, state_by blocks per
 // sequence. The two touch disjoint memory, so their order within the launch does not matter.
-template <int kW>
+template <int kW, bool kStream>
 __global__ void __launch_bounds__(256) LayerTailKernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gate,
                                                        const void* __restrict__ weight, uint32_t w_t,
                                                        uint16_t* __restrict__ out, uint64_t rows, uint32_t lanes,
                                                        float eps, uint32_t norm_blocks, ConvArgs a, uint32_t state_by) {
   const uint32_t bx = blockIdx.x;
   if (bx < norm_blocks) {
-    GatedRmsNormRows<uint16_t, kRmsRows, false>(x, gate, weight, w_t, out, rows, 128, lanes, eps, bx);
+    GatedRmsNormRows<uint16_t, kRmsRows, kStream>(x, gate, weight, w_t, out, rows, 128, lanes, eps, bx);
   } else {
     ConvStateVecBlock<kW>(a, (bx - norm_blocks) / state_by, (bx - norm_blocks) % state_by);
   }
@@ -1065,7 +1152,7 @@ RoostStatus roost_layer::ConvStateUpdate(const RoostCausalConv1dParams& p, hipSt
 }
 
 RoostStatus roost_layer::RunNormAndConvState(const RoostGatedRmsNormParams& np, const RoostCausalConv1dParams& cp,
-                                             hipStream_t s, const char* op) {
+                                             hipStream_t s, bool stream_input, const char* op) {
   const NormShape f = NormForm(np);
   const bool state_vec = cp.batch != 0 && cp.tokens != 0 && cp.width >= 2 && cp.width <= 4 &&
                          cp.input.dtype == ROOST_DTYPE_BF16 && cp.channels % 8 == 0 &&
@@ -1073,7 +1160,7 @@ RoostStatus roost_layer::RunNormAndConvState(const RoostGatedRmsNormParams& np, 
                          cp.channels / 8 <= 65535u * 256u;
   const bool norm_rows = np.rows != 0 && np.input.dtype == ROOST_DTYPE_BF16 && f.single && np.dim == 128;
   if (!state_vec || !norm_rows) {
-    ROOST_RETURN_IF_FAILED(RunNorm(np, s, false, op));
+    ROOST_RETURN_IF_FAILED(RunNorm(np, s, stream_input, op));
     return ConvStateUpdate(cp, s, op);
   }
   const uint64_t rows_per_block = 4ull * (64 / f.lanes) * kRmsRows;
@@ -1081,7 +1168,7 @@ RoostStatus roost_layer::RunNormAndConvState(const RoostGatedRmsNormParams& np, 
   const uint32_t state_by = Blocks(cp.channels / 8, 256);
   const uint64_t total = norm_blocks + uint64_t{cp.batch} * state_by;
   if (total > 0xFFFFFFFFull) {
-    ROOST_RETURN_IF_FAILED(RunNorm(np, s, false, op));
+    ROOST_RETURN_IF_FAILED(RunNorm(np, s, stream_input, op));
     return ConvStateUpdate(cp, s, op);
   }
   const ConvArgs a = MakeConvArgs(cp);
@@ -1090,15 +1177,80 @@ RoostStatus roost_layer::RunNormAndConvState(const RoostGatedRmsNormParams& np, 
   auto* o = static_cast<uint16_t*>(np.output.address);
   const dim3 grid(static_cast<uint32_t>(total));
   const uint32_t nb = static_cast<uint32_t>(norm_blocks);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, x, g, np.weight.address, np.weight.dtype, o, uint64_t{np.rows},
+                       f.lanes, np.eps, nb, a, state_by);
+  };
   switch (cp.width) {
-    case 2: hipLaunchKernelGGL(LayerTailKernel<2>, grid, dim3(256), 0, s, x, g, np.weight.address, np.weight.dtype, o,
-                               uint64_t{np.rows}, f.lanes, np.eps, nb, a, state_by); break;
-    case 3: hipLaunchKernelGGL(LayerTailKernel<3>, grid, dim3(256), 0, s, x, g, np.weight.address, np.weight.dtype, o,
-                               uint64_t{np.rows}, f.lanes, np.eps, nb, a, state_by); break;
-    default: hipLaunchKernelGGL(LayerTailKernel<4>, grid, dim3(256), 0, s, x, g, np.weight.address, np.weight.dtype, o,
-                                uint64_t{np.rows}, f.lanes, np.eps, nb, a, state_by); break;
+    case 2: stream_input ? launch(LayerTailKernel<2, true>) : launch(LayerTailKernel<2, false>); break;
+    case 3: stream_input ? launch(LayerTailKernel<3, true>) : launch(LayerTailKernel<3, false>); break;
+    default: stream_input ? launch(LayerTailKernel<4, true>) : launch(LayerTailKernel<4, false>); break;
   }
   return roost::HipStatus(hipGetLastError(), op, "norm and state launch");
+}
+
+// Tokens per tile of the tiled convolution: 8, or 4 where there are few tokens (latency) or many sequence boundaries.
+// Measured over 6,144 channels, width 4 (us, with the state update): 4 lengths around 3,940 79.5 at 8, 91 at 4, 85 at 16,
+// 98 at 32; 1,777 tokens 17.1 / 17.4 / 18.7 / 21.5; 4 x 40 9.8 at 8, 8.6 at 4; 48 one-token sequences beside 2 x 512 20.2
+// at 8, 16.5 at 4.
+static int32_t ConvTile(const RoostCausalConv1dParams& p) {
+  return p.tokens >= 1024 && uint64_t{p.tokens} >= uint64_t{p.batch} * 32 ? 8 : 4;
+}
+// Mean tokens per sequence from which the tiled form serves a bf16 call: at 17 it took 16.7 us against 19.2 for the
+// short-sequence form (60 one-token sequences beside 500 and 520 tokens), at 9 14.8 against 13.7.
+constexpr uint32_t kConvMinMean = 16;
+
+RoostStatus roost_layer::RunConv(const RoostCausalConv1dParams& p, hipStream_t s, const char* op) {
+  if (p.batch == 0 || p.tokens == 0) return ROOST_STATUS_OK;
+  const uint32_t act = p.input.dtype;
+  const ConvArgs a = MakeConvArgs(p);
+  const uint64_t v = 16 / ElemBytes(act);
+  const bool vec = p.channels % v == 0 && roost::IsAligned(p.input.address, 16) && roost::IsAligned(p.output.address, 16);
+  const uint32_t per_thread = vec ? static_cast<uint32_t>(v) : 1u;
+  const bool bf = act == ROOST_DTYPE_BF16;
+  // The tiled kernel takes 8-byte channel vectors (4 bf16 or 2 f32 channels) when the channel count and the
+  // buffers allow them.
+  const bool vec8 = p.channels % (8 / ElemBytes(act)) == 0 && roost::IsAligned(p.input.address, 8) &&
+                    roost::IsAligned(p.output.address, 8) && roost::IsAligned(p.weight.address, 8) &&
+                    roost::IsAligned(p.bias.address, 8);
+  const uint32_t cblocks = Blocks(p.channels / (8 / ElemBytes(act)), 256);
+  const int32_t tile = ConvTile(p);
+  const uint64_t tiled_blocks = uint64_t{cblocks} * Blocks(p.tokens, static_cast<uint32_t>(tile));
+  // Tiles pay off when sequences are long; a batch of short ones (a decode step: every tile would cross sequences)
+  // runs on the one-thread-per-token form.
+  const bool long_seqs = uint64_t{p.tokens} >= uint64_t{p.batch} * kConvMinMean;
+  const bool short_form = !long_seqs && bf && p.width >= 2 && p.width <= 4 && p.channels % 8 == 0 &&
+                          roost::IsAligned(p.input.address, 16) && roost::IsAligned(p.output.address, 16) &&
+                          roost::IsAligned(p.weight.address, 16) && roost::IsAligned(a.bias, 16) &&
+                          roost::IsAligned(p.conv_state.address, 16) && p.channels / 8 <= 65535u * 256u;
+  if (short_form) {
+    const dim3 grid(p.tokens, Blocks(p.channels / 8, 256));
+    switch (p.width) {
+      case 2: hipLaunchKernelGGL(ConvShortKernel<2>, grid, dim3(256), 0, s, a); break;
+      case 3: hipLaunchKernelGGL(ConvShortKernel<3>, grid, dim3(256), 0, s, a); break;
+      default: hipLaunchKernelGGL(ConvShortKernel<4>, grid, dim3(256), 0, s, a); break;
+    }
+  } else if (vec8 && long_seqs && p.width >= 2 && p.width <= 4 && tiled_blocks <= 0xFFFFFFFFull) {
+    const dim3 tiled(static_cast<uint32_t>(tiled_blocks));
+    switch (p.width * 2 + (bf ? 1 : 0)) {
+      case 5: hipLaunchKernelGGL((ConvTileKernel<uint16_t, 2, 8>), tiled, dim3(256), 0, s, a, cblocks, tile); break;
+      case 7: hipLaunchKernelGGL((ConvTileKernel<uint16_t, 3, 8>), tiled, dim3(256), 0, s, a, cblocks, tile); break;
+      case 9: hipLaunchKernelGGL((ConvTileKernel<uint16_t, 4, 8>), tiled, dim3(256), 0, s, a, cblocks, tile); break;
+      case 4: hipLaunchKernelGGL((ConvTileKernel<float, 2, 8>), tiled, dim3(256), 0, s, a, cblocks, tile); break;
+      case 6: hipLaunchKernelGGL((ConvTileKernel<float, 3, 8>), tiled, dim3(256), 0, s, a, cblocks, tile); break;
+      default: hipLaunchKernelGGL((ConvTileKernel<float, 4, 8>), tiled, dim3(256), 0, s, a, cblocks, tile); break;
+    }
+  } else {
+    const dim3 grid(p.tokens, Blocks(roost::CeilDiv(p.channels, per_thread), 256));
+    if (bf) {
+      if (vec) hipLaunchKernelGGL((ConvKernel<uint16_t, true>), grid, dim3(256), 0, s, a);
+      else hipLaunchKernelGGL((ConvKernel<uint16_t, false>), grid, dim3(256), 0, s, a);
+    } else {
+      if (vec) hipLaunchKernelGGL((ConvKernel<float, true>), grid, dim3(256), 0, s, a);
+      else hipLaunchKernelGGL((ConvKernel<float, false>), grid, dim3(256), 0, s, a);
+    }
+  }
+  return roost::HipStatus(hipGetLastError(), op, "convolution launch");
 }
 
 extern "C" ROOST_API RoostStatus roost_causal_conv1d_run(RoostContext* ctx, const void* params, const RoostWorkspace*,
@@ -1110,56 +1262,8 @@ extern "C" ROOST_API RoostStatus roost_causal_conv1d_run(RoostContext* ctx, cons
   const auto& p = *pp;
   return roost::CatchAll(kOp, [&]() -> RoostStatus {
     ROOST_RETURN_IF_FAILED(roost_layer::AdmitConv(p, kOp));
-    if (p.batch == 0 || p.tokens == 0) return ROOST_STATUS_OK;
-    const uint32_t act = p.input.dtype;
-    const ConvArgs a = MakeConvArgs(p);
-    const uint64_t v = 16 / ElemBytes(act);
-    const bool vec = p.channels % v == 0 && roost::IsAligned(p.input.address, 16) && roost::IsAligned(p.output.address, 16);
-    const uint32_t per_thread = vec ? static_cast<uint32_t>(v) : 1u;
     hipStream_t s = roost::Stream(stream);
-    const bool bf = act == ROOST_DTYPE_BF16;
-    // The tiled kernel takes 8-byte channel vectors (4 bf16 or 2 f32 channels) when the channel count and the
-    // buffers allow them.
-    const bool vec8 = p.channels % (8 / ElemBytes(act)) == 0 && roost::IsAligned(p.input.address, 8) &&
-                      roost::IsAligned(p.output.address, 8) && roost::IsAligned(p.weight.address, 8) &&
-                      roost::IsAligned(p.bias.address, 8);
-    const uint32_t cblocks = Blocks(p.channels / (8 / ElemBytes(act)), 256);
-    const uint64_t tiled_blocks = uint64_t{cblocks} * Blocks(p.tokens, kConvTile);
-    // Tiles of kConvTile tokens pay off when sequences are long; a batch of short ones (a decode step: every tile
-    // would cross sequences and take the per-token path) runs on the one-thread-per-token form.
-    const bool long_seqs = uint64_t{p.tokens} >= uint64_t{p.batch} * kConvTile;
-    const bool short_form = !long_seqs && bf && p.width >= 2 && p.width <= 4 && p.channels % 8 == 0 &&
-                            roost::IsAligned(p.input.address, 16) && roost::IsAligned(p.output.address, 16) &&
-                            roost::IsAligned(p.weight.address, 16) && roost::IsAligned(a.bias, 16) &&
-                            roost::IsAligned(p.conv_state.address, 16) && p.channels / 8 <= 65535u * 256u;
-    if (short_form) {
-      const dim3 grid(p.tokens, Blocks(p.channels / 8, 256));
-      switch (p.width) {
-        case 2: hipLaunchKernelGGL(ConvShortKernel<2>, grid, dim3(256), 0, s, a); break;
-        case 3: hipLaunchKernelGGL(ConvShortKernel<3>, grid, dim3(256), 0, s, a); break;
-        default: hipLaunchKernelGGL(ConvShortKernel<4>, grid, dim3(256), 0, s, a); break;
-      }
-    } else if (vec8 && long_seqs && p.width >= 2 && p.width <= 4 && tiled_blocks <= 0xFFFFFFFFull) {
-      const dim3 tiled(static_cast<uint32_t>(tiled_blocks));
-      switch (p.width * 2 + (bf ? 1 : 0)) {
-        case 5: hipLaunchKernelGGL((ConvTileKernel<uint16_t, 2, 8>), tiled, dim3(256), 0, s, a, cblocks); break;
-        case 7: hipLaunchKernelGGL((ConvTileKernel<uint16_t, 3, 8>), tiled, dim3(256), 0, s, a, cblocks); break;
-        case 9: hipLaunchKernelGGL((ConvTileKernel<uint16_t, 4, 8>), tiled, dim3(256), 0, s, a, cblocks); break;
-        case 4: hipLaunchKernelGGL((ConvTileKernel<float, 2, 8>), tiled, dim3(256), 0, s, a, cblocks); break;
-        case 6: hipLaunchKernelGGL((ConvTileKernel<float, 3, 8>), tiled, dim3(256), 0, s, a, cblocks); break;
-        default: hipLaunchKernelGGL((ConvTileKernel<float, 4, 8>), tiled, dim3(256), 0, s, a, cblocks); break;
-      }
-    } else {
-      const dim3 grid(p.tokens, Blocks(roost::CeilDiv(p.channels, per_thread), 256));
-      if (bf) {
-        if (vec) hipLaunchKernelGGL((ConvKernel<uint16_t, true>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((ConvKernel<uint16_t, false>), grid, dim3(256), 0, s, a);
-      } else {
-        if (vec) hipLaunchKernelGGL((ConvKernel<float, true>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((ConvKernel<float, false>), grid, dim3(256), 0, s, a);
-      }
-    }
-    ROOST_RETURN_IF_FAILED(roost::HipStatus(hipGetLastError(), kOp, "convolution launch"));
+    ROOST_RETURN_IF_FAILED(roost_layer::RunConv(p, s, kOp));
     return roost_layer::ConvStateUpdate(p, s, kOp);
   });
 }
