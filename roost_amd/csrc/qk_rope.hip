@@ -497,6 +497,78 @@ __global__ void __launch_bounds__(256) RopeKernel(T* q, T* k, RopeSpec rs, uint3
   }
 }
 
+// Rope of vector rows whose NeoX halves are whole chunks, a power of two of them (every Qwen and Llama shape). A thread's
+// item is one pair of chunks of a row, (c, c + R/2): both sides of eight (f32: four) rotations in its own registers, so
+// only the R rotated elements are read and written (a quarter of Qwen3.5's rows) and nothing passes between lanes. The
+// first kAhead items are requested before the angle table is built. Same arithmetic as RopeRowChunks.
+// Bound by the two requests' round trip and, at large calls, HBM. 8,192 tokens x 10 heads: 64 of 256 dims 19.7 -> 6.4 us
+// (5.1 with the angles left out, so they cost 1.3), all 256 22.3 -> 20.3 (84 MB read and written); 40
+// heads x 128 dims 38.7 -> 35.7 (4.7 TB/s); 1,072 tokens at 64 of 256 6.9 -> 3.9. Tokens per workgroup 4 / 8 / 16 / 32 at
+// 8,192 tokens, 64 of 256: 8.5 / 6.4 / 6.0 / 6.9; at 300 tokens of 40 x 128 1 is best (16: 10.5 against 4.4).
+constexpr int kRopeAhead = 4;
+
+template <typename T, int kV>
+__global__ void __launch_bounds__(256) RopePairsKernel(T* q, T* k, RopeSpec rs, uint32_t tokens, uint32_t q_heads,
+                                                       uint32_t kv_heads, uint32_t head_dim, uint32_t lane_shift,
+                                                       uint32_t tpb) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  const uint32_t heads = q_heads + kv_heads, half = rs.rot / 2, lanes = 1u << lane_shift;
+  auto* freq = reinterpret_cast<double*>(lds_raw);
+  auto* cs = reinterpret_cast<float2*>(lds_raw + uint64_t{half} * 8);
+  const TokenRows tr = BlockTokens(tokens, tpb, heads);
+  const uint32_t items = tr.rows << lane_shift;
+  struct Item {
+    T* x;          // the first chunk; the second half elements further
+    uint32_t pair;  // its first (cos, sin) entry
+  };
+  auto item = [&](uint32_t idx) {  // past the last item: the last again (never stored)
+    const uint32_t i = min(idx, items - 1), c = i & (lanes - 1), r = i >> lane_shift;
+    const uint32_t lt = r / heads, h = r - lt * heads;
+    const uint64_t t = tr.t0 + lt;
+    T* row = h < q_heads ? q + (t * q_heads + h) * head_dim : k + (t * kv_heads + (h - q_heads)) * head_dim;
+    return Item{row + c * kV, lt * half + c * kV};
+  };
+  uint4 w[kRopeAhead][2];
+  auto fetch = [&](uint32_t idx) {
+#pragma unroll
+    for (int a = 0; a < kRopeAhead; ++a) {
+      const Item it = item(idx + 256 * a);
+      w[a][0] = *reinterpret_cast<const uint4*>(it.x);
+      w[a][1] = *reinterpret_cast<const uint4*>(it.x + half);
+    }
+  };
+  fetch(threadIdx.x);
+  BuildAngles(rs, tr.t0, tr.count, freq, cs);
+  for (uint32_t idx = threadIdx.x; idx < items; idx += 256 * kRopeAhead) {
+#pragma unroll
+    for (int a = 0; a < kRopeAhead; ++a) {
+      const Item it = item(idx + 256 * a);
+      const auto* a4 = reinterpret_cast<const float4*>(cs + it.pair);
+      float x1[kV], x2[kV], y1[kV], y2[kV];
+      const uint32_t u[4] = {w[a][0].x, w[a][0].y, w[a][0].z, w[a][0].w};
+      const uint32_t v[4] = {w[a][1].x, w[a][1].y, w[a][1].z, w[a][1].w};
+#pragma unroll
+      for (int e = 0; e < kV; ++e) {
+        x1[e] = sizeof(T) == 2 ? ((e & 1) ? Bf16HiToF32(u[e >> 1]) : Bf16LoToF32(u[e >> 1])) : __uint_as_float(u[e & 3]);
+        x2[e] = sizeof(T) == 2 ? ((e & 1) ? Bf16HiToF32(v[e >> 1]) : Bf16LoToF32(v[e >> 1])) : __uint_as_float(v[e & 3]);
+      }
+#pragma unroll
+      for (int p = 0; p < kV / 2; ++p) {
+        const float4 cc = a4[p];  // (cos, sin) of pairs 2p and 2p + 1
+        y1[2 * p] = fmaf(x1[2 * p], cc.x, -(x2[2 * p] * cc.y));
+        y2[2 * p] = fmaf(x2[2 * p], cc.x, x1[2 * p] * cc.y);
+        y1[2 * p + 1] = fmaf(x1[2 * p + 1], cc.z, -(x2[2 * p + 1] * cc.w));
+        y2[2 * p + 1] = fmaf(x2[2 * p + 1], cc.z, x1[2 * p + 1] * cc.w);
+      }
+      if (idx + 256 * a < items) {
+        StoreChunk<T, kV>(it.x, y1);
+        StoreChunk<T, kV>(it.x + half, y2);
+      }
+    }
+    if (idx + 256 * kRopeAhead < items) fetch(idx + 256 * kRopeAhead);
+  }
+}
+
 // ---- QkvQkNormRopeCacheWrite: rows are (token, head) over q, k and v heads of each [q | k | v] row. ----------------
 struct QkvArgs {
   const void* qkv;
@@ -670,6 +742,12 @@ uint32_t ChunkPairs(const RowShape& s, uint32_t elem_bytes, uint32_t rot, bool i
 uint32_t Blocks(uint64_t items, uint32_t per) { return static_cast<uint32_t>(roost::CeilDiv(items, per)); }
 // Tokens per rope workgroup: about a thousand workgroups for large calls, one token each for small ones.
 uint32_t TokensPerBlock(uint32_t tokens) { return std::min<uint32_t>(kMaxTpb, std::max<uint32_t>(1, tokens / 1024)); }
+// Tokens per workgroup of RopePairsKernel: enough for an item per thread, about a thousand workgroups for large calls, an
+// angle table of at most 32 KB.
+uint32_t RopePairTokens(uint32_t tokens, uint32_t items_per_token, uint32_t half) {
+  const uint32_t want = std::max<uint32_t>(Blocks(256, items_per_token), Blocks(tokens, 1024));
+  return std::max<uint32_t>(1, std::min<uint32_t>(want, 4096 / half));
+}
 uint32_t GridFor(uint64_t rows, uint32_t g) {
   return static_cast<uint32_t>(roost::CeilDiv(rows, uint64_t{4} * (64 / g)));
 }
@@ -815,6 +893,21 @@ extern "C" ROOST_API RoostStatus roost_rope_run(RoostContext* ctx, const void* p
                      RowsAligned16(p.k.address, uint64_t{p.kv_heads} * p.head_dim, p.head_dim, eb);
     const RowShape s = ShapeFor(p.head_dim, eb, a16);
     rs.chunk_pairs = ChunkPairs(s, eb, rot, p.interleaved != 0u);
+    const uint32_t lanes = rot * eb / 32;  // chunk pairs of a row
+    if (rs.chunk_pairs != 0u && !rs.interleaved && roost::IsPow2(lanes)) {
+      const uint32_t per_token = (p.q_heads + p.kv_heads) * lanes;
+      const uint32_t tpb = RopePairTokens(p.tokens, per_token, rot / 2);
+      const uint32_t shift = static_cast<uint32_t>(__builtin_ctz(lanes));
+      auto launch = [&](auto t_tag, auto kv) {
+        using T = decltype(t_tag);
+        hipLaunchKernelGGL((RopePairsKernel<T, decltype(kv)::value>), dim3(Blocks(p.tokens, tpb)), dim3(256),
+                           uint64_t{rot / 2} * 8 * (1 + tpb), roost::Stream(stream), static_cast<T*>(p.q.address),
+                           static_cast<T*>(p.k.address), rs, p.tokens, p.q_heads, p.kv_heads, p.head_dim, shift, tpb);
+      };
+      dt == ROOST_DTYPE_BF16 ? launch(uint16_t{}, std::integral_constant<int, 8>{})
+                             : launch(float{}, std::integral_constant<int, 4>{});
+      return roost::HipStatus(hipGetLastError(), kOp, "kernel launch");
+    }
     const uint32_t tpb = TokensPerBlock(p.tokens);
     DispatchShape(dt, s, [&](auto t_tag, auto kv, auto kj) {
       using T = decltype(t_tag);
