@@ -142,7 +142,7 @@ struct PlanRecord {
   int32_t window;        // WindowOf(params): the pieces start at the window
   uint32_t merges_two;   // prefill: the leading merge entries of exactly two pieces
   uint32_t overlap;      // prefill with single-token sequences: tile and decode kernels run side by side
-  uint32_t reserved1;
+  uint32_t dec_heads_per_wg;  // (virtual) KV heads per decode workgroup
   uint64_t pages;        // kv_indptr_host[batch]
   uint64_t work_items;   // decode pieces or prefill tiles
   uint64_t ranges;       // decode: workgroup ranges over the pieces
@@ -174,6 +174,7 @@ struct Layout {
   uint64_t float_bytes = 0;
   uint64_t total = 0;
   // Decode region (decode calls: the whole plan; prefill calls: the single-token sequences).
+  uint32_t dec_heads_per_wg = 1;
   uint64_t dec_items = 0, dec_ranges = 0, dec_merges = 0, dec_splits = 0;
   uint64_t dec_item_offset = 0, dec_range_offset = 0, dec_merge_offset = 0, dec_float_offset = 0;
 };
@@ -349,6 +350,7 @@ uint32_t HeadsPerWorkgroup(const RoostPagedAttentionParams& p) {
 }
 
 struct DecodePlan {
+  uint32_t heads_per_wg = 1;       // (virtual) KV heads per workgroup
   std::vector<DecodeWork> items;
   std::vector<int32_t> range_ptr;  // ranges + 1 entries; empty when no sequence is planned
   std::vector<DecodeMerge> merges;
@@ -365,10 +367,77 @@ struct DecodeRow {
   int64_t end;
 };
 
-// Cuts the rows' keys into 16-token groups and the groups into ranges of about equal length, one range per workgroup
-// slot (kDecodeWgsPerCu per CU); a row cut across ranges gets partial slots and a DecodeMerge entry.
-DecodePlan BuildDecodeRows(const RoostPagedAttentionParams& p, uint32_t cus, const std::vector<DecodeRow>& rows) {
+// How a call's rows are dealt to workgroups. Even: ranges of per_range groups, cut wherever a range is full, which fills
+// the chip when there are more groups than slots. Aligned (per_range = the groups of a piece): each row cut by itself into
+// pieces of at most per_range groups, a workgroup each, all of them resident at once.
+struct DecodeDeal {
+  bool aligned = false;
+  uint64_t per_range = 1;
+  uint32_t heads_per_wg = 1;
+};
+
+// Small calls are bound by latency: the steps a wavefront takes one after another (kStepUs each while HBM is not the
+// limit), the merge launch (kMergeUs, none if no row is cut) and its pieces (kMergePieceUs each, read in turn). So few
+// rows are cut into the piece count that balances the two, with fewer KV heads per workgroup where that gives a row more
+// wavefronts; a call that fills the chip keeps the even deal. Fitted on the MI355X (8 heads over 2, head dim 256, cold):
+// one context of 1,500 in pieces of 1 / 2 / 4 / 8 / 16 groups 13.5 / 11.7 / 11.9 / 13.1 / 17.8 us, one of 16,000 41 (2) /
+// 26 / 21 / 23. Against the
+// even deal (with the merge kernel below on both sides): one context of 1,500 13.5 -> 10.7 us, of 16,000 41 -> 18.6; three
+// around 2,500 22.4 -> 12.4; 8 around 2,000 21.6 -> 14.1; 17 of 67 9.2 -> 7.0.
+constexpr double kDecodeBytesPerUs = 5.6e6;  // the decode stream on the whole chip
+constexpr double kStepUs = 1.17;       // a 16-token group of a wavefront
+constexpr double kMergeUs = 4.0;       // the merge launch
+constexpr double kMergePieceUs = 0.05;
+constexpr double kPieceUs = 2.5;       // a further piece of a range: its tables, query and first rows, one after the other
+constexpr uint64_t kAlignMost = 16;    // groups per even range from which the even deal is kept unlooked-at
+
+DecodeDeal ChooseDeal(const RoostPagedAttentionParams& p, uint32_t cus, const std::vector<uint64_t>& groups,
+                      uint64_t total, uint64_t longest, bool may_align) {
+  const uint32_t heads = DecodeHeads(p), most = HeadsPerWorkgroup(p);
+  const uint64_t slots = static_cast<uint64_t>(cus) * kDecodeWgsPerCu;
+  const double group_us = 16.0 * p.head_dim * 2 * (p.q.dtype == ROOST_DTYPE_F32 ? 4 : 2) / kDecodeBytesPerUs;
+  auto cost = [&](uint64_t workgroups, uint32_t hpw, uint64_t piece, uint64_t pieces) {
+    const double steps = static_cast<double>(roost::CeilDiv(piece, 4 / hpw));
+    return steps * std::max(kStepUs, static_cast<double>(workgroups) * 4 * group_us) +
+           (pieces > 1 ? kMergeUs + kMergePieceUs * pieces : 0.0);
+  };
+  DecodeDeal best;
+  best.heads_per_wg = most;
+  const uint64_t wanted = std::max<uint64_t>(1, slots / (heads / most));
+  best.per_range = std::max<uint64_t>(1, roost::CeilDiv(total, std::max<uint64_t>(1, std::min(wanted, total))));
+  // A row spans at most ceil(groups / per_range) + 1 pieces; keep that within what the merge kernel combines.
+  best.per_range = std::max<uint64_t>(best.per_range, roost::CeilDiv(longest, kMaxMergeSplits - 2));
+  if (!may_align || groups.size() > slots || best.per_range > kAlignMost) return best;
+  const uint64_t ranges = roost::CeilDiv(total, best.per_range);
+  double best_us = cost(ranges * (heads / most), most, best.per_range,
+                        groups.size() == 1 && ranges == 1 ? 1 : roost::CeilDiv(longest, best.per_range) + 1);
+  if (groups.size() > 1) best_us += kPieceUs;  // ranges that hold the end of one row and the start of the next
+  for (uint64_t piece = 1; ; piece = std::min(longest, piece < 4 ? piece + 1 : piece + piece / 4)) {
+    uint64_t n = 0;
+    for (const uint64_t g : groups) n += roost::CeilDiv(g, piece);
+    const uint64_t pieces = roost::CeilDiv(longest, piece);
+    if (pieces <= kMaxMergeSplits) {
+      for (uint32_t hpw = most; hpw >= 1; hpw /= 2) {
+        const uint64_t workgroups = n * (heads / hpw);
+        if (workgroups > slots) break;
+        const double us = cost(workgroups, hpw, piece, pieces);
+        if (us < best_us) {
+          best_us = us;
+          best = DecodeDeal{true, piece, hpw};
+        }
+      }
+    }
+    if (piece >= longest) break;
+  }
+  return best;
+}
+
+// Cuts the rows' keys into 16-token groups and deals them out (ChooseDeal); a row cut into pieces gets partial slots and a
+// DecodeMerge entry.
+DecodePlan BuildDecodeRows(const RoostPagedAttentionParams& p, uint32_t cus, const std::vector<DecodeRow>& rows,
+                           bool may_align) {
   DecodePlan d;
+  d.heads_per_wg = HeadsPerWorkgroup(p);
   if (rows.empty()) return d;
   std::vector<uint64_t> groups(rows.size()), first_group(rows.size());
   uint64_t total = 0;
@@ -379,17 +448,16 @@ DecodePlan BuildDecodeRows(const RoostPagedAttentionParams& p, uint32_t cus, con
     groups[r] = rows[r].end > rows[r].first ? roost::CeilDiv(static_cast<uint64_t>(rows[r].end), 16) - first_group[r] : 0;
     total += groups[r];
   }
-  const uint64_t slots_wanted = std::max<uint64_t>(
-      1, static_cast<uint64_t>(cus) * kDecodeWgsPerCu / (DecodeHeads(p) / HeadsPerWorkgroup(p)));
-  const uint64_t ranges = std::max<uint64_t>(1, std::min<uint64_t>(slots_wanted, total));
-  uint64_t per_range = std::max<uint64_t>(1, roost::CeilDiv(total, ranges));
-  // A row spans at most ceil(groups / per_range) + 1 pieces; keep that within what the merge kernel combines.
   const uint64_t longest = *std::max_element(groups.begin(), groups.end());
-  per_range = std::max<uint64_t>(per_range, roost::CeilDiv(longest, kMaxMergeSplits - 2));
-  d.items.reserve(rows.size() + ranges * 2);
-  d.range_ptr.reserve(ranges + 1);
+  const DecodeDeal deal = ChooseDeal(p, cus, groups, total, std::max<uint64_t>(longest, 1), may_align);
+  d.heads_per_wg = deal.heads_per_wg;
+  d.items.reserve(rows.size() + total / deal.per_range + rows.size());
   d.range_ptr.push_back(0);
-  uint64_t room = per_range;  // groups left in the current range
+  uint64_t room = deal.per_range;  // groups left in the current range
+  auto next_range = [&]() {
+    d.range_ptr.push_back(static_cast<int32_t>(d.items.size()));
+    room = deal.per_range;
+  };
   for (size_t r = 0; r < rows.size(); ++r) {
     const auto seq = static_cast<int32_t>(rows[r].seq);
     const int32_t back = rows[r].q_back;
@@ -397,20 +465,20 @@ DecodePlan BuildDecodeRows(const RoostPagedAttentionParams& p, uint32_t cus, con
       d.items.push_back(DecodeWork{seq, 0, 0, -1, back});
       continue;
     }
+    const uint64_t cuts = deal.aligned ? roost::CeilDiv(groups[r], deal.per_range) : 0;  // pieces of an aligned row
+    if (deal.aligned && d.items.size() > static_cast<size_t>(d.range_ptr.back())) next_range();
     const size_t first_item = d.items.size();
     uint64_t g = 0;
     while (g < groups[r]) {
-      if (room == 0) {
-        d.range_ptr.push_back(static_cast<int32_t>(d.items.size()));
-        room = per_range;
-      }
-      const uint64_t n = std::min(room, groups[r] - g);
+      if (room == 0 || (deal.aligned && g > 0)) next_range();
+      const uint64_t done = d.items.size() - first_item;
+      const uint64_t n = deal.aligned ? groups[r] * (done + 1) / cuts - g : std::min(room, groups[r] - g);
       d.items.push_back(DecodeWork{seq, static_cast<int32_t>((first_group[r] + g) * 16),
                                    static_cast<int32_t>(std::min<uint64_t>((first_group[r] + g + n) * 16,
                                                                            static_cast<uint64_t>(rows[r].end))),
                                    -1, back});
       g += n;
-      room -= n;
+      room -= std::min(room, n);
     }
     const size_t pieces = d.items.size() - first_item;
     if (pieces > 1) {
@@ -425,7 +493,7 @@ DecodePlan BuildDecodeRows(const RoostPagedAttentionParams& p, uint32_t cus, con
 // The last-token rows of the sequences b with take(b) (all of them in a decode call, the single-token ones in a
 // prefill call).
 template <typename Take>
-DecodePlan BuildDecode(const RoostPagedAttentionParams& p, uint32_t cus, Take take) {
+DecodePlan BuildDecode(const RoostPagedAttentionParams& p, uint32_t cus, bool may_align, Take take) {
   std::vector<DecodeRow> rows;
   const int32_t window = WindowOf(p);
   for (uint32_t b = 0; b < p.batch; ++b) {
@@ -433,7 +501,7 @@ DecodePlan BuildDecode(const RoostPagedAttentionParams& p, uint32_t cus, Take ta
     const int64_t kv = KvLenHost(p, b);
     rows.push_back(DecodeRow{b, 0, DecodeFirstKey(kv, window), kv});
   }
-  return BuildDecodeRows(p, cus, rows);
+  return BuildDecodeRows(p, cus, rows, may_align);
 }
 
 // Every query token of every sequence as its own row (the f32 prefill, which runs on the VALU decode kernel): token i
@@ -452,12 +520,13 @@ DecodePlan BuildDecodeAllTokens(const RoostPagedAttentionParams& p, uint32_t cus
       rows.push_back(DecodeRow{b, static_cast<int32_t>(n - 1 - i), std::min(first, end), end});
     }
   }
-  return BuildDecodeRows(p, cus, rows);
+  return BuildDecodeRows(p, cus, rows, true);
 }
 
 // Places a decode plan at the end of the int region [0, l.int_bytes) and its partials at the end of the float region
 // (which must not be laid out yet), then writes it to host when given.
 void AppendDecode(const RoostPagedAttentionParams& p, const DecodePlan& d, Layout& l, unsigned char* host) {
+  l.dec_heads_per_wg = d.heads_per_wg;
   l.dec_items = d.items.size();
   l.dec_ranges = d.ranges();
   l.dec_merges = d.merges.size();
@@ -484,7 +553,7 @@ void PlaceFloats(const RoostPagedAttentionParams& p, uint64_t prefill_floats, La
 }
 
 Layout PlanDecode(const RoostPagedAttentionParams& p, uint32_t cus, unsigned char* host) {
-  const DecodePlan d = BuildDecode(p, cus, [](uint32_t) { return true; });
+  const DecodePlan d = BuildDecode(p, cus, true, [](uint32_t) { return true; });
   Layout l;
   AppendDecode(p, d, l, host);
   PlaceFloats(p, 0, l);
@@ -600,7 +669,6 @@ struct OverlapChoice {
 };
 
 constexpr double kTileUsD256 = 3.7;
-constexpr double kDecodeBytesPerUs = 5.6e6;
 constexpr double kMixedLaunchUs = 3.0;
 
 double TileUs(uint32_t head_dim) { return kTileUsD256 * (0.25 + 0.75 * head_dim / 256.0); }
@@ -729,7 +797,8 @@ Layout PlanPrefill(const RoostPagedAttentionParams& p, uint32_t cus, unsigned ch
   l.overlap = overlap.use ? 1u : 0u;
   // Side by side, a decode workgroup has 8 wavefronts and a CU to itself: ranges for dec_cus / 2 CUs at
   // kDecodeWgsPerCu 4-wavefront workgroups each are one range per free CU.
-  AppendDecode(p, BuildDecode(p, overlap.use ? std::max(1u, overlap.dec_cus / kDecodeWgsPerCu) : cus, single), l, host);
+  AppendDecode(p, BuildDecode(p, overlap.use ? std::max(1u, overlap.dec_cus / kDecodeWgsPerCu) : cus, !overlap.use, single),
+               l, host);
   PlaceFloats(p, prefill_floats, l);
   return l;
 }
@@ -1475,9 +1544,11 @@ __global__ void __launch_bounds__(256, kDecodeWgsPerCu)
                            scale_log2, window, causal, cap, blockIdx.x, &m_lds[0][0], &l_lds[0][0], &o_lds[0][0][0]);
 }
 
-// Combines the pieces of each split sequence in key order: one workgroup per (sequence, query head), D threads, one
-// output element each. Wavefront 0 computes the per-piece rescale factors into LDS (lanes over pieces), then every
-// thread sums its element over the pieces with independent loads.
+// Combines the pieces of each split sequence: one workgroup per (sequence, query head) of D threads, four slices of D / 4
+// threads. Slice s sums pieces s, s + 4, ... (four dims per thread, several pieces' loads in flight), wavefront 0 forms the
+// per-piece rescale factors meanwhile, and the slices are added in order through LDS: a fixed order, so deterministic.
+// Latency bound: one element per thread and one dependent load per piece past the 16th took 9.8 us on 94 pieces
+// (the call over one context of 1,500 16.2 -> 13.5 us, three around 2,500 24.2 -> 22.4).
 struct DecodeMergeArgs {
   const DecodeMerge* merges;
   const float* part_o;
@@ -1488,8 +1559,10 @@ struct DecodeMergeArgs {
 template <typename T, int D>
 __device__ __forceinline__ void DecodeMergeBody(T* __restrict__ out, float* __restrict__ lse, const DecodeMergeArgs& m,
                                                 uint32_t q_heads, const void* out_gate, uint32_t bx) {
+  constexpr int kSlices = 4;
   __shared__ float f_lds[kMaxMergeSplits];
   __shared__ float inv_lds;
+  __shared__ __attribute__((aligned(16))) float o_lds[kSlices][D];
   const float* __restrict__ part_o = m.part_o;
   const float* __restrict__ part_ml = m.part_ml;
   const int32_t* __restrict__ q_rows = m.q_rows;
@@ -1500,17 +1573,17 @@ __device__ __forceinline__ void DecodeMergeBody(T* __restrict__ out, float* __re
   const uint32_t qh = bx % q_heads;
   const int n = min(mg.count, static_cast<int32_t>(kMaxMergeSplits));
   const uint64_t base = static_cast<uint64_t>(mg.first) * q_heads + qh;  // partial row of piece c: base + c * q_heads
-  // This thread's partial outputs of the first kPre pieces are requested first, so that they arrive while the pieces'
-  // weights are being computed (a sequence is usually cut into fewer than kPre pieces).
-  constexpr int kPre = 16;
-  const int d = threadIdx.x;
-  const float* po = part_o + base * D + d;
+  // The first kPre pieces of every slice are requested before the weights, which are formed while they arrive.
+  constexpr int kPre = 4;
+  const int slice = threadIdx.x / (D / 4), d4 = 4 * (threadIdx.x % (D / 4));
+  const float* po = part_o + base * D + d4;
   const uint64_t step = static_cast<uint64_t>(q_heads) * D;
-  const uint64_t e = (tok * q_heads + qh) * D + d;
+  auto piece = [&](int c) { return *reinterpret_cast<const f32x4_t*>(po + min(c, n - 1) * step); };
+  const uint64_t e = (tok * q_heads + qh) * D + threadIdx.x;
   const T gv = GateFetch<T>(out_gate, e);  // requested with the partials, applied at the end
-  float pre[kPre];
+  f32x4_t pre[kPre];
 #pragma unroll
-  for (int c = 0; c < kPre; ++c) pre[c] = c < n ? po[c * step] : 0.0f;
+  for (int c = 0; c < kPre; ++c) pre[c] = piece(slice + kSlices * c);
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
     // Piece `lane` (and lane + 64, ... for longer splits): its max and sum, read once.
@@ -1539,15 +1612,26 @@ __device__ __forceinline__ void DecodeMergeBody(T* __restrict__ out, float* __re
     }
   }
   __syncthreads();
-  // Pieces in key order, piece c into accumulator c % 4 (a fixed order: deterministic).
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto add = [&](f32x4_t x, int c) {
+    if (c >= n) return;
+    const float f = f_lds[c];
 #pragma unroll
-  for (int c = 0; c < kPre; ++c) {
-    if (c < n) acc[c & 3] = fmaf(pre[c], f_lds[c], acc[c & 3]);
+    for (int i = 0; i < 4; ++i) acc[i] = fmaf(x[i], f, acc[i]);
+  };
+#pragma unroll
+  for (int c = 0; c < kPre; ++c) add(pre[c], slice + kSlices * c);
+  for (int c0 = slice + kSlices * kPre; c0 < n; c0 += kSlices * kPre) {
+#pragma unroll
+    for (int c = 0; c < kPre; ++c) pre[c] = piece(c0 + kSlices * c);
+#pragma unroll
+    for (int c = 0; c < kPre; ++c) add(pre[c], c0 + kSlices * c);
   }
-  for (int c = kPre; c < n; ++c) acc[c & 3] = fmaf(po[c * step], f_lds[c], acc[c & 3]);
-  const float o0 = acc[0], o1 = acc[1], o2 = acc[2], o3 = acc[3];
-  out[e] = GateApply<T>(out_gate, gv, Narrow<T>(((o0 + o1) + (o2 + o3)) * inv_lds));
+  *reinterpret_cast<f32x4_t*>(&o_lds[slice][d4]) = acc;
+  __syncthreads();
+  const int d = threadIdx.x;
+  const float o = (o_lds[0][d] + o_lds[1][d]) + (o_lds[2][d] + o_lds[3][d]);
+  out[e] = GateApply<T>(out_gate, gv, Narrow<T>(o * inv_lds));
 }
 
 template <typename T, int D>
@@ -2362,6 +2446,13 @@ RoostStatus LaunchDecodeMerge(const RoostPagedAttentionParams& p, const PlanReco
   return roost::HipStatus(hipGetLastError(), "paged_attention", "decode merge launch");
 }
 
+// KV heads per decode workgroup at run time: the plan's, unless the call's heads are not what it was made for (the record
+// does not hold q_heads or the element type); the ranges it dealt serve any number.
+uint32_t RunHeadsPerWorkgroup(const RoostPagedAttentionParams& p, const PlanRecord& rec) {
+  const uint32_t hpw = rec.dec_heads_per_wg;
+  return (hpw == 1 || hpw == 2 || hpw == 4) && DecodeHeads(p) % hpw == 0 ? hpw : HeadsPerWorkgroup(p);
+}
+
 // The view of the decode kernels, whose virtual heads are groups of DecodeGroupOf query heads.
 KvView DecodeView(const RoostPagedAttentionParams& p, KvView kv) {
   kv.vheads = DecodeHeads(p);
@@ -2382,7 +2473,7 @@ RoostStatus LaunchDecode(const RoostPagedAttentionParams& p, const PlanRecord& r
       p.mode == ROOST_ATTENTION_PREFILL ? static_cast<const int32_t*>(p.q_indptr.address) : nullptr;
   auto* out = static_cast<T*>(p.output.address);
   auto* lse = static_cast<float*>(p.lse.address);
-  const uint32_t heads = DecodeHeads(p), hpw = HeadsPerWorkgroup(p);
+  const uint32_t heads = DecodeHeads(p), hpw = RunHeadsPerWorkgroup(p, rec);
   const KvView dkv = DecodeView(p, kv);
   const dim3 grid(static_cast<uint32_t>(rec.dec_ranges * (heads / hpw)));
   auto launch = [&](auto kernel) {
@@ -2457,7 +2548,7 @@ RoostStatus LaunchMixed(const RoostPagedAttentionParams& p, const PlanRecord& re
   const SoftCap raw{cap.capl / scale_log2, cap.k * scale_log2};
   const bool capped = cap.capl != 0.0f;
   const KvView dkv = DecodeView(p, kv);
-  const uint32_t hpw = HeadsPerWorkgroup(p);
+  const uint32_t hpw = RunHeadsPerWorkgroup(p, rec);
   const uint32_t n_items = static_cast<uint32_t>(rec.work_items);
   const dim3 grid(n_items + static_cast<uint32_t>(rec.dec_ranges * (dkv.vheads / hpw)));
   const auto* dec_items = reinterpret_cast<const DecodeWork*>(dev + rec.dec_item_offset);
@@ -2551,6 +2642,7 @@ PlanRecord MakeRecord(const RoostPagedAttentionParams& p, const Layout& l) {
   r.window = WindowOf(p);
   r.merges_two = static_cast<uint32_t>(l.merges_two);
   r.overlap = l.overlap;
+  r.dec_heads_per_wg = l.dec_heads_per_wg;
   r.pages = static_cast<uint64_t>(p.kv_indptr_host[p.batch]);
   r.work_items = l.work_items;
   r.ranges = l.ranges;

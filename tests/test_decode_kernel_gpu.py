@@ -28,6 +28,20 @@ def test_decode_group_and_page_edges(session, hq, hkv, d, ps, hnd, window):
     cases.assert_attention_class(got, ref, float(np.abs(cases.values(b.v_cache, True)).max()), what="decode")
 
 
+# Few rows, cut by themselves into pieces that are resident at once (or not cut at all), with fewer KV heads per workgroup
+# than the full batch takes, empty rows among them; 64 rows around the line to the even deal.
+@pytest.mark.parametrize("kv_lens", [[1], [16], [300], [1500], [9000], [0, 40, 0, 3000, 0], [17] * 9, [700, 1, 0, 5000, 33],
+                                     [450 + 7 * i for i in range(64)]], ids=lambda k: f"{len(k)}x{max(k)}")
+@pytest.mark.parametrize("hq,hkv,d,hnd", [(8, 2, 256, False), (32, 8, 128, True), (64, 4, 64, False)])
+def test_decode_few_rows(session, kv_lens, hq, hkv, d, hnd):
+    rng = np.random.default_rng(sum(kv_lens) + d)
+    b = cases.make_paged_batch(rng, kv_lens, [1] * len(kv_lens), hq=hq, hkv=hkv, d=d, hnd=hnd, std=1.0)
+    causal = 0 not in kv_lens  # the oracle refuses a causal row without keys; a decode row sees every key either way
+    got = run_case(session, b, causal=causal)
+    ref = cases.values(cases.oracle_attention(b, causal), True)
+    cases.assert_attention_class(got, ref, float(np.abs(cases.values(b.v_cache, True)).max()), what="decode")
+
+
 @pytest.mark.parametrize("hq,hkv,d", [(32, 4, 128), (32, 2, 128), (16, 2, 256), (16, 4, 64)])
 def test_mixed_launch_query_head_groups(session, hq, hkv, d):
     rng = np.random.default_rng(hq + d)
