@@ -59,6 +59,17 @@ constexpr uint32_t kPrefillTileQ = 32;          // query tokens per workgroup of
 constexpr uint32_t kPrefillTileK = 64;          // keys per LDS tile
 constexpr uint32_t kPfTokens = 64;              // query tokens per workgroup of the prefill for page sizes % 16 == 0
 constexpr uint32_t kPfRows = kPfTokens * kGroup;  // query rows (token, head) of one such workgroup
+// The 12-wavefront form of the tile kernel: 96 query tokens, so that each SIMD holds three wavefronts (153 of 168
+// registers, no spills) and one's softmax has two others' multiplies to run beside, and each K/V tile is copied for
+// half as many more queries. Four prompts around 3,800 tokens x 32 heads over 8, head dim 128: 524 -> 485 us (1,013
+// against 872 TFLOP/s). Head dim 64 is slower with it (83 -> 90 us); head dim 256 does not fit three wavefronts.
+constexpr uint32_t kPfWideTokens = 96;
+constexpr uint32_t kPfWideDim = 128;            // the head dim it is built for
+// A 96-token tile's time over a 64-token one's: plan() takes the 12-wavefront form when its dispatch ends that much
+// earlier in tiles. Ratios of the two dispatches and times (8 wavefronts, 12; us; head dim 128): 4 prompts around 3,800 x
+// 32 heads 1.45, 524 / 485; 8 ragged prompts to 4,000 1.45, 393 / 363; 6 chunks on prefixes 1.40, 408 / 384; 2 prompts
+// 1.40, 248 / 243; one prompt of 4,096 1.35, 154 / 162; one of 3,000 1.32, 103 / 108.
+constexpr double kPfWideTileCost = 1.39;
 constexpr uint32_t kPfMinSplitTiles = 8;        // a split piece covers at least this many 64-key tiles
 constexpr uint32_t kAlign = 256;
 constexpr uint32_t kPlanMagic = 0x41504752;     // "RGPA"
@@ -157,6 +168,7 @@ struct PlanRecord {
   // Single-token sequences of a prefill call run as decode: their pieces, ranges, merges and partials.
   uint64_t dec_items, dec_ranges, dec_merges, dec_splits;
   uint64_t dec_item_offset, dec_range_offset, dec_merge_offset, dec_float_offset;
+  uint64_t item_tokens;  // prefill: query tokens per work item (kPfTokens or kPfWideTokens)
 };
 
 struct Layout {
@@ -164,6 +176,7 @@ struct Layout {
   uint64_t ranges = 0;
   uint64_t merges = 0;
   uint64_t merges_two = 0;  // prefill: leading merge entries of two pieces
+  uint32_t item_tokens = kPfTokens;  // prefill: query tokens per work item
   uint32_t overlap = 0;     // prefill: tile and decode kernels on two streams (ChooseOverlap)
   uint64_t range_offset = 0;
   uint64_t merge_offset = 0;
@@ -568,7 +581,7 @@ Layout PlanDecode(const RoostPagedAttentionParams& p, uint32_t cus, unsigned cha
 }
 
 // Prefill work items: one per (query tile, KV head) -- 64-token tiles when the page size is a multiple of 16 (the
-// DMA-fed kernel), 32-token tiles otherwise. For the 64-token kernel the key range of an item longer than 3/4 of the
+// DMA-fed kernel; 96-token ones at head dim 128 where that ends earlier), 32-token tiles otherwise. For the 64-token kernel the key range of an item longer than 3/4 of the
 // average load of a CU is cut into pieces of whole 64-key tiles (at least kPfMinSplitTiles each), so that the longest causal
 // tile does not set the makespan; the pieces write partials merged by PrefillMergeKernel. Items are ordered longest
 // first. The cuts depend on the whole batch, so the variant is deterministic but not batch invariant.
@@ -576,35 +589,50 @@ bool PrefillFastPath(const RoostPagedAttentionParams& p) {
   return p.page_size % 16 == 0 && (p.page_size & (p.page_size - 1)) == 0;
 }
 
-// Tiles of a work item (its key range in 64-key tiles), and of the pieces it is cut into with at most `target` each.
-int64_t ItemTiles(const PrefillWork& w) { return roost::CeilDiv(static_cast<int64_t>(w.kend - w.kbeg), 64); }
+// The work items of a call by their key ranges in 64-key tiles: `tiles` holds one entry per query tile, of which `heads`
+// items (one per group of kGroup query heads) are cut alike.
+struct ItemList {
+  std::vector<int64_t> tiles;
+  int64_t heads = 1;
+  int64_t count() const { return static_cast<int64_t>(tiles.size()) * heads; }
+  int64_t longest() const { return tiles.empty() ? 0 : *std::max_element(tiles.begin(), tiles.end()); }
+  int64_t total() const {
+    int64_t sum = 0;
+    for (int64_t t : tiles) sum += t;
+    return sum * heads;
+  }
+};
+
+// The pieces an item of `tiles` tiles is cut into with at most `target` each.
 int64_t Pieces(int64_t tiles, int64_t target) { return std::min<int64_t>(roost::CeilDiv(tiles, target), kMaxMergeSplits); }
 
 // The longest-first dispatch of the items cut at `target` onto `cus` workgroup slots, each piece costing its tiles
 // plus kPfPieceCost (its set-up and epilogue): the finishing time of the last slot, in tiles.
 constexpr int64_t kPfPieceCost = 2;
-template <typename Items>
-int64_t PrefillMakespan(const Items& items, int64_t target, uint32_t cus) {
+int64_t PrefillMakespan(const ItemList& items, int64_t target, uint32_t cus) {
   // Piece costs by counting (they are small integers), then longest first onto the least loaded slot.
-  std::vector<uint32_t> count;
-  for (const auto& it : items) {
-    const int64_t tiles = ItemTiles(it.w), n = Pieces(tiles, target);
+  std::vector<int64_t> count;
+  for (const int64_t tiles : items.tiles) {
+    const int64_t n = Pieces(tiles, target);
     for (int64_t i = 0; i < n; ++i) {
       const auto c = static_cast<size_t>(tiles * (i + 1) / n - tiles * i / n + kPfPieceCost);
       if (c >= count.size()) count.resize(c + 1, 0);
-      ++count[c];
+      count[c] += items.heads;
     }
   }
-  // Slots by load (at[L]: how many slots carry L tiles); loads only grow, so the least loaded level only moves up.
-  std::vector<uint32_t> at(1, std::max<uint32_t>(cus, 1));
+  // Slots by load (at[L]: how many slots carry L tiles); loads only grow, so the least loaded level only moves up, and
+  // pieces of one cost fill a level's slots together.
+  std::vector<int64_t> at(1, std::max<uint32_t>(cus, 1));
   size_t lo = 0, end = 0;
   for (size_t c = count.size(); c-- > 0;) {
-    for (uint32_t k = 0; k < count[c]; ++k) {
+    for (int64_t left = count[c]; left > 0;) {
       while (at[lo] == 0) ++lo;
-      --at[lo];
+      const int64_t n = std::min(at[lo], left);
+      left -= n;
+      at[lo] -= n;
       const size_t load = lo + c;
       if (load >= at.size()) at.resize(load + 1, 0);
-      ++at[load];
+      at[load] += n;
       end = std::max(end, load);
     }
   }
@@ -616,23 +644,27 @@ int64_t PrefillMakespan(const Items& items, int64_t target, uint32_t cus) {
 // (config 5's two 512-token chunks: 256 pieces of 9 tiles instead of 288 of 8, whose last 32 ran in a second round);
 // the one whose longest-first dispatch ends first wins. Config 3 keeps 3/4 (0.197 ms, against 0.203 at 17/20 and
 // 0.234 at 13/20); a dense 4 x 4096 batch takes the whole average (1,095 against 950 TFLOP/s at 3/4).
-template <typename Items>
-int64_t PrefillPieceTiles(const Items& items, int64_t total_tiles, uint32_t cus) {
+struct PieceChoice {
+  int64_t target;  // piece size in tiles
+  int64_t end;     // the dispatch's finishing time in tiles
+};
+
+PieceChoice PrefillPieceTiles(const ItemList& items, uint32_t cus) {
   const uint32_t slots = std::max<uint32_t>(cus, 1);
+  const int64_t total_tiles = items.total();
   auto of_avg = [&](int64_t num, int64_t den) {
     return std::max<int64_t>(kPfMinSplitTiles, roost::CeilDiv(total_tiles * num, den * int64_t{slots}));
   };
   std::vector<int64_t> cand{of_avg(3, 4), of_avg(17, 20), of_avg(1, 1)};
-  int64_t longest = 0;
-  for (const auto& it : items) longest = std::max(longest, ItemTiles(it.w));
+  const int64_t longest = items.longest();
   for (int64_t rounds = 1; rounds <= 2; ++rounds) {
-    if (static_cast<int64_t>(items.size()) > rounds * slots) break;
+    if (items.count() > rounds * slots) break;
     // Smallest target whose pieces number at most rounds x slots (the count only falls as the target grows).
     int64_t lo = kPfMinSplitTiles, hi = std::max<int64_t>(longest, kPfMinSplitTiles);
     auto count = [&](int64_t t) {
       int64_t n = 0;
-      for (const auto& it : items) n += Pieces(ItemTiles(it.w), t);
-      return n;
+      for (const int64_t tiles : items.tiles) n += Pieces(tiles, t);
+      return n * items.heads;
     };
     if (count(hi) > rounds * slots) continue;
     while (lo < hi) {
@@ -647,6 +679,41 @@ int64_t PrefillPieceTiles(const Items& items, int64_t total_tiles, uint32_t cus)
     if (end < best_end || (end == best_end && cand[i] > best)) {
       best = cand[i];
       best_end = end;
+    }
+  }
+  return {best, best_end};
+}
+
+// Calls whose pieces do not fill the CUs once (a short prompt: 1,777 tokens x 2 KV heads made 128 pieces of up to 8
+// tiles for 256 CUs): pieces below kPfMinSplitTiles, down to 2 tiles, while they still run in one round. Each is priced by
+// what such calls measured: a tile on a chip with idle CUs 2.3 us at head dim 256, the merge launch 4.5 us, and 0.08 us
+// per piece for its partial rows written and merged (both sides less at smaller head dims). Fresh prompts at head dim
+// 256, 8 heads, pieces of at most 8 tiles against this choice: 500 tokens 34.6 -> 25.3 us (2 tiles), 1,000 41.7 -> 32.2
+// (2), 1,777 49.9 -> 42.6 (4); 256 tokens on 4,000 cached ones 44.6 -> 35.6 (4). 200 tokens stay whole: 21.1 against
+// 23.0 us in pieces of 2.
+constexpr double kSparseTileUs = 2.3;
+constexpr double kPieceMergeUs = 0.08;
+constexpr double kMergeLaunchUs = 4.5;
+
+int64_t SparsePieceTiles(const ItemList& items, int64_t target, uint32_t head_dim, uint32_t cus) {
+  if (items.count() >= static_cast<int64_t>(cus)) return target;
+  const double rel = head_dim / 256.0;
+  const double tile_us = kSparseTileUs * (0.25 + 0.75 * rel);
+  int64_t best = target;
+  double best_us = 0.0;
+  for (int64_t t = target; t >= 2; t = std::min(t, static_cast<int64_t>(kPfMinSplitTiles)) - 1) {
+    int64_t n = 0, longest = 0;
+    for (const int64_t tiles : items.tiles) {
+      const int64_t pieces = Pieces(tiles, t);
+      n += pieces * items.heads;
+      longest = std::max<int64_t>(longest, pieces > 0 ? (tiles + pieces - 1) / pieces : 0);
+    }
+    if (n > static_cast<int64_t>(cus)) break;  // one round: the longest piece ends last
+    const double us = (longest + kPfPieceCost) * tile_us + n * kPieceMergeUs * rel +
+                      (n > items.count() ? kMergeLaunchUs : 0.0);
+    if (t == target || us < best_us) {
+      best_us = us;
+      best = t;
     }
   }
   return best;
@@ -676,25 +743,24 @@ double DecodeUs(double bytes, uint32_t cus_used, uint32_t cus) {
   return bytes / (kDecodeBytesPerUs * std::pow(static_cast<double>(cus_used) / cus, 0.26));
 }
 
-template <typename Items, typename Single>
-OverlapChoice ChooseOverlap(const RoostPagedAttentionParams& p, const Items& items, int64_t serial_target, uint32_t cus,
+template <typename Single>
+OverlapChoice ChooseOverlap(const RoostPagedAttentionParams& p, const ItemList& items, int64_t serial_target, uint32_t cus,
                             Single single) {
   OverlapChoice best;
   double dec_bytes = 0.0;
   for (uint32_t b = 0; b < p.batch; ++b) {
     if (single(b)) dec_bytes += static_cast<double>(KvLenHost(p, b)) * DecodeHeads(p) * p.head_dim * 2.0 * 2.0;
   }
-  if (dec_bytes == 0.0 || items.empty() || cus < 2 || p.page_size % 16 != 0) return best;
-  int64_t longest = 0;
-  for (const auto& it : items) longest = std::max(longest, ItemTiles(it.w));
+  if (dec_bytes == 0.0 || items.tiles.empty() || cus < 2 || p.page_size % 16 != 0) return best;
+  const int64_t longest = items.longest();
   const double tile_us = TileUs(p.head_dim);
   double best_us = PrefillMakespan(items, serial_target, cus) * tile_us + DecodeUs(dec_bytes, cus, cus);
   for (int64_t k = 1; k <= 16; ++k) {
     const int64_t target = std::max<int64_t>(1, roost::CeilDiv(longest, k));
     int64_t pieces = 0, piece_max = 0;
-    for (const auto& it : items) {
-      const int64_t tiles = ItemTiles(it.w), n = Pieces(tiles, target);
-      pieces += n;
+    for (const int64_t tiles : items.tiles) {
+      const int64_t n = Pieces(tiles, target);
+      pieces += n * items.heads;
       piece_max = std::max<int64_t>(piece_max, roost::CeilDiv(tiles, n));
     }
     if (pieces >= static_cast<int64_t>(cus)) break;
@@ -719,46 +785,76 @@ Layout PlanPrefill(const RoostPagedAttentionParams& p, uint32_t cus, unsigned ch
     return l;
   }
   const bool fast = PrefillFastPath(p);
-  const int64_t tile_q = fast ? kPfTokens : kPrefillTileQ;
   struct Item {
     PrefillWork w;
     int64_t cost;
   };
-  std::vector<Item> items;
-  int64_t total_tiles = 0;
   const int32_t window = WindowOf(p);
   // A sequence with one query token (a decode row of a mixed step) sees every key whether causal or not: the decode
   // kernel streams it at HBM speed instead of a 64-row MFMA tile holding one row.
   auto single = [&](uint32_t b) { return p.q_indptr_host[b + 1] - p.q_indptr_host[b] == 1; };
-  for (uint32_t b = 0; b < p.batch; ++b) {
-    if (single(b)) continue;
-    const int64_t n = p.q_indptr_host[b + 1] - p.q_indptr_host[b];
-    const int64_t kv = KvLenHost(p, b);
-    for (int64_t q0 = 0; q0 < n; q0 += tile_q) {
-      const int64_t rows = std::min<int64_t>(tile_q, n - q0);
-      int64_t kend = p.causal ? std::min<int64_t>(kv, kv - n + q0 + rows) : kv;
-      if (kend < 0) kend = 0;
-      // With a window the item's first query (position kv - n + q0) sees keys from kv - n + q0 - window on; the
-      // range starts at that key rounded down to 16 (a 16-row group never straddles a page), and keys before it are
-      // never read.
-      int64_t kbeg = window < 0 ? 0 : std::max<int64_t>(0, kv - n + q0 - window) / 16 * 16;
-      if (kbeg > kend) kbeg = kend;
-      total_tiles += roost::CeilDiv(kend - kbeg, 64) * VirtualHeads(p);
-      for (uint32_t h = 0; h < VirtualHeads(p); ++h) {  // item per group of kGroup query heads
-        items.push_back(Item{PrefillWork{static_cast<int32_t>(b), static_cast<int32_t>(q0), static_cast<int32_t>(h),
-                                         static_cast<int32_t>(rows), static_cast<int32_t>(kbeg),
-                                         static_cast<int32_t>(kend), -1, kPieceFirst | kPieceLast},
-                             kend - kbeg + 64});
+  // Visits every query tile of tile_q tokens: (sequence, first token, tokens, key range).
+  auto query_tiles = [&](int64_t tile_q, auto&& visit) {
+    for (uint32_t b = 0; b < p.batch; ++b) {
+      if (single(b)) continue;
+      const int64_t n = p.q_indptr_host[b + 1] - p.q_indptr_host[b];
+      const int64_t kv = KvLenHost(p, b);
+      for (int64_t q0 = 0; q0 < n; q0 += tile_q) {
+        const int64_t rows = std::min<int64_t>(tile_q, n - q0);
+        int64_t kend = p.causal ? std::min<int64_t>(kv, kv - n + q0 + rows) : kv;
+        if (kend < 0) kend = 0;
+        // With a window the item's first query (position kv - n + q0) sees keys from kv - n + q0 - window on; the
+        // range starts at that key rounded down to 16 (a 16-row group never straddles a page), and keys before it are
+        // never read.
+        int64_t kbeg = window < 0 ? 0 : std::max<int64_t>(0, kv - n + q0 - window) / 16 * 16;
+        if (kbeg > kend) kbeg = kend;
+        visit(b, q0, rows, kbeg, kend);
       }
     }
-  }
-  std::vector<PrefillMerge> merges;
-  int32_t slot = 0;
+  };
+  auto item_list = [&](int64_t tile_q) {
+    ItemList l;
+    l.heads = VirtualHeads(p);
+    query_tiles(tile_q, [&](uint32_t, int64_t, int64_t, int64_t kbeg, int64_t kend) {
+      l.tiles.push_back(roost::CeilDiv(kend - kbeg, 64));
+    });
+    return l;
+  };
+  int64_t tile_q = fast ? kPfTokens : kPrefillTileQ;
+  int64_t target = 0;
   OverlapChoice overlap;
   if (fast) {
-    int64_t target = PrefillPieceTiles(items, total_tiles, cus);
-    overlap = ChooseOverlap(p, items, target, cus, single);
-    if (overlap.use) target = overlap.target;
+    ItemList list = item_list(tile_q);
+    const PieceChoice narrow = PrefillPieceTiles(list, cus);
+    target = narrow.target;
+    overlap = ChooseOverlap(p, list, target, cus, single);
+    if (overlap.use) {
+      target = overlap.target;
+    } else {
+      if (p.head_dim == kPfWideDim) {
+        ItemList wide_list = item_list(kPfWideTokens);
+        const PieceChoice wide = PrefillPieceTiles(wide_list, cus);
+        if (wide.end * kPfWideTileCost < narrow.end) {
+          tile_q = kPfWideTokens;
+          target = wide.target;
+          list = std::move(wide_list);
+        }
+      }
+      target = SparsePieceTiles(list, target, p.head_dim, cus);
+    }
+  }
+  std::vector<Item> items;
+  query_tiles(tile_q, [&](uint32_t b, int64_t q0, int64_t rows, int64_t kbeg, int64_t kend) {
+    for (uint32_t h = 0; h < VirtualHeads(p); ++h) {  // item per group of kGroup query heads
+      items.push_back(Item{PrefillWork{static_cast<int32_t>(b), static_cast<int32_t>(q0), static_cast<int32_t>(h),
+                                       static_cast<int32_t>(rows), static_cast<int32_t>(kbeg),
+                                       static_cast<int32_t>(kend), -1, kPieceFirst | kPieceLast},
+                           kend - kbeg + 64});
+    }
+  });
+  std::vector<PrefillMerge> merges;
+  int32_t slot = 0;
+  if (fast) {
     std::vector<Item> cut;
     cut.reserve(items.size());
     for (const Item& it : items) {
@@ -784,8 +880,9 @@ Layout PlanPrefill(const RoostPagedAttentionParams& p, uint32_t cus, unsigned ch
   std::stable_sort(items.begin(), items.end(), [](const Item& a, const Item& b) { return a.cost > b.cost; });
   // Merges of exactly two pieces first: they run on the 8-rows-per-block form of the merge kernel.
   std::stable_partition(merges.begin(), merges.end(), [](const PrefillMerge& m) { return m.count == 2; });
-  Layout l = MakeLayout(items.size(), 0, merges.size(), static_cast<uint64_t>(slot), kPfRows, p.head_dim,
-                        ROOST_ATTENTION_PREFILL);
+  Layout l = MakeLayout(items.size(), 0, merges.size(), static_cast<uint64_t>(slot),
+                        static_cast<uint32_t>(tile_q) * kGroup, p.head_dim, ROOST_ATTENTION_PREFILL);
+  l.item_tokens = fast ? static_cast<uint32_t>(tile_q) : kPfTokens;
   l.merges_two = static_cast<uint64_t>(
       std::count_if(merges.begin(), merges.end(), [](const PrefillMerge& m) { return m.count == 2; }));
   if (host != nullptr) {
@@ -1936,7 +2033,7 @@ template <int D>
 constexpr int kPfTileBytes = kPrefillTileK * 2 * D;  // one 64-key K or V tile in LDS
 
 // The tile kernel's work for item `item`; `tiles` is the caller's LDS, [2 buffers][K, V][kPfTileBytes<D>].
-template <int D, bool kCap>
+template <int D, bool kCap, int kWaves>
 __device__ __forceinline__ void PrefillTileBody(const uint16_t* __restrict__ q, uint16_t* __restrict__ out,
                                                 float* __restrict__ lse, KvView kv,
                                                 const int32_t* __restrict__ kv_indices,
@@ -1953,6 +2050,7 @@ __device__ __forceinline__ void PrefillTileBody(const uint16_t* __restrict__ q, 
   constexpr int kDt = D / 32;                   // 32-dim blocks of O^T
   constexpr int kNv = kDt / 2;                  // V blocks each wavefront copies per tile (4 kDt blocks / 8)
   constexpr int kSw = (kPieces < 16 ? kPieces : 16) - 1;  // K swizzle mask
+  constexpr uint32_t kRows = 32 * kWaves;       // query rows of an item (8 kWaves tokens x kGroup heads)
 
   const PrefillWork wk = work[item];
   const int tid = threadIdx.x;
@@ -2025,6 +2123,7 @@ __device__ __forceinline__ void PrefillTileBody(const uint16_t* __restrict__ q, 
   // This wavefront's share of the copy of tile t: K rows 8w .. 8w + 7 (kRowsPerDma rows per instruction) and kNv
   // blocks of V.
   auto issue = [&](int t, int buf, const int32_t (&ids)[4], int ln) {
+    if (kWaves > 8 && w >= 8) return;  // the first 8 wavefronts copy
     const int32_t kb = kbeg + 64 * t;
     const int32_t pos0 = kb + 8 * w;  // this wavefront's first row; all 8 lie in one page
     const int32_t id = ids[w >> 1];
@@ -2103,6 +2202,10 @@ __device__ __forceinline__ void PrefillTileBody(const uint16_t* __restrict__ q, 
     const unsigned char* vl = vtile + 8 * ln;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
+      // Keys after every query of the wavefront (uniform): nothing to add. Four prompts around 3,800 tokens at head dim
+      // 128: 546 -> 534 us. At head dim 256 the branch costs more registers than it saves work (8 ragged chunks on
+      // prefixes: 357 -> 365 us).
+      if (D <= 128 && causal && kb + 32 * half > last_pos) break;
       f32x16_t sc;
 #pragma unroll
       for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
@@ -2200,7 +2303,7 @@ __device__ __forceinline__ void PrefillTileBody(const uint16_t* __restrict__ q, 
   if (!row_ok) return;
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
   if (wk.slot >= 0) {  // a piece of a split item: its normalised output in bf16 and its (max, sum)
-    const uint64_t prow = static_cast<uint64_t>(wk.slot) * kPfRows + static_cast<uint64_t>(r) * kGroup + hq;
+    const uint64_t prow = static_cast<uint64_t>(wk.slot) * kRows + static_cast<uint64_t>(r) * kGroup + hq;
     uint16_t* po = part_o + prow * D;
 #pragma unroll
     for (int dt = 0; dt < kDt; ++dt)
@@ -2233,16 +2336,16 @@ __device__ __forceinline__ void PrefillTileBody(const uint16_t* __restrict__ q, 
 }
 
 
-template <int D, bool kCap>
-__global__ void __launch_bounds__(512, 1)
+template <int D, bool kCap, int kWaves>
+__global__ void __launch_bounds__(64 * kWaves, 1)
     PrefillTileKernel(const uint16_t* __restrict__ q, uint16_t* __restrict__ out, float* __restrict__ lse, KvView kv,
                       const int32_t* __restrict__ kv_indices, const int32_t* __restrict__ q_indptr,
                       const PrefillWork* __restrict__ work, uint16_t* __restrict__ part_o, float* __restrict__ part_ml,
                       uint32_t q_heads, uint32_t causal, uint32_t ps_shift, float scale_log2, int32_t window,
                       SoftCap cap) {
   __shared__ __attribute__((aligned(16))) unsigned char tiles[2][2][kPfTileBytes<D>];  // [buffer][K, V]
-  PrefillTileBody<D, kCap>(q, out, lse, kv, kv_indices, q_indptr, work, part_o, part_ml, q_heads, causal, ps_shift,
-                           scale_log2, window, cap, blockIdx.x, tiles);
+  PrefillTileBody<D, kCap, kWaves>(q, out, lse, kv, kv_indices, q_indptr, work, part_o, part_ml, q_heads, causal,
+                                   ps_shift, scale_log2, window, cap, blockIdx.x, tiles);
 }
 
 // A mixed step's attention in one launch: workgroups [0, items) run the tile pieces, the rest the decode ranges with 8
@@ -2267,9 +2370,9 @@ __global__ void __launch_bounds__(512, 1)
   constexpr int kLds = kTileLds > kMixedDecodeLds<D, NH> ? kTileLds : kMixedDecodeLds<D, NH>;
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
   if (blockIdx.x < items) {
-    PrefillTileBody<D, kCap>(q, out, lse, kv, kv_indices, q_indptr, work, part_o, part_ml, q_heads, causal, ps_shift,
-                             scale_log2, window, raw_cap, blockIdx.x,
-                             reinterpret_cast<unsigned char (*)[2][kPfTileBytes<D>]>(lds));
+    PrefillTileBody<D, kCap, 8>(q, out, lse, kv, kv_indices, q_indptr, work, part_o, part_ml, q_heads, causal, ps_shift,
+                                scale_log2, window, raw_cap, blockIdx.x,
+                                reinterpret_cast<unsigned char (*)[2][kPfTileBytes<D>]>(lds));
     return;
   }
   constexpr int W = kMixedDecodeWaves;
@@ -2308,7 +2411,7 @@ __device__ __forceinline__ void MergeAdd(float4& acc, u32x2_t raw, float f) {
   acc.w = fmaf(__uint_as_float(raw[1] & 0xFFFF0000u), f, acc.w);
 }
 
-template <int D, int kRows>
+template <int D, int kTokens, int kRows>
 __device__ __forceinline__ void PrefillMergeRows(uint16_t* __restrict__ out, float* __restrict__ lse,
                                                  const PrefillMerge& mg, int r0, const uint16_t* __restrict__ part_o,
                                                  const float* __restrict__ part_ml,
@@ -2319,9 +2422,9 @@ __device__ __forceinline__ void PrefillMergeRows(uint16_t* __restrict__ out, flo
   const int d = 4 * (threadIdx.x % (D / 4));
   const uint32_t head = mg.kv_head * kGroup + hq;
   const uint64_t tok0 = static_cast<uint64_t>(q_indptr[mg.seq] + mg.q0);
-  // Partial row of piece i for token row r: (first + i) * kPfRows + r * kGroup + hq.
+  // Partial row of piece i for token row r: ((first + i) * kTokens + r) * kGroup + hq.
   auto prow = [&](int i, int r) {
-    return (static_cast<uint64_t>(mg.first) + i) * kPfRows + static_cast<uint64_t>(r) * kGroup + hq;
+    return ((static_cast<uint64_t>(mg.first) + i) * kTokens + r) * kGroup + hq;
   };
   if constexpr (kRows > 1) {  // merges of exactly two pieces
     float2 ml[kRows][2];
@@ -2385,30 +2488,31 @@ struct PrefillMergeArgs {
   uint32_t blocks;  // blocks of the launch's prefill share
 };
 
-template <int D>
+template <int D, int kTokens>
 __device__ __forceinline__ void PrefillMergeBody(uint16_t* __restrict__ out, float* __restrict__ lse,
                                                  const PrefillMergeArgs& m, uint32_t q_heads, const void* gate,
                                                  uint32_t b) {
-  constexpr uint32_t kTwoBlocks = kPfTokens / kPfMergeRows;  // blocks per two-piece merge
+  constexpr uint32_t kTwoBlocks = kTokens / kPfMergeRows;  // blocks per two-piece merge
   const PrefillMerge* __restrict__ merges = m.merges;
   const uint16_t* __restrict__ part_o = m.part_o;
   const float* __restrict__ part_ml = m.part_ml;
   const int32_t* __restrict__ q_indptr = m.q_indptr;
   const uint32_t two = m.two;
   if (b < two * kTwoBlocks) {
-    PrefillMergeRows<D, kPfMergeRows>(out, lse, merges[b / kTwoBlocks], static_cast<int>(b % kTwoBlocks) * kPfMergeRows,
-                                      part_o, part_ml, q_indptr, q_heads, gate);
+    PrefillMergeRows<D, kTokens, kPfMergeRows>(out, lse, merges[b / kTwoBlocks],
+                                               static_cast<int>(b % kTwoBlocks) * kPfMergeRows, part_o, part_ml,
+                                               q_indptr, q_heads, gate);
   } else {
     const uint32_t k = b - two * kTwoBlocks;
-    PrefillMergeRows<D, 1>(out, lse, merges[two + k / kPfTokens], static_cast<int>(k % kPfTokens), part_o, part_ml,
-                           q_indptr, q_heads, gate);
+    PrefillMergeRows<D, kTokens, 1>(out, lse, merges[two + k / kTokens], static_cast<int>(k % kTokens), part_o, part_ml,
+                                    q_indptr, q_heads, gate);
   }
 }
 
-template <int D>
+template <int D, int kTokens>
 __global__ void __launch_bounds__(256) PrefillMergeKernel(uint16_t* __restrict__ out, float* __restrict__ lse,
                                                           PrefillMergeArgs m, uint32_t q_heads, const void* gate) {
-  PrefillMergeBody<D>(out, lse, m, q_heads, gate, blockIdx.x);
+  PrefillMergeBody<D, kTokens>(out, lse, m, q_heads, gate, blockIdx.x);
 }
 
 // A mixed step's two merges in one launch (both take D threads per block): the tile pieces' merge blocks first, then
@@ -2419,7 +2523,7 @@ __global__ void __launch_bounds__(D) MixedMergeKernel(uint16_t* __restrict__ out
                                                       const void* gate) {
   static_assert(kGroup * D / 4 == D, "a prefill merge block has D threads");
   if (blockIdx.x < pm.blocks) {
-    PrefillMergeBody<D>(out, lse, pm, q_heads, gate, blockIdx.x);
+    PrefillMergeBody<D, kPfTokens>(out, lse, pm, q_heads, gate, blockIdx.x);
   } else {
     DecodeMergeBody<uint16_t, D>(out, lse, dm, q_heads, gate, blockIdx.x - pm.blocks);
   }
@@ -2503,7 +2607,7 @@ uint16_t* PrefillPartO(const RoostPagedAttentionParams& p, const PlanRecord& rec
   return reinterpret_cast<uint16_t*>(dev + rec.float_offset);
 }
 float* PrefillPartMl(const RoostPagedAttentionParams& p, const PlanRecord& rec, unsigned char* dev) {
-  return reinterpret_cast<float*>(PrefillPartO(p, rec, dev) + rec.splits * kPfRows * p.head_dim);
+  return reinterpret_cast<float*>(PrefillPartO(p, rec, dev) + rec.splits * rec.item_tokens * kGroup * p.head_dim);
 }
 
 PrefillMergeArgs PrefillMergeArgsOf(const RoostPagedAttentionParams& p, const PlanRecord& rec, unsigned char* dev) {
@@ -2513,7 +2617,8 @@ PrefillMergeArgs PrefillMergeArgsOf(const RoostPagedAttentionParams& p, const Pl
   m.part_ml = PrefillPartMl(p, rec, dev);
   m.q_indptr = static_cast<const int32_t*>(p.q_indptr.address);
   m.two = static_cast<uint32_t>(rec.merges_two);
-  m.blocks = m.two * (kPfTokens / kPfMergeRows) + (static_cast<uint32_t>(rec.merges) - m.two) * kPfTokens;
+  const auto tokens = static_cast<uint32_t>(rec.item_tokens);
+  m.blocks = m.two * (tokens / kPfMergeRows) + (static_cast<uint32_t>(rec.merges) - m.two) * tokens;
   return m;
 }
 
@@ -2524,13 +2629,11 @@ RoostStatus LaunchPrefillMerge(const RoostPagedAttentionParams& p, const PlanRec
   auto* lsep = static_cast<float*>(p.lse.address);
   const PrefillMergeArgs m = PrefillMergeArgsOf(p, rec, dev);
   const dim3 block(kGroup * p.head_dim / 4), g(m.blocks);
-  if (p.head_dim == 64) {
-    hipLaunchKernelGGL(PrefillMergeKernel<64>, g, block, 0, stream, outp, lsep, m, p.q_heads, kv.out_gate);
-  } else if (p.head_dim == 128) {
-    hipLaunchKernelGGL(PrefillMergeKernel<128>, g, block, 0, stream, outp, lsep, m, p.q_heads, kv.out_gate);
-  } else {
-    hipLaunchKernelGGL(PrefillMergeKernel<256>, g, block, 0, stream, outp, lsep, m, p.q_heads, kv.out_gate);
-  }
+  const bool wide = rec.item_tokens == kPfWideTokens;
+  auto* kernel = p.head_dim == 64    ? PrefillMergeKernel<64, kPfTokens>
+                 : p.head_dim == 128 ? (wide ? PrefillMergeKernel<128, kPfWideTokens> : PrefillMergeKernel<128, kPfTokens>)
+                                     : PrefillMergeKernel<256, kPfTokens>;
+  hipLaunchKernelGGL(kernel, g, block, 0, stream, outp, lsep, m, p.q_heads, kv.out_gate);
   return roost::HipStatus(hipGetLastError(), "paged_attention", "prefill merge launch");
 }
 
@@ -2602,15 +2705,17 @@ RoostStatus LaunchPrefill(const RoostPagedAttentionParams& p, const PlanRecord& 
     const SoftCap raw{cap.capl / scale_log2, cap.k * scale_log2};
     const bool capped = cap.capl != 0.0f;
     auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, q16, outp, lsep, kv, kv.kv_indices, q_indptr, items,
-                         part_o, part_ml, p.q_heads, p.causal, ps_shift, scale_log2, WindowOf(p), raw);
+      hipLaunchKernelGGL(kernel, grid, dim3(static_cast<uint32_t>(8 * rec.item_tokens)), 0, stream, q16, outp, lsep, kv, kv.kv_indices,
+                         q_indptr, items, part_o, part_ml, p.q_heads, p.causal, ps_shift, scale_log2, WindowOf(p), raw);
     };
+    const bool wide = rec.item_tokens == kPfWideTokens;
     if (p.head_dim == 64) {
-      capped ? launch(PrefillTileKernel<64, true>) : launch(PrefillTileKernel<64, false>);
+      capped ? launch(PrefillTileKernel<64, true, 8>) : launch(PrefillTileKernel<64, false, 8>);
     } else if (p.head_dim == 128) {
-      capped ? launch(PrefillTileKernel<128, true>) : launch(PrefillTileKernel<128, false>);
+      wide ? (capped ? launch(PrefillTileKernel<128, true, 12>) : launch(PrefillTileKernel<128, false, 12>))
+           : (capped ? launch(PrefillTileKernel<128, true, 8>) : launch(PrefillTileKernel<128, false, 8>));
     } else {
-      capped ? launch(PrefillTileKernel<256, true>) : launch(PrefillTileKernel<256, false>);
+      capped ? launch(PrefillTileKernel<256, true, 8>) : launch(PrefillTileKernel<256, false, 8>);
     }
     ROOST_RETURN_IF_FAILED(roost::HipStatus(hipGetLastError(), "paged_attention", "prefill launch"));
     return LaunchPrefillMerge(p, rec, dev, kv, stream);
@@ -2641,6 +2746,7 @@ PlanRecord MakeRecord(const RoostPagedAttentionParams& p, const Layout& l) {
   r.kv_heads = p.kv_heads;
   r.window = WindowOf(p);
   r.merges_two = static_cast<uint32_t>(l.merges_two);
+  r.item_tokens = l.item_tokens;
   r.overlap = l.overlap;
   r.dec_heads_per_wg = l.dec_heads_per_wg;
   r.pages = static_cast<uint64_t>(p.kv_indptr_host[p.batch]);

@@ -1,0 +1,52 @@
+"""The prefill plan's two late choices against float32 torch: the 12-wavefront, 96-token items of head dim 128 (item edges
+around 32, 64 and 96 tokens, split and whole items, prefixes, both layouts), and short prompts cut into pieces of 2 to 7 tiles
+while CUs are idle (piece edges, several pieces per item, every head dim)."""
+import ctypes as C
+import dataclasses
+
+import numpy as np
+import pytest
+
+import cases
+import roost_amd
+from test_attention_gpu import Dev, torch_reference
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(session, b, key, **kw):
+    """The result and, from the plan record: work items, merges, and its last word, the query tokens per item."""
+    dev = Dev(b, **kw)
+    entry = session.lib.entry(roost_amd.ATTENTION_VARIANT)
+    session.launch(entry, dev.params(), key=key)
+    ws = session._ws[(entry.variant_id, key)][3]
+    words = np.frombuffer(C.string_at(ws.plan, ws.plan_bytes), np.uint64)
+    got = dev.result()
+    assert not np.isnan(got).any()
+    return got, int(words[7]), int(words[9]), int(words[-1])
+
+
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (64, 4)])
+@pytest.mark.parametrize("new,pre", [([1791, 1889, 1984, 2000, 33, 2], [0, 5, 1000, 64, 0, 7]),
+                                           ([4001, 97, 4096, 96, 3999, 95], [0, 0, 0, 31, 17, 900])])
+@pytest.mark.parametrize("hnd,ps", [(False, 16), (True, 64)])
+def test_wide_items(session, hq, hkv, new, pre, hnd, ps):
+    rng = np.random.default_rng(sum(new) + hq)
+    b = cases.make_paged_batch(rng, [a + p for a, p in zip(new, pre)], new, page_size=ps, hnd=hnd, hq=hq, hkv=hkv, d=128,
+                               std=0.5)
+    got, _, _, tokens = _run(session, b, ("wide", hq, sum(new), hnd))
+    assert tokens == 96, "the plan did not take the wide items"
+    if hnd:  # the reference reads NHD pools
+        b = dataclasses.replace(b, k_cache=b.k_cache.transpose(0, 2, 1, 3), v_cache=b.v_cache.transpose(0, 2, 1, 3))
+    cases.assert_close(got, torch_reference(b), what="wide prefill vs fp32 torch")
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 256), (8, 2, 128), (4, 1, 64)])
+@pytest.mark.parametrize("new,pre", [([500], [0]), ([1025], [0]), ([1777], [0]), ([256], [4001]), ([64], [8000]),
+                                     ([129, 2, 1, 300], [0, 640, 900, 33])])
+def test_short_prompts_in_small_pieces(session, hq, hkv, d, new, pre):
+    rng = np.random.default_rng(sum(new) + d)
+    b = cases.make_paged_batch(rng, [a + p for a, p in zip(new, pre)], new, hq=hq, hkv=hkv, d=d, std=0.5)
+    got, items, merges, tokens = _run(session, b, ("sparse", d, sum(new)))
+    assert tokens == 64 and (merges > 0 or d < 256 or len(new) > 1) and items <= 256
+    cases.assert_close(got, torch_reference(b), what="short prompt vs fp32 torch")
