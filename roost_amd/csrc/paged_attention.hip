@@ -688,9 +688,8 @@ PieceChoice PrefillPieceTiles(const ItemList& items, uint32_t cus) {
 // tiles for 256 CUs): pieces below kPfMinSplitTiles, down to 2 tiles, while they still run in one round. Each is priced by
 // what such calls measured: a tile on a chip with idle CUs 2.3 us at head dim 256, the merge launch 4.5 us, and 0.08 us
 // per piece for its partial rows written and merged (both sides less at smaller head dims). Fresh prompts at head dim
-// 256, 8 heads, pieces of at most 8 tiles against this choice: 500 tokens 34.6 -> 25.3 us (2 tiles), 1,000 41.7 -> 32.2
-// (2), 1,777 49.9 -> 42.6 (4); 256 tokens on 4,000 cached ones 44.6 -> 35.6 (4). 200 tokens stay whole: 21.1 against
-// 23.0 us in pieces of 2.
+// 256, 8 heads, pieces of at most 8 tiles against this choice: 500 tokens 34.6 -> 25.1 us, 1,000 41.7 -> 35.0, 1,777
+// 49.9 -> 43.4; 256 tokens on 4,000 cached ones 44.6 -> 35.2. 200 tokens stay whole: 21.1 against 23.0 us in pieces of 2.
 constexpr double kSparseTileUs = 2.3;
 constexpr double kPieceMergeUs = 0.08;
 constexpr double kMergeLaunchUs = 4.5;
