@@ -499,9 +499,9 @@ __global__ void __launch_bounds__(256) ConvTileKernel(ConvArgs a, uint32_t cbloc
         starts |= 1 << i;
         const int32_t slot = __builtin_amdgcn_readlane(lane_slot, k);
         slots[i] = slot >= 0 && static_cast<uint64_t>(slot) < a.pool_slots ? slot : -1;
-        if (pairs) {
+        if (pairs && slots[i] >= 0) {  // a slot outside the pool: nothing is read (the pool may hold no slot at all)
           const auto* sp = reinterpret_cast<const uint32_t*>(
-              static_cast<const uint16_t*>(a.state) + (static_cast<uint64_t>(max(slots[i], 0)) * a.channels + c0) * sl);
+              static_cast<const uint16_t*>(a.state) + (static_cast<uint64_t>(slots[i]) * a.channels + c0) * sl);
 #pragma unroll
           for (int k = 0; k < kSw; ++k) sw[i][k] = sp[k];
         }
@@ -558,9 +558,9 @@ __global__ void __launch_bounds__(256) ConvShortKernel(ConvArgs a) {
   const bool bf_state = a.state_t == ROOST_DTYPE_BF16;
   const int32_t slot = rel < sl ? a.slots[b] : -1;
   const bool ok = slot >= 0 && static_cast<uint64_t>(slot) < a.pool_slots;
-  uint32_t sq[kSq][4] = {};
-  if (rel < sl) {  // some taps come from the state: the 8 channels' entries are 8 x sl contiguous elements
-    const uint64_t so = (static_cast<uint64_t>(ok ? slot : 0) * a.channels + c0) * sl;
+  uint32_t sq[kSq][4] = {};  // zeros: the history of a slot outside the pool, which is not read (it may hold no slot)
+  if (ok) {  // some taps come from the state: the 8 channels' entries are 8 x sl contiguous elements
+    const uint64_t so = (static_cast<uint64_t>(slot) * a.channels + c0) * sl;
     if (bf_state) {
 #pragma unroll
       for (int q = 0; q < sl; ++q) LoadWords<16>(static_cast<const uint16_t*>(a.state) + so + 8 * q, sq[q]);
@@ -601,7 +601,7 @@ __global__ void __launch_bounds__(256) ConvShortKernel(ConvArgs a) {
 #pragma unroll
     for (int e = 0; e < kV; ++e)
 #pragma unroll
-      for (int i = 0; i < sl; ++i) st[e][i] = ok ? flat[e * sl + i] : 0.0f;
+      for (int i = 0; i < sl; ++i) st[e][i] = flat[e * sl + i];
   }
 #pragma unroll
   for (int j = 0; j < kW; ++j) {

@@ -59,6 +59,32 @@ def test_conv_tile_odd_state_address(session):
     assert np.array_equal(from_dev(pool, True), want_state)
 
 
+@pytest.mark.parametrize("whole", [0, 1], ids=["no slot", "one slot"])
+@pytest.mark.parametrize("bf16_state", [True, False])
+@pytest.mark.parametrize("lens", [[5, 70, 0, 33, 1, 2, 40, 300], [1, 2, 1, 5, 1]], ids=["tiles", "short"])
+def test_conv_slots_outside_the_pool(session, lens, bf16_state, whole):
+    """A call without history: slots of -1 and beyond a pool that may hold no slot at all (the span ends with it). Absent
+    slots read nothing, so the results are those of a zero history and the pool, NaN throughout, stays as it is."""
+    rng = np.random.default_rng(len(lens) + whole)
+    ch, width, T, B = 2048, 4, sum(lens), len(lens)
+    x, w = (cases.bf16_bits(rng.standard_normal(n).astype(np.float32)) for n in (T * ch, ch * width))
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    want, zeros = np.zeros(T * ch, np.uint16), np.zeros(B * ch * 3, np.float32)
+    oracle.causal_conv1d(x, w, None, want, zeros, np.arange(B, dtype=np.int32), cu, batch=B, tokens=T, channels=ch,
+                         width=width, silu=True)
+    slots = np.array([-1 if i % 2 else whole + i for i in range(B)], np.int32)
+    nan = np.full(ch * 3, np.nan, np.float32)
+    pool = to_dev(cases.bf16_bits(nan), True) if bf16_state else to_dev(nan, False)
+    before = pool.clone()
+    out = to_dev(np.zeros(T * ch, np.uint16), True)
+    p = roost_amd.causal_conv1d_params(to_dev(x, True), to_dev(w, True), None, out, pool, to_dev(slots), to_dev(cu),
+                                       batch=B, tokens=T, channels=ch, width=width, silu=True)
+    p.conv_state.length = whole * ch * 3
+    session.launch(session.lib.entry(roost_amd.CAUSAL_CONV1D_VARIANT), p)
+    assert_close(from_dev(out, True), want, True)
+    assert from_dev(pool, bf16_state).tobytes() == from_dev(before, bf16_state).tobytes()
+
+
 def test_layer_output_over_the_convolution_input(session):
     """The GDN output in the convolution's input buffer (dead once the convolution has run): the state update, which reads
     that input, may then not wait for the layer's last launch."""
