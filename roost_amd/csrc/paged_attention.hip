@@ -1356,8 +1356,10 @@ __global__ void __launch_bounds__(256, kDecodeWgsPerCu)
 //     v_mfma_f32_16x16x16_bf16;
 //   * it loads the D / 16 dims of slice c of tokens 4g .. 4g + 3 (whole rows per 16 lanes), and pairs of those rows
 //     interleaved with v_perm are the B operands: one multiply per dim e of the slice gives heads 4g + j, dim (c, e).
-// The running maximum moves only when a score exceeds it by more than 2^8 (as in the prefill kernels: weights stay below
-// 256), so the exchange that brings a head's rescale factor to the lanes holding its sums is rare.
+// The running maximum is the exact one, so a head's largest weight is 1, which bf16 holds: kept up to 2^8 below the scores
+// (as the prefill kernels do), it let a dominant weight be rounded where its denominator was not, and a whole peaked row
+// came out up to 2^-8 off, or infinite for V past 1e36. It moves in a wavefront's first groups and rarely later; only then
+// are a head's rescale factors brought to the lanes holding its sums.
 //
 // Bound by HBM. One register buffer each for a group's K and V rows: the next group's K rows are requested once the
 // scores have read these, its V rows once P.V has, so one of the two is in flight at all times. Two buffers of each
@@ -1521,9 +1523,8 @@ __device__ __forceinline__ void DecodeMfmaBody(const uint16_t* __restrict__ q, u
       }
       mx = fmaxf(mx, ShflXor(mx, 16));
       mx = MaxXor32(mx);
-      const bool grow = mx > m_run + 8.0f;
-      if (__any(grow)) {
-        const float m_new = grow ? mx : m_run;
+      if (__any(mx > m_run)) {
+        const float m_new = fmaxf(m_run, mx);
         const float corr = m_run == -INFINITY ? 0.0f : exp2f(m_run - m_new);
         l_lane *= corr;
         m_run = m_new;
@@ -1538,7 +1539,7 @@ __device__ __forceinline__ void DecodeMfmaBody(const uint16_t* __restrict__ q, u
       const float m_use = m_run == -INFINITY ? 0.0f : m_run;  // a head with no visible key yet keeps p = 0
       float p[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(s[j] - m_use);
+      for (int j = 0; j < 4; ++j) p[j] = exp2f(s[j] - m_use);
       l_lane += (p[0] + p[1]) + (p[2] + p[3]);
       const i16x4v_t pa = __builtin_bit_cast(i16x4v_t, u32x2_t{PackRne(p[0], p[1]), PackRne(p[2], p[3])});
 #pragma unroll
@@ -1609,8 +1610,10 @@ __device__ __forceinline__ void DecodeMfmaBody(const uint16_t* __restrict__ q, u
       const uint32_t qh = ((block % hblocks) * heads_per_wg + hk) * NH + h;
       if (split < 0) {
         const uint64_t row = tok * q_heads + qh;
-        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-        const u32x2_t v{PackBf16(o[0] * inv, o[1] * inv), PackBf16(o[2] * inv, o[3] * inv)};
+        float y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = L > 0.0f ? o[i] / L : 0.0f;
+        const u32x2_t v{PackBf16(y[0], y[1]), PackBf16(y[2], y[3])};
         *reinterpret_cast<u32x2_t*>(out + row * D + d) = GateOut2(kv.out_gate, row * D + d, v);
         if (lse != nullptr && d == 0) lse[row] = L > 0.0f ? M + log2f(L) : -INFINITY;
       } else {

@@ -2,12 +2,14 @@
 heads a wavefront serves (4, 8, 16; 32 as two of 16), every head dim, pages that hold whole groups and pages that do not,
 windows that start inside a group, and scores large enough to move the running maximum many times. Against the CpuOps
 oracle within the attention-bf16 class of tests/cases.py; the one-launch mixed step against float32 torch."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import cases
 import roost_amd
-from test_attention_gpu import Dev, _plan_overlap, run_case, torch_reference
+from test_attention_gpu import Dev, _plan_overlap, from_dev, run_case, to_dev, torch_reference
 
 pytestmark = pytest.mark.gpu
 
@@ -52,3 +54,43 @@ def test_mixed_launch_query_head_groups(session, hq, hkv, d):
     session.launch(session.lib.entry(roost_amd.ATTENTION_VARIANT), dev.params(), key=key)
     assert _plan_overlap(session, key) == 1
     cases.assert_close(dev.result(), torch_reference(b), what="mixed step vs fp32 torch")
+
+
+def _staircase(rng, hq, hkv, d, rows, groups, v_bits):
+    """Contexts whose 16-token groups each hold one visible key, its score a step above that of the group before (the step
+    is left to q's first element); every value of V the same."""
+    b = cases.make_paged_batch(rng, [16 * groups] * rows, [1] * rows, hq=hq, hkv=hkv, d=1, pool_factor=1.0)
+    shape = b.k_cache.shape[:3] + (d,)
+    k = np.zeros(shape, np.float32)
+    k[..., 0] = -300.0
+    for r in range(rows):
+        k[b.kv_indices[b.kv_indptr[r]:b.kv_indptr[r + 1]], 0, :, 0] = np.arange(groups)[:, None]
+    b.d, b.q = d, np.zeros((rows, hq, d), np.uint16)
+    b.k_cache, b.v_cache = cases.bf16_bits(k), np.full(shape, v_bits, np.uint16)
+    return b
+
+
+@pytest.mark.parametrize("hq", [16, 32, 64, 128], ids=["g4", "g8", "g16", "g32"])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("v_bits", [0x3FFF, 0x7BFF], ids=["V 1.99", "V 2.65e36"])
+def test_decode_rising_scores_keep_the_dominant_weight(session, hq, d, v_bits):
+    """A head's largest weight is exactly 1 in bf16, whatever the scores before it. A wavefront's scores rise by a step of 2
+    to 7.5 in log2 (another for every row and head) from each of its groups to the next, so the roundings of the other
+    weights (2^-8 of each at most) move a row by at most 2^-8 * 2^-2: less than half a unit of V's last place (2^-9 of it,
+    V's mantissa being full), and the output is V to the bit. A weight of up to 2^7.5 would also overflow: 2^7.5 * 2.65e36
+    is past the largest float."""
+    rng = np.random.default_rng(d + hq)
+    rows, groups = 48, 64
+    b = _staircase(rng, hq, 4, d, rows, groups, v_bits)
+    dev = Dev(b)
+    entry = session.lib.entry(roost_amd.ATTENTION_VARIANT)
+    ws = session.prepare(entry, dev.params(), ("staircase", d, hq))
+    words = np.frombuffer(C.string_at(ws.plan, ws.plan_bytes), np.uint64)
+    waves = 4 // (int(words[5]) >> 32)  # wavefronts that take a head's groups in turn
+    assert int(words[7]) * 2 * waves <= rows * groups, "the plan leaves a wavefront fewer than two groups"
+    q = np.zeros(b.q.shape, np.float32)
+    q[..., 0] = rng.uniform(2.0 / waves, 7.5 / waves, q.shape[:2]) * np.sqrt(d) / np.log2(np.e)
+    dev.q.copy_(to_dev(cases.bf16_bits(q), True))
+    session.run(entry, dev.params(), ws)
+    got = from_dev(dev.out, True)
+    assert (got == v_bits).all(), f"{(got != v_bits).sum()} of {got.size} outputs differ from V"
