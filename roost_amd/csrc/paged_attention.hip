@@ -1539,7 +1539,7 @@ __device__ __forceinline__ void DecodeMfmaBody(const uint16_t* __restrict__ q, u
       const float m_use = m_run == -INFINITY ? 0.0f : m_run;  // a head with no visible key yet keeps p = 0
       float p[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) p[j] = exp2f(s[j] - m_use);
+      for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(s[j] - m_use);
       l_lane += (p[0] + p[1]) + (p[2] + p[3]);
       const i16x4v_t pa = __builtin_bit_cast(i16x4v_t, u32x2_t{PackRne(p[0], p[1]), PackRne(p[2], p[3])});
 #pragma unroll
@@ -1610,10 +1610,8 @@ __device__ __forceinline__ void DecodeMfmaBody(const uint16_t* __restrict__ q, u
       const uint32_t qh = ((block % hblocks) * heads_per_wg + hk) * NH + h;
       if (split < 0) {
         const uint64_t row = tok * q_heads + qh;
-        float y[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) y[i] = L > 0.0f ? o[i] / L : 0.0f;
-        const u32x2_t v{PackBf16(y[0], y[1]), PackBf16(y[2], y[3])};
+        const float inv = L > 0.0f ? 1.0f / L : 0.0f;  // four divisions: 2% of a call of one-group contexts
+        const u32x2_t v{PackBf16(o[0] * inv, o[1] * inv), PackBf16(o[2] * inv, o[3] * inv)};
         *reinterpret_cast<u32x2_t*>(out + row * D + d) = GateOut2(kv.out_gate, row * D + d, v);
         if (lse != nullptr && d == 0) lse[row] = L > 0.0f ? M + log2f(L) : -INFINITY;
       } else {
