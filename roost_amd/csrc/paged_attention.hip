@@ -168,6 +168,8 @@ struct PlanRecord {
   // Single-token sequences of a prefill call run as decode: their pieces, ranges, merges and partials.
   uint64_t dec_items, dec_ranges, dec_merges, dec_splits;
   uint64_t dec_item_offset, dec_range_offset, dec_merge_offset, dec_float_offset;
+  uint32_t q_heads;      // the partials' row stride and, in a prefill, the items' heads
+  uint32_t dtype;        // PlanDtype(params): the kernels the tables were made for
   uint64_t item_tokens;  // prefill: query tokens per work item (kPfTokens or kPfWideTokens)
 };
 
@@ -2550,13 +2552,6 @@ RoostStatus LaunchDecodeMerge(const RoostPagedAttentionParams& p, const PlanReco
   return roost::HipStatus(hipGetLastError(), "paged_attention", "decode merge launch");
 }
 
-// KV heads per decode workgroup at run time: the plan's, unless the call's heads are not what it was made for (the record
-// does not hold q_heads or the element type); the ranges it dealt serve any number.
-uint32_t RunHeadsPerWorkgroup(const RoostPagedAttentionParams& p, const PlanRecord& rec) {
-  const uint32_t hpw = rec.dec_heads_per_wg;
-  return (hpw == 1 || hpw == 2 || hpw == 4) && DecodeHeads(p) % hpw == 0 ? hpw : HeadsPerWorkgroup(p);
-}
-
 // The view of the decode kernels, whose virtual heads are groups of DecodeGroupOf query heads.
 KvView DecodeView(const RoostPagedAttentionParams& p, KvView kv) {
   kv.vheads = DecodeHeads(p);
@@ -2577,7 +2572,7 @@ RoostStatus LaunchDecode(const RoostPagedAttentionParams& p, const PlanRecord& r
       p.mode == ROOST_ATTENTION_PREFILL ? static_cast<const int32_t*>(p.q_indptr.address) : nullptr;
   auto* out = static_cast<T*>(p.output.address);
   auto* lse = static_cast<float*>(p.lse.address);
-  const uint32_t heads = DecodeHeads(p), hpw = RunHeadsPerWorkgroup(p, rec);
+  const uint32_t heads = DecodeHeads(p), hpw = rec.dec_heads_per_wg;
   const KvView dkv = DecodeView(p, kv);
   const dim3 grid(static_cast<uint32_t>(rec.dec_ranges * (heads / hpw)));
   auto launch = [&](auto kernel) {
@@ -2651,7 +2646,7 @@ RoostStatus LaunchMixed(const RoostPagedAttentionParams& p, const PlanRecord& re
   const SoftCap raw{cap.capl / scale_log2, cap.k * scale_log2};
   const bool capped = cap.capl != 0.0f;
   const KvView dkv = DecodeView(p, kv);
-  const uint32_t hpw = RunHeadsPerWorkgroup(p, rec);
+  const uint32_t hpw = rec.dec_heads_per_wg;
   const uint32_t n_items = static_cast<uint32_t>(rec.work_items);
   const dim3 grid(n_items + static_cast<uint32_t>(rec.dec_ranges * (dkv.vheads / hpw)));
   const auto* dec_items = reinterpret_cast<const DecodeWork*>(dev + rec.dec_item_offset);
@@ -2733,6 +2728,13 @@ const RoostPagedAttentionParams* Params(const void* params) {
   return static_cast<const RoostPagedAttentionParams*>(params);
 }
 
+// The element type a plan is made for. plan() reads no spans, so a caller may leave it out: the tables are then those of
+// bf16, which in a decode call also serve f32 (the partials are f32 rows either way, and every workgroup's share of bf16
+// head groups divides the f32 ones).
+uint32_t PlanDtype(const RoostPagedAttentionParams& p) {
+  return p.q.dtype == ROOST_DTYPE_F32 || p.q.dtype == ROOST_DTYPE_BF16 ? p.q.dtype : ROOST_DTYPE_UNDEFINED;
+}
+
 // The plan record plan() leaves for run(): the batch shape it was made for and where its tables sit.
 PlanRecord MakeRecord(const RoostPagedAttentionParams& p, const Layout& l) {
   PlanRecord r{};
@@ -2747,6 +2749,8 @@ PlanRecord MakeRecord(const RoostPagedAttentionParams& p, const Layout& l) {
   r.window = WindowOf(p);
   r.merges_two = static_cast<uint32_t>(l.merges_two);
   r.item_tokens = l.item_tokens;
+  r.q_heads = p.q_heads;
+  r.dtype = PlanDtype(p);
   r.overlap = l.overlap;
   r.dec_heads_per_wg = l.dec_heads_per_wg;
   r.pages = static_cast<uint64_t>(p.kv_indptr_host[p.batch]);
@@ -2771,8 +2775,12 @@ PlanRecord MakeRecord(const RoostPagedAttentionParams& p, const Layout& l) {
   return r;
 }
 
+// The partials and, in a prefill, the items are laid out for the plan's query heads, and a prefill's tables for its element
+// type: run with others, the kernels would write past the workspace or leave rows unwritten.
 bool RecordFits(const PlanRecord& r, const RoostPagedAttentionParams& p) {
-  return r.mode == p.mode && r.batch == p.batch && r.tokens == p.tokens && r.page_size == p.page_size &&
+  const bool dtype = r.dtype == p.q.dtype || (r.dtype == ROOST_DTYPE_UNDEFINED &&
+                                              (p.mode == ROOST_ATTENTION_DECODE || p.q.dtype == ROOST_DTYPE_BF16));
+  return dtype && r.q_heads == p.q_heads && r.mode == p.mode && r.batch == p.batch && r.tokens == p.tokens && r.page_size == p.page_size &&
          r.kv_layout == p.kv_layout && r.head_dim == p.head_dim && r.kv_heads == p.kv_heads && r.window == WindowOf(p);
 }
 
@@ -2855,7 +2863,7 @@ RoostStatus RunAttention(RoostContext* ctx, const void* params, const RoostWorks
     }
     gate.Expect(RecordFits(rec, p), ROOST_STATUS_INVALID_ARGUMENT,
                 "the plan record describes batch %u / tokens %u / mode %u / window %d; this call is batch %u / tokens "
-                "%u / mode %u / window %d (or its page size, layout, head shape differ)", rec.batch, rec.tokens,
+                "%u / mode %u / window %d (or its page size, layout, head shape or element type differ)", rec.batch, rec.tokens,
                 rec.mode, rec.window, p.batch, p.tokens, p.mode, WindowOf(p))
         .Tensor("kv_indices", p.kv_indices, ROOST_DTYPE_I32, rec.pages)
         .Expect(HasDeviceRegion(ws, rec.float_offset + rec.float_bytes, kAlign), ROOST_STATUS_WORKSPACE_TOO_SMALL,

@@ -557,6 +557,34 @@ def test_sliding_window_plan_must_match_run(session):
     assert session.run_raw(entry, d.params(), ws) == abi.INVALID_ARGUMENT
 
 
+@pytest.mark.parametrize("q_lens", [[1, 1], [130, 1]], ids=["decode", "prefill"])
+def test_plan_must_match_the_query_heads_and_element_type(session, q_lens):
+    """A plan's partial rows are laid out for its query heads and its tables for its element type: a run with others is
+    refused (it would write past the workspace, or leave rows unwritten). A plan without a type is one for bf16, which in a
+    decode call serves f32 too."""
+    rng = np.random.default_rng(78)
+    heads = {hq: cases.make_paged_batch(rng, [700, 4000], q_lens, hq=hq, hkv=2) for hq in (8, 16, 32)}
+    f32 = cases.make_paged_batch(rng, [700, 4000], q_lens, bf16=False)
+    entry = session.lib.entry(roost_amd.ATTENTION_VARIANT)
+    key = ("plan match", len(q_lens), q_lens[0])
+    for planned, runs in ((heads[8], [heads[16], heads[32], f32]), (heads[32], [heads[8]]), (f32, [heads[8]])):
+        ws = session.prepare(entry, Dev(planned).params(), key)
+        for b in runs:
+            d = Dev(b)
+            assert session.run_raw(entry, d.params(), ws) == abi.INVALID_ARGUMENT
+            assert torch().isnan(d.out).all()
+    for b in (heads[8], f32):
+        d = Dev(b)
+        untyped = d.params()
+        untyped.q.dtype = 0  # undefined
+        ws = session.prepare(entry, untyped, key)
+        if b.bf16 or q_lens[0] == 1:
+            session.run(entry, d.params(), ws)
+            check_against_oracle(d.result(), b)
+        else:
+            assert session.run_raw(entry, d.params(), ws) == abi.INVALID_ARGUMENT
+
+
 # ---- Prefill at head_dim 128 (the tile kernel templated on the head dim; decode already serves 64/128/256) ---------
 
 HD128_PREFILL_CASES = [
