@@ -1039,6 +1039,10 @@ __device__ __forceinline__ float Pick4(const float* x, int i) {
   return i == 0 ? x[0] : (i == 1 ? x[1] : (i == 2 ? x[2] : x[3]));
 }
 
+// What the f32 decode kernel reads as the V row of a token that is not there, where no visible token's row is at hand: its
+// weight is 0, but 0 times a row that nobody wrote may be NaN. 256 floats, the longest row.
+__device__ __align__(16) uint32_t kZeroRow[256];
+
 // ---- f32 decode kernel -----------------------------------------------------------------------------------------------
 
 template <int D>
@@ -1232,6 +1236,9 @@ __global__ void __launch_bounds__(256, kDecodeWgsPerCu)
   // Every load is unconditional: a group index past the end is clamped to the wave's last group and its keys are
   // masked, so the number of loads in flight is the same on every path and the compiler can wait for exactly the
   // current group's data (vmcnt) while the next group's loads stay in flight.
+  constexpr bool kZeroGroup = D <= 128;
+  // Absent tokens read the V row of their group's first visible token. A group without any reads kZeroRow, or at head dim
+  // 256, where the registers spill and the further address costs more (16 contexts around 4,000: 203 -> 224 us; 209 as it is), is not computed.
   auto load = [&](uint32_t gi, uint4* kr, uint4* vr, uint32_t& valid) {
     valid = 0;
     const uint32_t g0 = t_begin + 16u * (wave + waves_per_head * min(gi, nw - 1));
@@ -1246,15 +1253,21 @@ __global__ void __launch_bounds__(256, kDecodeWgsPerCu)
       const uint64_t row0 = kv.hnd ? (pg * kv.kv_heads + kvr) * kv.page_size + off0
                                    : (pg * kv.page_size + off0) * kv.kv_heads + kvr;
       const char* kg = reinterpret_cast<const char*>(kbase + row0 * D);
+      const uint32_t n = page_ok ? min(16u, t_end - g0) : 0u;
+      const bool any = page_ok && max(lo, g0) < min(g0 + 16u, t_end);  // a visible token in the group
+      const uint32_t first = any ? max(lo, g0) - g0 : 0;
+      const uint32_t visible = any ? ((1u << n) - 1u) & ~((1u << first) - 1u) : 0u;  // bit t: token t
       const char* vg = reinterpret_cast<const char*>(vbase + row0 * D);
+      if (kZeroGroup && !any) vg = reinterpret_cast<const char*>(kZeroRow);
 #pragma unroll
       for (int i = 0; i < kNi; ++i) {
         const uint32_t tv = i * kTpi + ri;  // V register i: slot i
-        const bool okv = live && page_ok && g0 + tv < t_end && g0 + tv >= lo;
-        vr[i] = LoadStream16(vg + ((okv ? tv : 0) * tok_bytes + r * 16));
+        const bool okv = kZeroGroup ? ((visible >> tv) & 1u) != 0 && live
+                                    : live && page_ok && g0 + tv < t_end && g0 + tv >= lo;
+        vr[i] = LoadStream16(vg + ((okv ? tv : first) * tok_bytes + r * 16));
         const uint32_t tk = (i ^ kperm) * kTpi + ri;  // K register i: slot i ^ kperm
-        const bool okk = page_ok && g0 + tk < t_end;
-        kr[i] = LoadStream16(kg + ((okk ? tk : 0) * tok_bytes + r * 16));
+        const uint32_t row = kZeroGroup ? min(tk, max(n, 1u) - 1) : (page_ok && g0 + tk < t_end ? tk : 0);
+        kr[i] = LoadStream16(kg + (row * tok_bytes + r * 16));
         valid |= static_cast<uint32_t>(okv) << i;
       }
     } else {
@@ -1267,7 +1280,7 @@ __global__ void __launch_bounds__(256, kDecodeWgsPerCu)
                                             static_cast<int32_t>(t_end), kvh, &okv);
         okv = okv && g0 + i * kTpi + ri >= lo;
         kr[i] = *reinterpret_cast<const uint4*>(kbase + rowk + r * kVec);
-        vr[i] = LoadStream16(vbase + rowv + r * kVec);
+        vr[i] = LoadStream16((okv ? vbase + rowv : reinterpret_cast<const float*>(kZeroRow)) + r * kVec);
         valid |= static_cast<uint32_t>(okv && live) << i;
       }
     }
@@ -1286,7 +1299,7 @@ __global__ void __launch_bounds__(256, kDecodeWgsPerCu)
         constexpr int kLast = kDecodeRing - 1;
         const int nxt = (s + kLast) % kDecodeRing;
         load(gi + s + kLast, kbuf[nxt], vbuf[nxt], valid[nxt]);
-        if (gi + s < nw) {
+        if (gi + s < nw && (kZeroGroup || !kFastPage || __any(valid[s] != 0))) {
           DecodeGroup<D>(st, kbuf[s], vbuf[s], valid[s], qr, x_lds[wave_id], r, ri, lane, scale_log2, cap);
         }
       }
@@ -1472,7 +1485,9 @@ __device__ __forceinline__ void DecodeMfmaBody(const uint16_t* __restrict__ q, u
       if (a.g0 < lo) a.valid &= ~((1u << min(16u, lo - a.g0)) - 1u);  // before the window
       return a;
     };
-    // Rows of absent tokens are read as the group's first (general pages: as the pool's first).
+    // Rows of absent tokens: K reads the group's first (general pages: the pool's first), whose score is masked. V reads
+    // the group's first visible token's, since a weight of 0 times a row that nobody wrote may be NaN; a group without a
+    // visible token is not folded.
     auto load_k = [&](const Place& a, u32x4_t* kr) {
       const char* kg = reinterpret_cast<const char*>(kbase + a.row);
       const uint32_t ko = (kFastPage && a.page_ok && a.g0 + c < t_end ? c : 0) * tok_bytes + g * 16;
@@ -1483,13 +1498,14 @@ __device__ __forceinline__ void DecodeMfmaBody(const uint16_t* __restrict__ q, u
       }
     };
     auto load_v = [&](const Place& a, vword_t (*vr)[4]) {
+      const uint32_t first = a.valid != 0 ? __builtin_ctz(a.valid) : 0;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const uint32_t tv = 4 * g + i;
+        const uint32_t tv = ((a.valid >> (4 * g + i)) & 1u) ? 4 * g + i : first;
         uint64_t row = a.row;
         uint32_t vo = c * (2 * kSlice);
         if constexpr (kFastPage) {
-          vo += (((a.valid >> tv) & 1u) ? tv : 0) * tok_bytes;
+          vo += tv * tok_bytes;
         } else {
           bool ok;
           row = KeyRowSafe<D>(kv, p0, static_cast<int32_t>(a.g0 + tv), static_cast<int32_t>(t_end), kvh, &ok);
@@ -1569,7 +1585,7 @@ __device__ __forceinline__ void DecodeMfmaBody(const uint16_t* __restrict__ q, u
         const f32x4_t s = scores(kr);
         __builtin_amdgcn_sched_barrier(0);  // the next K rows are requested as soon as the scores have read these
         load_k(nxt, kr);
-        fold(s, vr, cur.valid);
+        if (cur.valid != 0) fold(s, vr, cur.valid);
         __builtin_amdgcn_sched_barrier(0);
         load_v(nxt, vr);
         cur = nxt;

@@ -3,6 +3,7 @@ heads a wavefront serves (4, 8, 16; 32 as two of 16), every head dim, pages that
 windows that start inside a group, and scores large enough to move the running maximum many times. Against the CpuOps
 oracle within the attention-bf16 class of tests/cases.py; the one-launch mixed step against float32 torch."""
 import ctypes as C
+import dataclasses
 
 import numpy as np
 import pytest
@@ -94,3 +95,53 @@ def test_decode_rising_scores_keep_the_dominant_weight(session, hq, d, v_bits):
     session.run(entry, dev.params(), ws)
     got = from_dev(dev.out, True)
     assert (got == v_bits).all(), f"{(got != v_bits).sum()} of {got.size} outputs differ from V"
+
+
+def _unwritten_is_nan(b, window, bad_page):
+    """The batch with NaN wherever no query can look: page 0, pages of no sequence, a context's last page past its end and
+    everything before its window. bad_page: one page in the middle of each context of three pages or more gets an id
+    outside the pool. Returns the batch and one without those pages, whose result is the same (no window, not causal)."""
+    nan = np.uint16(0x7FC0) if b.bf16 else np.float32(np.nan)
+    b = dataclasses.replace(b, kv_indices=b.kv_indices + 1)
+    rows = [(0, 2, 1, 3) if b.hnd else (0, 1, 2, 3)] * 2  # views with the token on axis 1
+    pools = []
+    for pool in (b.k_cache, b.v_cache):
+        grown = np.full((pool.shape[0] + 1,) + pool.shape[1:], nan, pool.dtype)
+        new, old = grown.transpose(rows[0]), pool.transpose(rows[0])
+        for s, n in enumerate(b.kv_lens):
+            for j in range(max(0, n - 1 - window) if window >= 0 else 0, n):
+                page = b.kv_indices[b.kv_indptr[s] + j // b.page_size]
+                new[page, j % b.page_size] = old[page - 1, j % b.page_size]
+        pools.append(grown)
+    b = dataclasses.replace(b, k_cache=pools[0], v_cache=pools[1])
+    if not bad_page:
+        return b, b
+    idx, keep, lens = b.kv_indices.copy(), np.ones(b.kv_indices.size, bool), list(b.kv_lens)
+    for s in range(b.batch):
+        if b.kv_indptr[s + 1] - b.kv_indptr[s] >= 3:
+            at = b.kv_indptr[s] + 1
+            idx[at], keep[at] = (-1, pools[0].shape[0])[s % 2], False
+            lens[s] -= b.page_size
+    indptr = np.concatenate([[0], np.cumsum(keep)])[b.kv_indptr].astype(np.int32)
+    without = dataclasses.replace(b, kv_indices=b.kv_indices[keep], kv_indptr=indptr, kv_lens=lens)
+    return dataclasses.replace(b, kv_indices=idx), without
+
+
+@pytest.mark.parametrize("hq,hkv,d,bf16", [(8, 2, 256, True), (32, 4, 128, True), (16, 1, 64, True), (8, 2, 256, False),
+                                           (4, 1, 64, False)])
+@pytest.mark.parametrize("ps,hnd,window,bad_page", [(16, False, -1, False), (12, False, -1, False), (64, True, 37, False),
+                                                    (12, True, 21, False), (16, False, -1, True), (5, False, -1, True)])
+def test_decode_reads_nothing_that_nobody_wrote(session, hq, hkv, d, bf16, ps, hnd, window, bad_page):
+    """Cache rows outside the visible keys hold whatever the pool's memory held: NaN here. A masked key's weight is 0, but 0
+    times NaN is NaN, so such rows must not enter the products."""
+    rng = np.random.default_rng(d + hq + ps)
+    b = cases.make_paged_batch(rng, EDGES + [2500], [1] * (len(EDGES) + 1), page_size=ps, hnd=hnd, hq=hq, hkv=hkv, d=d,
+                               bf16=bf16)
+    b, without = _unwritten_is_nan(b, window, bad_page)
+    got = run_case(session, b, causal=not bad_page, window_left=window)
+    ref = cases.values(cases.oracle_attention(without, not bad_page, window_left=window), bf16)
+    if bf16:
+        v = cases.values(b.v_cache, True)
+        cases.assert_attention_class(got, ref, float(np.nanmax(np.abs(v))), what="decode")
+    else:
+        cases.assert_close(got, ref, 1e-5, 1e-5, what="f32 decode")
