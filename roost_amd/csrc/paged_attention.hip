@@ -70,7 +70,7 @@ constexpr uint32_t kPfWideDim = 128;            // the head dim it is built for
 // 32 heads 1.45, 524 / 485; 8 ragged prompts to 4,000 1.45, 393 / 363; 6 chunks on prefixes 1.40, 408 / 384; 2 prompts
 // 1.40, 248 / 243; one prompt of 4,096 1.35, 154 / 162; one of 3,000 1.32, 103 / 108.
 constexpr double kPfWideTileCost = 1.39;
-constexpr uint32_t kPfMinSplitTiles = 8;        // a split piece covers at least this many 64-key tiles
+constexpr uint32_t kPfMinSplitTiles = 8;        // load balance cuts no piece below this many 64-key tiles
 constexpr uint32_t kAlign = 256;
 constexpr uint32_t kPlanMagic = 0x41504752;     // "RGPA"
 constexpr float kLog2e = 1.4426950408889634f;
@@ -113,8 +113,8 @@ struct DecodeMerge {
 };
 // A prefill work item: query tokens q0 .. q0 + rows - 1 of sequence seq (all kGroup query heads of one KV head)
 // against keys [kbeg, kend). slot >= 0 marks one piece of a split key range: it writes partials (its output divided
-// by its own sum, in bf16, and its fp32 running max and sum) that PrefillMergeKernel combines; slot -1 writes the final
-// rows.
+// by its own sum, in bf16 in the plan's first slots and in fp32 in the rest, and its fp32 running max and sum) that
+// PrefillMergeKernel combines; slot -1 writes the final rows.
 struct PrefillWork {
   int32_t seq;
   int32_t q0;
@@ -168,6 +168,7 @@ struct PlanRecord {
   // Single-token sequences of a prefill call run as decode: their pieces, ranges, merges and partials.
   uint64_t dec_items, dec_ranges, dec_merges, dec_splits;
   uint64_t dec_item_offset, dec_range_offset, dec_merge_offset, dec_float_offset;
+  uint64_t splits_bf16;  // prefill: the leading partial slots, whose rows are bf16
   uint32_t q_heads;      // the partials' row stride and, in a prefill, the items' heads
   uint32_t dtype;        // PlanDtype(params): the kernels the tables were made for
   uint64_t item_tokens;  // prefill: query tokens per work item (kPfTokens or kPfWideTokens)
@@ -179,6 +180,7 @@ struct Layout {
   uint64_t merges = 0;
   uint64_t merges_two = 0;  // prefill: leading merge entries of two pieces
   uint32_t item_tokens = kPfTokens;  // prefill: query tokens per work item
+  uint64_t splits_bf16 = 0;          // prefill: leading partial slots in bf16
   uint32_t overlap = 0;     // prefill: tile and decode kernels on two streams (ChooseOverlap)
   uint64_t range_offset = 0;
   uint64_t merge_offset = 0;
@@ -305,8 +307,9 @@ RoostStatus Admit(const RoostPagedAttentionParams& p, bool for_run) {
 // ---- Host planning ---------------------------------------------------------------------------------------------------
 
 // rows_per_split: partial rows one split slot holds (decode: the query heads of a sequence; prefill: kPfRows).
-Layout MakeLayout(uint64_t work_items, uint64_t ranges, uint64_t merges, uint64_t splits, uint32_t rows_per_split,
-                  uint32_t head_dim, uint32_t mode) {
+// splits_bf16: the prefill slots among them whose rows are bf16; the others are fp32.
+Layout MakeLayout(uint64_t work_items, uint64_t ranges, uint64_t merges, uint64_t splits, uint64_t splits_bf16,
+                  uint32_t rows_per_split, uint32_t head_dim, uint32_t mode) {
   Layout l;
   l.work_items = work_items;
   l.ranges = ranges;
@@ -319,9 +322,10 @@ Layout MakeLayout(uint64_t work_items, uint64_t ranges, uint64_t merges, uint64_
   l.merge_offset = roost::RoundUp(l.range_offset + (ranges > 0 ? (ranges + 1) * sizeof(int32_t) : 0), 16);
   l.int_bytes = l.merge_offset + merges * merge_bytes;
   l.float_offset = roost::RoundUp(l.int_bytes, kAlign);
-  // decode partials: fp32 rows then (max, sum); prefill partials: bf16 rows then (max, sum)
-  l.float_bytes = splits * rows_per_split *
-                  (decode ? (static_cast<uint64_t>(head_dim) + 2) * sizeof(float) : 2 * static_cast<uint64_t>(head_dim) + 8);
+  // fp32 rows (a prefill's bf16 ones before them), then (max, sum) pairs
+  l.splits_bf16 = splits_bf16;
+  l.float_bytes = rows_per_split * (splits * (static_cast<uint64_t>(head_dim) + 2) * sizeof(float) -
+                                    splits_bf16 * head_dim * sizeof(uint16_t));
   l.total = l.float_offset + l.float_bytes;
   return l;
 }
@@ -583,10 +587,12 @@ Layout PlanDecode(const RoostPagedAttentionParams& p, uint32_t cus, unsigned cha
 }
 
 // Prefill work items: one per (query tile, KV head) -- 64-token tiles when the page size is a multiple of 16 (the
-// DMA-fed kernel; 96-token ones at head dim 128 where that ends earlier), 32-token tiles otherwise. For the 64-token kernel the key range of an item longer than 3/4 of the
-// average load of a CU is cut into pieces of whole 64-key tiles (at least kPfMinSplitTiles each), so that the longest causal
-// tile does not set the makespan; the pieces write partials merged by PrefillMergeKernel. Items are ordered longest
-// first. The cuts depend on the whole batch, so the variant is deterministic but not batch invariant.
+// DMA-fed kernel; 96-token ones at head dim 128 where that ends earlier), 32-token tiles otherwise. The DMA-fed kernel's
+// key ranges are cut into pieces of whole 64-key tiles where they are longer than a share of the average load of a CU
+// (at least kPfMinSplitTiles each, so that the longest causal tile does not set the makespan), where CUs would stay idle
+// (SparsePieceTiles, down to 2 tiles) and beside decode ranges (ChooseOverlap); the pieces write partials merged by
+// PrefillMergeKernel. Items are ordered longest first. The cuts depend on the whole batch, so the variant is deterministic
+// but not batch invariant.
 bool PrefillFastPath(const RoostPagedAttentionParams& p) {
   return p.page_size % 16 == 0 && (p.page_size & (p.page_size - 1)) == 0;
 }
@@ -689,9 +695,12 @@ PieceChoice PrefillPieceTiles(const ItemList& items, uint32_t cus) {
 // Calls whose pieces do not fill the CUs once (a short prompt: 1,777 tokens x 2 KV heads made 128 pieces of up to 8
 // tiles for 256 CUs): pieces below kPfMinSplitTiles, down to 2 tiles, while they still run in one round. Each is priced by
 // what such calls measured: a tile on a chip with idle CUs 2.3 us at head dim 256, the merge launch 4.5 us, and 0.08 us
-// per piece for its partial rows written and merged (both sides less at smaller head dims). Fresh prompts at head dim
-// 256, 8 heads, pieces of at most 8 tiles against this choice: 500 tokens 34.6 -> 25.1 us, 1,000 41.7 -> 35.0, 1,777
-// 49.9 -> 43.4; 256 tokens on 4,000 cached ones 44.6 -> 35.2. 200 tokens stay whole: 21.1 against 23.0 us in pieces of 2.
+// per piece for its partial rows written and merged (both sides less at smaller head dims). Fresh prompts of 8 heads over 2,
+// pieces of at least 8 tiles against this choice (us): head dim 256, 500 tokens 38.6 -> 29.2, 1,000 45.4 -> 37.8, 1,777
+// 51.8 -> 47.1, 256 on 4,000 cached ones 48.1 -> 40.4; 128, 500 23.4 -> 17.4, 1,000 28.9 -> 21.6; 64, 500 17.0 -> 14.3,
+// 1,000 23.0 -> 16.4. 200 tokens stay whole: 23.9 / 13.1 / 10.2 at 256 / 128 / 64 against 27.3 / 16.3 / 13.2 in pieces of 2.
+// Over prompts of 100 to 1,777 tokens at the three head dims the choice was within 5% of the best of 2 to 8 tiles, but for
+// chunks of 100 on 300 at 64 (12%, left whole).
 constexpr double kSparseTileUs = 2.3;
 constexpr double kPieceMergeUs = 0.08;
 constexpr double kMergeLaunchUs = 4.5;
@@ -734,6 +743,7 @@ struct OverlapChoice {
   bool use = false;
   int64_t target = 0;    // piece size (tiles) of the tile kernel
   uint32_t dec_cus = 0;  // CUs the decode ranges are sized for
+  bool bf16 = true;      // the pieces' partials are bf16
 };
 
 constexpr double kTileUsD256 = 3.7;
@@ -780,7 +790,7 @@ OverlapChoice ChooseOverlap(const RoostPagedAttentionParams& p, const ItemList& 
 
 Layout PlanPrefill(const RoostPagedAttentionParams& p, uint32_t cus, unsigned char* host) {
   if (p.q.dtype == ROOST_DTYPE_F32) {  // no f32 MFMA tile kernel: every query token is a row of the f32 decode kernel
-    Layout l = MakeLayout(0, 0, 0, 0, kPfRows, p.head_dim, ROOST_ATTENTION_PREFILL);
+    Layout l = MakeLayout(0, 0, 0, 0, 0, kPfRows, p.head_dim, ROOST_ATTENTION_PREFILL);
     AppendDecode(p, BuildDecodeAllTokens(p, cus), l, host);
     PlaceFloats(p, 0, l);
     return l;
@@ -823,11 +833,12 @@ Layout PlanPrefill(const RoostPagedAttentionParams& p, uint32_t cus, unsigned ch
   };
   int64_t tile_q = fast ? kPfTokens : kPrefillTileQ;
   int64_t target = 0;
+  int64_t whole = 0;  // longest key range in tiles that load balance alone leaves whole
   OverlapChoice overlap;
   if (fast) {
     ItemList list = item_list(tile_q);
     const PieceChoice narrow = PrefillPieceTiles(list, cus);
-    target = narrow.target;
+    target = whole = narrow.target;
     overlap = ChooseOverlap(p, list, target, cus, single);
     if (overlap.use) {
       target = overlap.target;
@@ -853,18 +864,33 @@ Layout PlanPrefill(const RoostPagedAttentionParams& p, uint32_t cus, unsigned ch
                            kend - kbeg + 64});
     }
   });
+  // A bf16 partial row is one rounding more (2-norm error of a row against 64 bits: 0.0023 whole, 0.0029 merged from bf16,
+  // however many pieces). Items that load balance cuts anyway take it: their merge would read twice the bytes. An item that
+  // is cut only for idle CUs or under the wide form keeps fp32 partials: fresh prompts of 500 / 1,000 tokens (8 heads over 2,
+  // head dim 256) 26.7 / 34.9 us in bf16 pieces, 29.5 / 37.3 in fp32, 38.5 / 45.3 not cut so.
   std::vector<PrefillMerge> merges;
-  int32_t slot = 0;
+  uint64_t splits_bf16 = 0, splits = 0;
   if (fast) {
+    auto tiles_of = [](const Item& it) { return roost::CeilDiv(static_cast<int64_t>(it.w.kend - it.w.kbeg), 64); };
+    // (The 64-token items under a 96-token one are at most a tile shorter.)
+    auto bf16_partials = [&](const Item& it) {
+      return overlap.use ? overlap.bf16 : tiles_of(it) - (tile_q == kPfWideTokens ? 1 : 0) > whole;
+    };
+    for (const Item& it : items) {
+      const int64_t pieces = Pieces(tiles_of(it), target);
+      if (pieces > 1) (bf16_partials(it) ? splits_bf16 : splits) += static_cast<uint64_t>(pieces);
+    }
+    splits += splits_bf16;
+    auto slot16 = int32_t{0}, slot32 = static_cast<int32_t>(splits_bf16);
     std::vector<Item> cut;
     cut.reserve(items.size());
     for (const Item& it : items) {
-      const int64_t tiles = roost::CeilDiv(static_cast<int64_t>(it.w.kend - it.w.kbeg), 64);
-      const int64_t pieces = std::min<int64_t>(roost::CeilDiv(tiles, target), kMaxMergeSplits);
+      const int64_t tiles = tiles_of(it), pieces = Pieces(tiles, target);
       if (pieces <= 1) {
         cut.push_back(it);
         continue;
       }
+      int32_t& slot = bf16_partials(it) ? slot16 : slot32;
       merges.push_back(PrefillMerge{it.w.seq, it.w.q0, it.w.kv_head, it.w.rows, slot, static_cast<int32_t>(pieces), {0, 0}});
       for (int64_t i = 0; i < pieces; ++i) {
         const int64_t t0 = tiles * i / pieces, t1 = tiles * (i + 1) / pieces;
@@ -881,7 +907,7 @@ Layout PlanPrefill(const RoostPagedAttentionParams& p, uint32_t cus, unsigned ch
   std::stable_sort(items.begin(), items.end(), [](const Item& a, const Item& b) { return a.cost > b.cost; });
   // Merges of exactly two pieces first: they run on the 8-rows-per-block form of the merge kernel.
   std::stable_partition(merges.begin(), merges.end(), [](const PrefillMerge& m) { return m.count == 2; });
-  Layout l = MakeLayout(items.size(), 0, merges.size(), static_cast<uint64_t>(slot),
+  Layout l = MakeLayout(items.size(), 0, merges.size(), splits, splits_bf16,
                         static_cast<uint32_t>(tile_q) * kGroup, p.head_dim, ROOST_ATTENTION_PREFILL);
   l.item_tokens = fast ? static_cast<uint32_t>(tile_q) : kPfTokens;
   l.merges_two = static_cast<uint64_t>(
@@ -2050,6 +2076,12 @@ __device__ __forceinline__ u32x2_t LdsTr16(const unsigned char* base, uint32_t o
 template <int D>
 constexpr int kPfTileBytes = kPrefillTileK * 2 * D;  // one 64-key K or V tile in LDS
 
+// Row `prow` (counted over all slots of `rows` rows) of the fp32 partials, which follow the splits_bf16 slots of bf16 rows.
+__device__ __forceinline__ float* PartRowF32(uint16_t* part_o, uint32_t splits_bf16, uint64_t prow, uint32_t rows, int d) {
+  const uint64_t first = static_cast<uint64_t>(splits_bf16) * rows;
+  return reinterpret_cast<float*>(part_o + first * d) + (prow - first) * d;
+}
+
 // The tile kernel's work for item `item`; `tiles` is the caller's LDS, [2 buffers][K, V][kPfTileBytes<D>].
 template <int D, bool kCap, int kWaves>
 __device__ __forceinline__ void PrefillTileBody(const uint16_t* __restrict__ q, uint16_t* __restrict__ out,
@@ -2057,8 +2089,8 @@ __device__ __forceinline__ void PrefillTileBody(const uint16_t* __restrict__ q, 
                                                 const int32_t* __restrict__ kv_indices,
                                                 const int32_t* __restrict__ q_indptr,
                                                 const PrefillWork* __restrict__ work, uint16_t* __restrict__ part_o,
-                                                float* __restrict__ part_ml, uint32_t q_heads, uint32_t causal,
-                                                uint32_t ps_shift, float scale_log2, int32_t window, SoftCap cap,
+                                                float* __restrict__ part_ml, uint32_t splits_bf16, uint32_t q_heads,
+                                                uint32_t causal, uint32_t ps_shift, float scale_log2, int32_t window, SoftCap cap,
                                                 uint32_t item, unsigned char (*tiles)[2][kPfTileBytes<D>]) {
   static_assert(D == 64 || D == 128 || D == 256, "the tile kernel is built for head dims 64, 128 and 256");
   constexpr int kRowB = 2 * D;                  // bytes of one K or V row in LDS
@@ -2320,18 +2352,29 @@ __device__ __forceinline__ void PrefillTileBody(const uint16_t* __restrict__ q, 
   const float l_tot = SumXor32(l_run);
   if (!row_ok) return;
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-  if (wk.slot >= 0) {  // a piece of a split item: its normalised output in bf16 and its (max, sum)
+  if (wk.slot >= 0) {  // a piece of a split item: its normalised output and its (max, sum)
     const uint64_t prow = static_cast<uint64_t>(wk.slot) * kRows + static_cast<uint64_t>(r) * kGroup + hq;
-    uint16_t* po = part_o + prow * D;
+    if (static_cast<uint32_t>(wk.slot) < splits_bf16) {
+      uint16_t* po = part_o + prow * D;
 #pragma unroll
-    for (int dt = 0; dt < kDt; ++dt)
+      for (int dt = 0; dt < kDt; ++dt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = dt * 32 + i * 8 + hl * 4;
-        const u32x2_t v{PackRne(o[dt][i * 4] * inv, o[dt][i * 4 + 1] * inv),
-                        PackRne(o[dt][i * 4 + 2] * inv, o[dt][i * 4 + 3] * inv)};
-        *reinterpret_cast<u32x2_t*>(po + d) = v;
-      }
+        for (int i = 0; i < 4; ++i) {
+          const int d = dt * 32 + i * 8 + hl * 4;
+          const u32x2_t v{PackRne(o[dt][i * 4] * inv, o[dt][i * 4 + 1] * inv),
+                          PackRne(o[dt][i * 4 + 2] * inv, o[dt][i * 4 + 3] * inv)};
+          *reinterpret_cast<u32x2_t*>(po + d) = v;
+        }
+    } else {
+      float* po = PartRowF32(part_o, splits_bf16, prow, kRows, D);
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const f32x4_t v{o[dt][i * 4] * inv, o[dt][i * 4 + 1] * inv, o[dt][i * 4 + 2] * inv, o[dt][i * 4 + 3] * inv};
+          *reinterpret_cast<f32x4_t*>(po + dt * 32 + i * 8 + hl * 4) = v;
+        }
+    }
     if (hl == 0) {
       part_ml[2 * prow] = m_run;
       part_ml[2 * prow + 1] = l_tot;
@@ -2359,11 +2402,11 @@ __global__ void __launch_bounds__(64 * kWaves, 1)
     PrefillTileKernel(const uint16_t* __restrict__ q, uint16_t* __restrict__ out, float* __restrict__ lse, KvView kv,
                       const int32_t* __restrict__ kv_indices, const int32_t* __restrict__ q_indptr,
                       const PrefillWork* __restrict__ work, uint16_t* __restrict__ part_o, float* __restrict__ part_ml,
-                      uint32_t q_heads, uint32_t causal, uint32_t ps_shift, float scale_log2, int32_t window,
-                      SoftCap cap) {
+                      uint32_t splits_bf16, uint32_t q_heads, uint32_t causal, uint32_t ps_shift, float scale_log2,
+                      int32_t window, SoftCap cap) {
   __shared__ __attribute__((aligned(16))) unsigned char tiles[2][2][kPfTileBytes<D>];  // [buffer][K, V]
-  PrefillTileBody<D, kCap, kWaves>(q, out, lse, kv, kv_indices, q_indptr, work, part_o, part_ml, q_heads, causal,
-                                   ps_shift, scale_log2, window, cap, blockIdx.x, tiles);
+  PrefillTileBody<D, kCap, kWaves>(q, out, lse, kv, kv_indices, q_indptr, work, part_o, part_ml, splits_bf16, q_heads,
+                                   causal, ps_shift, scale_log2, window, cap, blockIdx.x, tiles);
 }
 
 // A mixed step's attention in one launch: workgroups [0, items) run the tile pieces, the rest the decode ranges with 8
@@ -2379,8 +2422,8 @@ __global__ void __launch_bounds__(512, 1)
     MixedAttentionKernel(const uint16_t* __restrict__ q, uint16_t* __restrict__ out, float* __restrict__ lse,
                          KvView kv, const int32_t* __restrict__ kv_indices, const int32_t* __restrict__ q_indptr,
                          const PrefillWork* __restrict__ work, uint16_t* __restrict__ part_o,
-                         float* __restrict__ part_ml, uint32_t q_heads, uint32_t causal, uint32_t ps_shift,
-                         float scale_log2, int32_t window, SoftCap raw_cap, uint32_t items,
+                         float* __restrict__ part_ml, uint32_t splits_bf16, uint32_t q_heads, uint32_t causal,
+                         uint32_t ps_shift, float scale_log2, int32_t window, SoftCap raw_cap, uint32_t items,
                          const DecodeWork* __restrict__ dec_work, const int32_t* __restrict__ dec_range_ptr,
                          float* __restrict__ dec_part_o, float* __restrict__ dec_part_ml, uint32_t heads_per_wg,
                          uint32_t dec_vheads, uint32_t dec_shift, SoftCap cap) {
@@ -2388,8 +2431,8 @@ __global__ void __launch_bounds__(512, 1)
   constexpr int kLds = kTileLds > kMixedDecodeLds<D, NH> ? kTileLds : kMixedDecodeLds<D, NH>;
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
   if (blockIdx.x < items) {
-    PrefillTileBody<D, kCap, 8>(q, out, lse, kv, kv_indices, q_indptr, work, part_o, part_ml, q_heads, causal, ps_shift,
-                                scale_log2, window, raw_cap, blockIdx.x,
+    PrefillTileBody<D, kCap, 8>(q, out, lse, kv, kv_indices, q_indptr, work, part_o, part_ml, splits_bf16, q_heads,
+                                causal, ps_shift, scale_log2, window, raw_cap, blockIdx.x,
                                 reinterpret_cast<unsigned char (*)[2][kPfTileBytes<D>]>(lds));
     return;
   }
@@ -2421,7 +2464,13 @@ __device__ __forceinline__ void MergeWrite(uint16_t* __restrict__ out, float* __
   if (lse != nullptr && d == 0) lse[token * q_heads + head] = l > 0.0f ? mx + log2f(l) : -INFINITY;
 }
 
-// acc += o * f for one piece's bf16 output slice (already divided by the piece's own sum).
+// acc += o * f for one piece's output slice (already divided by the piece's own sum), bf16 or fp32.
+__device__ __forceinline__ void MergeAdd(float4& acc, f32x4_t o, float f) {
+  acc.x = fmaf(o[0], f, acc.x);
+  acc.y = fmaf(o[1], f, acc.y);
+  acc.z = fmaf(o[2], f, acc.z);
+  acc.w = fmaf(o[3], f, acc.w);
+}
 __device__ __forceinline__ void MergeAdd(float4& acc, u32x2_t raw, float f) {
   acc.x = fmaf(__uint_as_float(raw[0] << 16), f, acc.x);
   acc.y = fmaf(__uint_as_float(raw[0] & 0xFFFF0000u), f, acc.y);
@@ -2429,12 +2478,14 @@ __device__ __forceinline__ void MergeAdd(float4& acc, u32x2_t raw, float f) {
   acc.w = fmaf(__uint_as_float(raw[1] & 0xFFFF0000u), f, acc.w);
 }
 
-template <int D, int kTokens, int kRows>
+// T: the type of the item's partial rows; part_o holds row 0 of slot 0 as if every slot were of that type.
+template <typename T, int D, int kTokens, int kRows>
 __device__ __forceinline__ void PrefillMergeRows(uint16_t* __restrict__ out, float* __restrict__ lse,
-                                                 const PrefillMerge& mg, int r0, const uint16_t* __restrict__ part_o,
+                                                 const PrefillMerge& mg, int r0, const T* __restrict__ part_o,
                                                  const float* __restrict__ part_ml,
                                                  const int32_t* __restrict__ q_indptr, uint32_t q_heads,
                                                  const void* gate) {
+  using Slice = std::conditional_t<sizeof(T) == 2, u32x2_t, f32x4_t>;  // four dims
   if (r0 >= mg.rows) return;
   const int hq = threadIdx.x / (D / 4);
   const int d = 4 * (threadIdx.x % (D / 4));
@@ -2446,7 +2497,8 @@ __device__ __forceinline__ void PrefillMergeRows(uint16_t* __restrict__ out, flo
   };
   if constexpr (kRows > 1) {  // merges of exactly two pieces
     float2 ml[kRows][2];
-    u32x2_t o[kRows][2], gw[kRows];
+    Slice o[kRows][2];
+    u32x2_t gw[kRows];
 #pragma unroll
     for (int j = 0; j < kRows; ++j) {
       const int r = min(r0 + j, mg.rows - 1);  // rows past the item's end re-read its last row and are not written
@@ -2454,7 +2506,7 @@ __device__ __forceinline__ void PrefillMergeRows(uint16_t* __restrict__ out, flo
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         ml[j][i] = *reinterpret_cast<const float2*>(part_ml + 2 * prow(i, r));
-        o[j][i] = *reinterpret_cast<const u32x2_t*>(part_o + prow(i, r) * D + d);
+        o[j][i] = *reinterpret_cast<const Slice*>(part_o + prow(i, r) * D + d);
       }
     }
 #pragma unroll
@@ -2488,7 +2540,7 @@ __device__ __forceinline__ void PrefillMergeRows(uint16_t* __restrict__ out, flo
         const float2 m = *reinterpret_cast<const float2*>(part_ml + 2 * prow(i, r0));
         const float f = m.y * exp2f(m.x - mx);
         l += f;
-        MergeAdd(acc, *reinterpret_cast<const u32x2_t*>(part_o + prow(i, r0) * D + d), f);
+        MergeAdd(acc, *reinterpret_cast<const Slice*>(part_o + prow(i, r0) * D + d), f);
       }
     }
     MergeWrite<D>(out, lse, gate, gw, tok0 + r0, q_heads, head, d, acc, l, mx);
@@ -2502,6 +2554,7 @@ struct PrefillMergeArgs {
   const uint16_t* part_o;
   const float* part_ml;
   const int32_t* q_indptr;
+  uint32_t splits_bf16;
   uint32_t two;     // merges of exactly two pieces, listed first
   uint32_t blocks;  // blocks of the launch's prefill share
 };
@@ -2511,19 +2564,23 @@ __device__ __forceinline__ void PrefillMergeBody(uint16_t* __restrict__ out, flo
                                                  const PrefillMergeArgs& m, uint32_t q_heads, const void* gate,
                                                  uint32_t b) {
   constexpr uint32_t kTwoBlocks = kTokens / kPfMergeRows;  // blocks per two-piece merge
-  const PrefillMerge* __restrict__ merges = m.merges;
-  const uint16_t* __restrict__ part_o = m.part_o;
-  const float* __restrict__ part_ml = m.part_ml;
-  const int32_t* __restrict__ q_indptr = m.q_indptr;
   const uint32_t two = m.two;
-  if (b < two * kTwoBlocks) {
-    PrefillMergeRows<D, kTokens, kPfMergeRows>(out, lse, merges[b / kTwoBlocks],
-                                               static_cast<int>(b % kTwoBlocks) * kPfMergeRows, part_o, part_ml,
-                                               q_indptr, q_heads, gate);
-  } else {
-    const uint32_t k = b - two * kTwoBlocks;
-    PrefillMergeRows<D, kTokens, 1>(out, lse, merges[two + k / kTokens], static_cast<int>(k % kTokens), part_o, part_ml,
-                                    q_indptr, q_heads, gate);
+  const bool pair = b < two * kTwoBlocks;
+  const uint32_t k = b - two * kTwoBlocks;
+  const PrefillMerge mg = m.merges[pair ? b / kTwoBlocks : two + k / kTokens];
+  const int r0 = pair ? static_cast<int>(b % kTwoBlocks) * kPfMergeRows : static_cast<int>(k % kTokens);
+  auto rows = [&](auto n, const auto* part_o, int first) {
+    using T = std::remove_cv_t<std::remove_pointer_t<decltype(part_o)>>;
+    PrefillMergeRows<T, D, kTokens, decltype(n)::value>(out, lse, mg, first, part_o, m.part_ml, m.q_indptr, q_heads, gate);
+  };
+  if (static_cast<uint32_t>(mg.first) < m.splits_bf16) {
+    pair ? rows(std::integral_constant<int, kPfMergeRows>{}, m.part_o, r0)
+         : rows(std::integral_constant<int, 1>{}, m.part_o, r0);
+  } else {  // fp32 rows: half as many at a time, for the same registers
+    const float* part_f = reinterpret_cast<const float*>(m.part_o) -
+                          static_cast<uint64_t>(m.splits_bf16) * kTokens * kGroup * (D / 2);
+    if (!pair) rows(std::integral_constant<int, 1>{}, part_f, r0);
+    for (int h = 0; pair && h < 2; ++h) rows(std::integral_constant<int, kPfMergeRows / 2>{}, part_f, r0 + h * kPfMergeRows / 2);
   }
 }
 
@@ -2613,12 +2670,14 @@ RoostStatus LaunchDecode(const RoostPagedAttentionParams& p, const PlanRecord& r
   return LaunchDecodeMerge<T, D>(p, rec, dev, kv, stream);
 }
 
-// Partials of the tile pieces: bf16 rows of the pieces' normalised outputs, then their fp32 (max, sum) pairs.
+// Partials of the tile pieces: rows of the pieces' normalised outputs, first the bf16 slots, then the fp32 ones, then their
+// fp32 (max, sum) pairs.
 uint16_t* PrefillPartO(const RoostPagedAttentionParams& p, const PlanRecord& rec, unsigned char* dev) {
   return reinterpret_cast<uint16_t*>(dev + rec.float_offset);
 }
 float* PrefillPartMl(const RoostPagedAttentionParams& p, const PlanRecord& rec, unsigned char* dev) {
-  return reinterpret_cast<float*>(PrefillPartO(p, rec, dev) + rec.splits * rec.item_tokens * kGroup * p.head_dim);
+  return reinterpret_cast<float*>(PrefillPartO(p, rec, dev) +
+                                  (2 * rec.splits - rec.splits_bf16) * rec.item_tokens * kGroup * p.head_dim);
 }
 
 PrefillMergeArgs PrefillMergeArgsOf(const RoostPagedAttentionParams& p, const PlanRecord& rec, unsigned char* dev) {
@@ -2627,6 +2686,7 @@ PrefillMergeArgs PrefillMergeArgsOf(const RoostPagedAttentionParams& p, const Pl
   m.part_o = PrefillPartO(p, rec, dev);
   m.part_ml = PrefillPartMl(p, rec, dev);
   m.q_indptr = static_cast<const int32_t*>(p.q_indptr.address);
+  m.splits_bf16 = static_cast<uint32_t>(rec.splits_bf16);
   m.two = static_cast<uint32_t>(rec.merges_two);
   const auto tokens = static_cast<uint32_t>(rec.item_tokens);
   m.blocks = m.two * (tokens / kPfMergeRows) + (static_cast<uint32_t>(rec.merges) - m.two) * tokens;
@@ -2671,8 +2731,8 @@ RoostStatus LaunchMixed(const RoostPagedAttentionParams& p, const PlanRecord& re
   auto* dec_ml = dec_o + rec.dec_splits * p.q_heads * p.head_dim;
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, q16, outp, lsep, kv, kv.kv_indices, q_indptr, items,
-                       PrefillPartO(p, rec, dev), PrefillPartMl(p, rec, dev), p.q_heads, p.causal, ps_shift,
-                       scale_log2, WindowOf(p), raw, n_items, dec_items, dec_ranges, dec_o, dec_ml, hpw, dkv.vheads,
+                       PrefillPartO(p, rec, dev), PrefillPartMl(p, rec, dev), static_cast<uint32_t>(rec.splits_bf16),
+                       p.q_heads, p.causal, ps_shift, scale_log2, WindowOf(p), raw, n_items, dec_items, dec_ranges, dec_o, dec_ml, hpw, dkv.vheads,
                        dkv.head_shift, cap);
   };
   auto of_group = [&](auto d, auto capped_c) {
@@ -2716,8 +2776,9 @@ RoostStatus LaunchPrefill(const RoostPagedAttentionParams& p, const PlanRecord& 
     const SoftCap raw{cap.capl / scale_log2, cap.k * scale_log2};
     const bool capped = cap.capl != 0.0f;
     auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, grid, dim3(static_cast<uint32_t>(8 * rec.item_tokens)), 0, stream, q16, outp, lsep, kv, kv.kv_indices,
-                         q_indptr, items, part_o, part_ml, p.q_heads, p.causal, ps_shift, scale_log2, WindowOf(p), raw);
+      hipLaunchKernelGGL(kernel, grid, dim3(static_cast<uint32_t>(8 * rec.item_tokens)), 0, stream, q16, outp, lsep, kv,
+                         kv.kv_indices, q_indptr, items, part_o, part_ml, static_cast<uint32_t>(rec.splits_bf16), p.q_heads,
+                         p.causal, ps_shift, scale_log2, WindowOf(p), raw);
     };
     const bool wide = rec.item_tokens == kPfWideTokens;
     if (p.head_dim == 64) {
@@ -2765,6 +2826,7 @@ PlanRecord MakeRecord(const RoostPagedAttentionParams& p, const Layout& l) {
   r.window = WindowOf(p);
   r.merges_two = static_cast<uint32_t>(l.merges_two);
   r.item_tokens = l.item_tokens;
+  r.splits_bf16 = l.splits_bf16;
   r.q_heads = p.q_heads;
   r.dtype = PlanDtype(p);
   r.overlap = l.overlap;

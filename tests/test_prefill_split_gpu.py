@@ -50,3 +50,38 @@ def test_short_prompts_in_small_pieces(session, hq, hkv, d, new, pre):
     got, items, merges, tokens = _run(session, b, ("sparse", d, sum(new)))
     assert tokens == 64 and (merges > 0 or d < 256 or len(new) > 1) and items <= 256
     cases.assert_close(got, torch_reference(b), what="short prompt vs fp32 torch")
+
+
+def _near_ties(b, rng):
+    """Queries of zeros, so that a row is the plain mean of the V rows it sees, and V one of two neighbouring bf16 values,
+    1 and 1 + 2^-7, with another share of each in every dim. The means, in units of 2^-7 above 1."""
+    share = rng.uniform(0.3, 0.7, (b.hkv, b.d))
+    upper = rng.random(b.v_cache.shape) < share
+    pages = [b.kv_indices[b.kv_indptr[s]:b.kv_indptr[s + 1]] for s in range(b.batch)]
+    rows = [upper[p].reshape(-1, b.hkv, b.d)[:n] for p, n in zip(pages, b.kv_lens)]
+    means = [np.cumsum(r, 0)[n - m:] / np.arange(n - m + 1, n + 1)[:, None, None]
+             for r, n, m in zip(rows, b.kv_lens, b.q_lens)]
+    b = dataclasses.replace(b, q=np.zeros_like(b.q), v_cache=np.where(upper, 0x3F81, 0x3F80).astype(np.uint16))
+    return b, np.repeat(np.concatenate(means), b.hq // b.hkv, axis=1)
+
+
+def _check_single_rounding(got, mean, rows):
+    """The weights are exactly 1 and every sum is exact in fp32, so a row rounded once is the mean's neighbour, but for the
+    last place of the division and of the merge (2^-18 of a unit here); a piece's mean rounded to bf16 first would land on
+    the other neighbour in a few dims of a hundred."""
+    sure = rows[:, None, None] & (np.abs(mean - 0.5) > 1e-3)
+    want = 1.0 + np.where(mean > 0.5, 2.0 ** -7, 0.0)
+    wrong = sure & (got != want)
+    assert sure.mean() > 0.1 and not wrong.any(), f"{wrong.sum()} of {sure.sum()} elements were rounded more than once"
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 256), (8, 2, 128), (4, 1, 64)])
+@pytest.mark.parametrize("new,pre", [([500], [0]), ([1025], [0]), ([129, 450, 300], [40, 0, 33])])
+def test_items_cut_for_idle_cus_keep_fp32(session, hq, hkv, d, new, pre):
+    """A prompt cut into small pieces because CUs would idle is as precise as a whole one."""
+    rng = np.random.default_rng(sum(new) + d)
+    b, mean = _near_ties(cases.make_paged_batch(rng, [a + p for a, p in zip(new, pre)], new, hq=hq, hkv=hkv, d=d), rng)
+    got, _, merges, _ = _run(session, b, ("ties", d, sum(new)))
+    assert merges > 0
+    pos = np.concatenate([p + np.arange(a) for a, p in zip(new, pre)])
+    _check_single_rounding(got, mean, pos < 512 - 64)  # items of up to 8 tiles
