@@ -2252,10 +2252,12 @@ __device__ __forceinline__ void PrefillTileBody(const uint16_t* __restrict__ q, 
     const unsigned char* vl = vtile + 8 * ln;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
-      // Keys after every query of the wavefront (uniform): nothing to add. Four prompts around 3,800 tokens at head dim
-      // 128: 546 -> 534 us. At head dim 256 the branch costs more registers than it saves work (8 ragged chunks on
-      // prefixes: 357 -> 365 us).
-      if (D <= 128 && causal && kb + 32 * half > last_pos) break;
+      // Keys after every query of the wavefront (uniform): nothing to add. Only the second half is left out: a test of the
+      // first as well costs every tile more than it saves (chunks of 512 on 8,000 cached tokens, us, none / both / second:
+      // 16 heads over 4 x 64 132 / 138 / 130, 32 over 8 x 128 330 / 334 / 326; four fresh prompts of 1,500 and 3,900 at 64
+      // 48.0 / 46.4 / 46.2 and 173 / 175 / 170, of 3,900 at 128 530 / 527 / 522). At head dim 256 the branch costs more
+      // registers than it saves work (8 ragged chunks on prefixes: 357 -> 365 us).
+      if (D <= 128 && half == 1 && causal && kb + 32 > last_pos) break;
       f32x16_t sc;
 #pragma unroll
       for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
