@@ -734,11 +734,19 @@ int64_t SparsePieceTiles(const ItemList& items, int64_t target, uint32_t head_di
 // wavefronts per SIMD and 128 KB of LDS), so the two kinds cannot share CUs; but when the tile items are cut into fewer,
 // longer pieces they hold only as many CUs as there are pieces, and decode ranges sized for the remaining CUs stream
 // K/V on those, both in one launch (MixedAttentionKernel). ChooseOverlap estimates both schedules with rates measured
-// on the MI355X -- a 64-key tile at head dim 256 takes ~3.7 us of a CU (less at smaller head dims), the decode stream
-// reaches 5.6 TB/s on 256 CUs and falls off as (CUs / 256)^0.26 (5.2 TB/s on 192), and the merged launch costs ~3 us
-// more than its longer side -- and keeps the cheaper. Config 5 (48 decode rows over 831 MB of K/V, two 512-token
-// chunks): 64 pieces beside decode ranges for the other 191 CUs. The decode side needs page sizes that are multiples
-// of 16 (its fast-page form).
+// on the MI355X -- a 64-key tile at head dim 256 takes ~3.7 us of a CU (less at smaller head dims), the decode stream as
+// below, and the merged launch costs ~3 us more than its longer side -- and keeps the cheaper. Config 5 (48 decode rows
+// over 831 MB of K/V, two 512-token chunks): 64 pieces beside decode ranges for the other 191 CUs. The decode side needs
+// page sizes that are multiples of 16 (its fast-page form).
+// The decode stream with groups of 8 and more query heads: 28 KB a us and CU up to 5.6 TB/s, 4 us for every piece a CU
+// takes in turn (an epilogue of up to 16 heads); 16 us for the further launches of the two schedules one after the other;
+// 2 us for the merge of the pieces and 0.01 (bf16) or 0.04 us (fp32) for each at head dim 256. Fitted to 140 mixed calls of
+// such groups (1 to 128 rows of 4 to 16,384 keys, 1 to 3 chunks, head dims 64 to 256): the choice is 1% above the best of 1
+// to 16 cuts on average and 17% at worst. Priced as groups of 4 are, it was 11% and 3.4 times: 2 rows of 9,577 keys beside
+// a chunk of 190 on 1,769, 32 heads over 2 x 256, 141 us (53 now).
+// With groups of 4: 5.6 TB/s on 256 CUs, falling off as (CUs / 256)^0.26 (5.2 TB/s on 192, but with few CUs 64 reach 2.5
+// TB/s and not 3.9). On 60 such calls the choice is 8% above the best on average and 65% at worst; where it goes wrong, too
+// few CUs are left for the decode ranges.
 struct OverlapChoice {
   bool use = false;
   int64_t target = 0;    // piece size (tiles) of the tile kernel
@@ -753,36 +761,59 @@ double TileUs(uint32_t head_dim) { return kTileUsD256 * (0.25 + 0.75 * head_dim 
 double DecodeUs(double bytes, uint32_t cus_used, uint32_t cus) {
   return bytes / (kDecodeBytesPerUs * std::pow(static_cast<double>(cus_used) / cus, 0.26));
 }
+constexpr double kBigGroupCuBytesPerUs = 28e3;
+constexpr double kBigGroupPieceUs = 4.0;
+constexpr double kBigGroupSerialUs = 16.0;
+constexpr double kBigGroupMergeUs = 2.0;
+constexpr double kBigGroupMergeBf16Us = 0.01, kBigGroupMergeF32Us = 0.04;
 
 template <typename Single>
 OverlapChoice ChooseOverlap(const RoostPagedAttentionParams& p, const ItemList& items, int64_t serial_target, uint32_t cus,
                             Single single) {
   OverlapChoice best;
   double dec_bytes = 0.0;
+  uint64_t rows = 0;
   for (uint32_t b = 0; b < p.batch; ++b) {
-    if (single(b)) dec_bytes += static_cast<double>(KvLenHost(p, b)) * DecodeHeads(p) * p.head_dim * 2.0 * 2.0;
+    if (!single(b)) continue;
+    ++rows;
+    dec_bytes += static_cast<double>(KvLenHost(p, b)) * DecodeHeads(p) * p.head_dim * 2.0 * 2.0;
   }
+  const bool big = DecodeGroupOf(p) > kGroup;
+  const double blocks = static_cast<double>(rows) * (DecodeHeads(p) / HeadsPerWorkgroup(p));
+  auto stream_us = [&](uint32_t n) {
+    return big ? dec_bytes / std::min(kDecodeBytesPerUs, n * kBigGroupCuBytesPerUs) : DecodeUs(dec_bytes, n, cus);
+  };
   if (dec_bytes == 0.0 || items.tiles.empty() || cus < 2 || p.page_size % 16 != 0) return best;
   const int64_t longest = items.longest();
   const double tile_us = TileUs(p.head_dim);
-  double best_us = PrefillMakespan(items, serial_target, cus) * tile_us + DecodeUs(dec_bytes, cus, cus);
+  double best_us = PrefillMakespan(items, serial_target, cus) * tile_us + stream_us(cus) + (big ? kBigGroupSerialUs : 0.0);
   for (int64_t k = 1; k <= 16; ++k) {
     const int64_t target = std::max<int64_t>(1, roost::CeilDiv(longest, k));
-    int64_t pieces = 0, piece_max = 0;
+    int64_t pieces = 0, merged = 0, piece_max = 0;
     for (const int64_t tiles : items.tiles) {
       const int64_t n = Pieces(tiles, target);
       pieces += n * items.heads;
+      if (n > 1) merged += n * items.heads;
       piece_max = std::max<int64_t>(piece_max, roost::CeilDiv(tiles, n));
     }
     if (pieces >= static_cast<int64_t>(cus)) break;
     const uint32_t left = cus - static_cast<uint32_t>(pieces);
-    const double us = std::max(static_cast<double>(piece_max + kPfPieceCost) * tile_us, DecodeUs(dec_bytes, left, cus)) +
-                      kMixedLaunchUs;
+    const double pieces_us = static_cast<double>(piece_max + kPfPieceCost) * tile_us;
+    const double decode_us = stream_us(left) + (big ? kBigGroupPieceUs * blocks / left : 0.0);
+    // The decode ranges of larger groups end early, and items are cut to end with them. Where the ranges take any share of
+    // the time, such an item might as well run whole: its pieces keep fp32 partials (2 to 12% of a small call). In calls
+    // that the pieces alone decide, every schedule cuts the items, and they stay in bf16.
+    const bool bf16 = !big || 4 * stream_us(left) < pieces_us;
+    double us = std::max(pieces_us, decode_us) + kMixedLaunchUs;
+    if (big && merged > 0) {
+      us += kBigGroupMergeUs + (bf16 ? kBigGroupMergeBf16Us : kBigGroupMergeF32Us) * merged * p.head_dim / 256.0;
+    }
     if (us < best_us) {
       best_us = us;
       best.use = true;
       best.target = target;
       best.dec_cus = left;
+      best.bf16 = bf16;
     }
   }
   return best;
@@ -921,7 +952,11 @@ Layout PlanPrefill(const RoostPagedAttentionParams& p, uint32_t cus, unsigned ch
   l.overlap = overlap.use ? 1u : 0u;
   // Side by side, a decode workgroup has 8 wavefronts and a CU to itself: ranges for dec_cus / 2 CUs at
   // kDecodeWgsPerCu 4-wavefront workgroups each are one range per free CU.
-  AppendDecode(p, BuildDecode(p, overlap.use ? std::max(1u, overlap.dec_cus / kDecodeWgsPerCu) : cus, !overlap.use, single),
+  // With groups of 4 the even deal is kept there: cut row by row, calls of few rows took up to 12% longer. Larger groups,
+  // whose pieces end in longer epilogues, gain (by 7% on average, 4% at most lost; 109 rows of 141 keys beside a prompt of
+  // 68, 32 heads over 2 x 128: 20.9 -> 11.4 us).
+  AppendDecode(p, BuildDecode(p, overlap.use ? std::max(1u, overlap.dec_cus / kDecodeWgsPerCu) : cus,
+                              !overlap.use || DecodeGroupOf(p) > kGroup, single),
                l, host);
   PlaceFloats(p, prefill_floats, l);
   return l;

@@ -14,13 +14,17 @@ from test_attention_gpu import Dev, torch_reference
 pytestmark = pytest.mark.gpu
 
 
+def _words(session, key):
+    ws = session._ws[(session.lib.entry(roost_amd.ATTENTION_VARIANT).variant_id, key)][3]
+    return np.frombuffer(C.string_at(ws.plan, ws.plan_bytes), np.uint64)
+
+
 def _run(session, b, key, **kw):
     """The result and, from the plan record: work items, merges, and its last word, the query tokens per item."""
     dev = Dev(b, **kw)
     entry = session.lib.entry(roost_amd.ATTENTION_VARIANT)
     session.launch(entry, dev.params(), key=key)
-    ws = session._ws[(entry.variant_id, key)][3]
-    words = np.frombuffer(C.string_at(ws.plan, ws.plan_bytes), np.uint64)
+    words = _words(session, key)
     got = dev.result()
     assert not np.isnan(got).any()
     return got, int(words[7]), int(words[9]), int(words[-1])
@@ -85,3 +89,34 @@ def test_items_cut_for_idle_cus_keep_fp32(session, hq, hkv, d, new, pre):
     assert merges > 0
     pos = np.concatenate([p + np.arange(a) for a, p in zip(new, pre)])
     _check_single_rounding(got, mean, pos < 512 - 64)  # items of up to 8 tiles
+
+
+@pytest.mark.parametrize("hq,hkv,d,rows,kv,new,pre", [
+    (16, 2, 256, 16, 5300, 535, 143), (32, 2, 128, 81, 5800, 117, 5350), (32, 2, 256, 7, 5800, 200, 264),
+    (16, 1, 64, 64, 3000, 300, 700)], ids=["g8 d256", "g16 d128", "g16 d256", "g16 d64"])
+def test_items_cut_beside_decode_ranges_keep_fp32(session, hq, hkv, d, rows, kv, new, pre):
+    """Groups of 8 and more query heads: decode ranges that take a good part of a mixed step's one launch leave a prompt's
+    items as precise as whole ones."""
+    rng = np.random.default_rng(hq + d)
+    lens = [kv - 37 * i % 1000 for i in range(rows)] + [new + pre]
+    b, mean = _near_ties(cases.make_paged_batch(rng, lens, [1] * rows + [new], hq=hq, hkv=hkv, d=d), rng)
+    key = ("mixed ties", d, hq)
+    got, _, merges, _ = _run(session, b, key)
+    assert int(_words(session, key)[5]) & 0xFFFFFFFF == 1 and merges > 0, "the plan did not cut the items of one launch"
+    _check_single_rounding(got, mean, np.ones(rows + new, bool))
+
+
+@pytest.mark.parametrize("hq,hkv,d,rows,kv,new,pre", [(32, 2, 256, 2, 9577, [190], 1769), (16, 2, 256, 24, 4350, [512], 4088),
+                                                      (32, 2, 256, 89, 190, [123] * 3, 1100)])
+def test_mixed_step_leaves_the_decode_ranges_enough_cus(session, hq, hkv, d, rows, kv, new, pre):
+    """Groups of 8 and more query heads: a range's CU streams about 28 KB a microsecond, so with the pieces on most CUs the
+    few that are left would take longer than both parts one after the other."""
+    rng = np.random.default_rng(hq + rows)
+    b = cases.make_paged_batch(rng, [kv] * rows + [n + pre for n in new], [1] * rows + new, hq=hq, hkv=hkv, d=d, std=0.5)
+    key = ("mixed cus", hq, rows)
+    got, items, _, _ = _run(session, b, key)
+    cases.assert_close(got, torch_reference(b), what="mixed step vs fp32 torch")
+    if int(_words(session, key)[5]) & 0xFFFFFFFF:
+        tile_us, k_us = 3.7, rows * kv * (hq // min(hq // hkv, 16)) * d * 4 / 28e3
+        longest = -(-(max(new) + pre) // 64)
+        assert k_us / (256 - items) < k_us / 200 + longest * tile_us, f"{items} of 256 CUs hold pieces"
