@@ -404,6 +404,8 @@ struct DecodeDeal {
 // even deal (with the merge kernel below on both sides): one context of 1,500 13.5 -> 10.7 us, of 16,000 41 -> 18.6; three
 // around 2,500 22.4 -> 12.4; 8 around 2,000 21.6 -> 14.1; 17 of 67 9.2 -> 7.0.
 constexpr double kDecodeBytesPerUs = 5.6e6;  // the decode stream on the whole chip
+constexpr double kLoneBytesPerUs = 4.0e6;    // of a long stream with at most one workgroup on a CU
+constexpr double kLoneBytes = 200e6;
 constexpr double kStepUs = 1.17;       // a 16-token group of a wavefront
 constexpr double kMergeUs = 4.0;       // the merge launch
 constexpr double kMergePieceUs = 0.05;
@@ -415,9 +417,17 @@ DecodeDeal ChooseDeal(const RoostPagedAttentionParams& p, uint32_t cus, const st
   const uint32_t heads = DecodeHeads(p), most = HeadsPerWorkgroup(p);
   const uint64_t slots = static_cast<uint64_t>(cus) * kDecodeWgsPerCu;
   const double group_us = 16.0 * p.head_dim * 2 * (p.q.dtype == ROOST_DTYPE_F32 ? 4 : 2) / kDecodeBytesPerUs;
+  // A long stream (from about 200 MB) with at most one workgroup per CU stays below kLoneBytesPerUs: 17 contexts of 6,960,
+  // 8 heads over 2 x 256, took 65.5 us in 255 workgroups, 54 in the even deal's 493. With a second one on a few CUs those end
+  // last, as if all had two, where the pieces are about equal: 44 of 1,024, 32 over 8 x 128, 47.7 us in 352 workgroups, 41.2
+  // in 474; but 82 of 7 to 116 11.7 us in 328 and 15.1 in 164.
+  const double bytes = static_cast<double>(total) * heads * group_us * kDecodeBytesPerUs;
+  const double lone_us = bytes > kLoneBytes ? bytes / kLoneBytesPerUs : 0.0;
   auto cost = [&](uint64_t workgroups, uint32_t hpw, uint64_t piece, uint64_t pieces) {
     const double steps = static_cast<double>(roost::CeilDiv(piece, 4 / hpw));
-    return steps * std::max(kStepUs, static_cast<double>(workgroups) * 4 * group_us) +
+    const bool lopsided = workgroups > cus && 2 * workgroups <= 3 * cus && 4 * workgroups * piece <= 5 * total * (heads / hpw);
+    const double streams = static_cast<double>(lopsided ? 2 * cus : workgroups);
+    return std::max(steps * std::max(kStepUs, streams * 4 * group_us), workgroups <= cus ? lone_us : 0.0) +
            (pieces > 1 ? kMergeUs + kMergePieceUs * pieces : 0.0);
   };
   DecodeDeal best;

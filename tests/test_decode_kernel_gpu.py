@@ -10,7 +10,7 @@ import pytest
 
 import cases
 import roost_amd
-from test_attention_gpu import Dev, _plan_overlap, from_dev, run_case, to_dev, torch_reference
+from test_attention_gpu import Dev, _plan_overlap, from_dev, run_case, to_dev, torch, torch_reference
 
 pytestmark = pytest.mark.gpu
 
@@ -145,3 +145,26 @@ def test_decode_reads_nothing_that_nobody_wrote(session, hq, hkv, d, bf16, ps, h
         cases.assert_attention_class(got, ref, float(np.nanmax(np.abs(v))), what="decode")
     else:
         cases.assert_close(got, ref, 1e-5, 1e-5, what="f32 decode")
+
+
+@pytest.mark.parametrize("kv_lens,hq,hkv,d,by_row", [
+    ([1500], 8, 2, 256, True), ([2400, 2500, 2600], 8, 2, 256, True), ([3000] * 10, 8, 2, 256, True),
+    ([9000], 32, 8, 128, True), ([512 + 120 * i for i in range(64)], 8, 2, 256, False), ([6960] * 17, 8, 2, 256, False),
+    ([15107] * 7, 8, 2, 256, None), ([1025] * 44, 32, 8, 128, None)],
+                         ids=lambda k: f"{len(k)}x{max(k)}" if isinstance(k, list) else None)
+def test_decode_deal(session, kv_lens, hq, hkv, d, by_row):
+    """Few rows are cut row by row, with fewer KV heads per workgroup; calls that fill the chip are dealt out evenly; a long
+    stream (200 MB) takes more than one workgroup per CU; and no call leaves a second workgroup on a few CUs only."""
+    rng = np.random.default_rng(len(kv_lens))
+    b = cases.make_paged_batch(rng, kv_lens, [1] * len(kv_lens), hq=hq, hkv=hkv, d=d)
+    dev = Dev(b)
+    ws = session.prepare(session.lib.entry(roost_amd.ATTENTION_VARIANT), dev.params(), ("deal", d, len(kv_lens)))
+    words = np.frombuffer(C.string_at(ws.plan, ws.plan_bytes), np.uint64)
+    heads_per_wg, ranges = int(words[5]) >> 32, int(words[8])
+    workgroups = ranges * hkv // heads_per_wg  # 4 query heads per KV head: a wavefront serves one KV head
+    cus = torch().cuda.get_device_properties(0).multi_processor_count
+    assert not cus < workgroups <= cus * 3 // 2, f"{workgroups} workgroups on {cus} CUs"
+    if by_row is not None:
+        most = 2 if d == 256 else 4  # the even deal's
+        assert (heads_per_wg < most) == by_row, (heads_per_wg, ranges)
+    assert sum(kv_lens) * hkv * d * 4 < 200e6 or workgroups > cus, f"{workgroups} workgroups on {cus} CUs"
