@@ -61,15 +61,17 @@ constexpr uint32_t kPfTokens = 64;              // query tokens per workgroup of
 constexpr uint32_t kPfRows = kPfTokens * kGroup;  // query rows (token, head) of one such workgroup
 // The 12-wavefront form of the tile kernel: 96 query tokens, so that each SIMD holds three wavefronts (153 of 168
 // registers, no spills) and one's softmax has two others' multiplies to run beside, and each K/V tile is copied for
-// half as many more queries. Four prompts around 3,800 tokens x 32 heads over 8, head dim 128: 524 -> 485 us (1,013
-// against 872 TFLOP/s). Head dim 64 is slower with it (83 -> 90 us); head dim 256 does not fit three wavefronts.
+// half as many more queries. Four prompts around 3,800 tokens x 32 heads over 8, head dim 128: 533 -> 492 us. Head dim 64 is
+// slower with it (83 -> 90 us); head dim 256 does not fit three wavefronts.
 constexpr uint32_t kPfWideTokens = 96;
 constexpr uint32_t kPfWideDim = 128;            // the head dim it is built for
-// A 96-token tile's time over a 64-token one's: plan() takes the 12-wavefront form when its dispatch ends that much
-// earlier in tiles. Ratios of the two dispatches and times (8 wavefronts, 12; us; head dim 128): 4 prompts around 3,800 x
-// 32 heads 1.45, 524 / 485; 8 ragged prompts to 4,000 1.45, 393 / 363; 6 chunks on prefixes 1.40, 408 / 384; 2 prompts
-// 1.40, 248 / 243; one prompt of 4,096 1.35, 154 / 162; one of 3,000 1.32, 103 / 108.
+// A 96-token tile's time over a 64-token one's, and what a piece of a cut item adds (partial rows, merge) in 64-token tiles:
+// plan() takes the 12-wavefront form when its dispatch ends earlier in these terms. Ratios of the two dispatches and times
+// (8 wavefronts, 12; us; head dim 128), no item cut: 4 prompts around 3,800 x 32 heads 1.45, 533 / 492; 8 ragged prompts to
+// 4,000 1.45, 319 / 300; 7 of 3,500 x 16 heads 1.41, 349 / 330; 8 of 1,900 with a window of 1,023 1.38, 132 / 136. Cut: 5
+// prompts to 2,800 x 8 heads 1.43 in 338 / 460 pieces, 87 / 95; 2 chunks of 1,100 in a window of 511 1.71 in 0 / 200, 36 / 42.
 constexpr double kPfWideTileCost = 1.39;
+constexpr double kPfCutPieceTiles = 0.02;
 constexpr uint32_t kPfMinSplitTiles = 8;        // load balance cuts no piece below this many 64-key tiles
 constexpr uint32_t kAlign = 256;
 constexpr uint32_t kPlanMagic = 0x41504752;     // "RGPA"
@@ -665,6 +667,7 @@ int64_t PrefillMakespan(const ItemList& items, int64_t target, uint32_t cus) {
 struct PieceChoice {
   int64_t target;  // piece size in tiles
   int64_t end;     // the dispatch's finishing time in tiles
+  int64_t cut;     // pieces of cut items
 };
 
 PieceChoice PrefillPieceTiles(const ItemList& items, uint32_t cus) {
@@ -699,7 +702,12 @@ PieceChoice PrefillPieceTiles(const ItemList& items, uint32_t cus) {
       best_end = end;
     }
   }
-  return {best, best_end};
+  int64_t cut = 0;
+  for (const int64_t tiles : items.tiles) {
+    const int64_t n = Pieces(tiles, best);
+    if (n > 1) cut += n * items.heads;
+  }
+  return {best, best_end, cut};
 }
 
 // Calls whose pieces do not fill the CUs once (a short prompt: 1,777 tokens x 2 KV heads made 128 pieces of up to 8
@@ -887,7 +895,7 @@ Layout PlanPrefill(const RoostPagedAttentionParams& p, uint32_t cus, unsigned ch
       if (p.head_dim == kPfWideDim) {
         ItemList wide_list = item_list(kPfWideTokens);
         const PieceChoice wide = PrefillPieceTiles(wide_list, cus);
-        if (wide.end * kPfWideTileCost < narrow.end) {
+        if (wide.end * kPfWideTileCost + wide.cut * kPfCutPieceTiles < narrow.end + narrow.cut * kPfCutPieceTiles) {
           tile_q = kPfWideTokens;
           target = wide.target;
           list = std::move(wide_list);
@@ -1309,7 +1317,8 @@ __global__ void __launch_bounds__(256, kDecodeWgsPerCu)
   // current group's data (vmcnt) while the next group's loads stay in flight.
   constexpr bool kZeroGroup = D <= 128;
   // Absent tokens read the V row of their group's first visible token. A group without any reads kZeroRow, or at head dim
-  // 256, where the registers spill and the further address costs more (16 contexts around 4,000: 203 -> 224 us; 209 as it is), is not computed.
+  // 256, where the registers spill and the further address costs more (16 contexts around 4,000: 203 -> 224 us; 209 as it
+  // is), is not computed.
   auto load = [&](uint32_t gi, uint4* kr, uint4* vr, uint32_t& valid) {
     valid = 0;
     const uint32_t g0 = t_begin + 16u * (wave + waves_per_head * min(gi, nw - 1));

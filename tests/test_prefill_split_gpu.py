@@ -9,7 +9,7 @@ import pytest
 
 import cases
 import roost_amd
-from test_attention_gpu import Dev, torch_reference
+from test_attention_gpu import Dev, from_dev, to_dev, torch, torch_reference
 
 pytestmark = pytest.mark.gpu
 
@@ -45,6 +45,64 @@ def test_wide_items(session, hq, hkv, new, pre, hnd, ps):
     cases.assert_close(got, torch_reference(b), what="wide prefill vs fp32 torch")
 
 
+def _torch_options(b, causal, window, cap):
+    """torch_reference with a window and a soft cap, and the base-2 log-sum-exp beside it."""
+    t = torch()
+    q, k, v = (t.from_numpy(cases.values(x, True).astype(np.float32)).cuda() for x in (b.q, b.k_cache, b.v_cache))
+    out, lse = t.zeros(q.shape, device="cuda"), t.zeros(q.shape[:2], device="cuda")
+    for s in range(b.batch):
+        pages = t.from_numpy(b.kv_indices[b.kv_indptr[s]:b.kv_indptr[s + 1]].astype(np.int64)).cuda()
+        n, rows = int(b.kv_lens[s]), slice(int(b.q_indptr[s]), int(b.q_indptr[s + 1]))
+        ks, vs = (c[pages].reshape(-1, b.hkv, b.d)[:n] for c in (k, v))
+        pos = t.arange(n - (rows.stop - rows.start), n, device="cuda")[:, None]
+        key = t.arange(n, device="cuda")[None, :]
+        hidden = (key > pos) & causal | (key < pos - window) & (window >= 0)
+        for h in range(b.hq):
+            sc = q[rows, h] @ ks[:, h // (b.hq // b.hkv)].T / float(np.sqrt(b.d))
+            if cap:
+                sc = cap * t.tanh(sc / cap)
+            sc = sc.masked_fill(hidden, float("-inf"))
+            out[rows, h] = t.softmax(sc, -1) @ vs[:, h // (b.hq // b.hkv)]
+            lse[rows, h] = t.logsumexp(sc, -1) / float(np.log(2.0))
+    return out.cpu().numpy(), lse.cpu().numpy()
+
+
+@pytest.mark.parametrize("causal,window,cap", [(True, -1, 0.0), (True, 3000, 0.0), (False, -1, 0.0), (True, -1, 3.0)],
+                         ids=["causal", "window", "not causal", "soft cap"])
+def test_wide_items_options(session, causal, window, cap):
+    """The 96-token items with every option, lse and the output gate on, whole items and (a chunk on 20,000 keys) merged
+    ones. The lse bar is that of the other prefill kernels."""
+    rng = np.random.default_rng(7)
+    new, pre = [3901, 3800, 3700, 3600, 300], [0, 0, 64, 5, 20000]
+    b = cases.make_paged_batch(rng, [a + p for a, p in zip(new, pre)], new, hq=32, hkv=8, d=128, std=1.0)
+    dev = Dev(b, causal, with_lse=True, window_left=window, soft_cap=cap)
+    key, params = ("wide options", causal, window, cap), dev.params()
+    session.launch(session.lib.entry(roost_amd.ATTENTION_VARIANT), params, key=key)
+    words = _words(session, key)
+    assert int(words[-1]) == 96 and (int(words[9]) > 0 or window >= 0 or not causal), "no wide items, or none merged"
+    out, lse = _torch_options(b, causal, window, cap)
+    cases.assert_close(dev.result(), out, what="wide prefill vs fp32 torch")
+    assert np.abs(from_dev(dev.lse) - lse).max() < 2e-3
+    plain, gate = dev.out.clone(), to_dev(cases.bf16_bits(rng.standard_normal(b.q.shape).astype(np.float32)), True)
+    roost_amd.sigmoid_mul(session, plain, gate, plain, rows=b.tokens, dim=b.hq * b.d)
+    dev.out.fill_(float("nan"))
+    sm = roost_amd.sigmoid_mul_params(dev.out, gate, dev.out, rows=b.tokens, dim=b.hq * b.d)
+    roost_amd.paged_attention_gated(session, params, sm, key=key)
+    assert np.array_equal(from_dev(dev.out, True), from_dev(plain, True)), "gated differs from attention then SigmoidMul"
+
+
+@pytest.mark.parametrize("hq,hkv,new,pre,window", [(16, 4, [993, 1263], [987, 2501], 511),
+                                                   (8, 2, [2490, 2096, 2803, 1375, 886], [10, 157, 146, 244, 62], -1)])
+def test_wide_form_pays_for_the_pieces_it_cuts(session, hq, hkv, new, pre, window):
+    """Calls whose 96-token items would be cut into more pieces than the 64-token ones, and lose more in partial rows than
+    their tiles gain, take the latter."""
+    rng = np.random.default_rng(sum(new))
+    b = cases.make_paged_batch(rng, [a + p for a, p in zip(new, pre)], new, hq=hq, hkv=hkv, d=128, std=0.5)
+    got, _, _, tokens = _run(session, b, ("narrow", sum(new)), window_left=window)
+    assert tokens == 64
+    cases.assert_close(got, _torch_options(b, True, window, 0.0)[0], what="prefill vs fp32 torch")
+
+
 @pytest.mark.parametrize("hq,hkv,d", [(8, 2, 256), (8, 2, 128), (4, 1, 64)])
 @pytest.mark.parametrize("new,pre", [([500], [0]), ([1025], [0]), ([1777], [0]), ([256], [4001]), ([64], [8000]),
                                      ([129, 2, 1, 300], [0, 640, 900, 33])])
@@ -52,7 +110,10 @@ def test_short_prompts_in_small_pieces(session, hq, hkv, d, new, pre):
     rng = np.random.default_rng(sum(new) + d)
     b = cases.make_paged_batch(rng, [a + p for a, p in zip(new, pre)], new, hq=hq, hkv=hkv, d=d, std=0.5)
     got, items, merges, tokens = _run(session, b, ("sparse", d, sum(new)))
-    assert tokens == 64 and (merges > 0 or d < 256 or len(new) > 1) and items <= 256
+    # Items that pieces of at least 8 tiles would leave are fewer; every one of these calls is cut further.
+    tiles = [-(-(p + min(q + 64, a)) // 64) for a, p in zip(new, pre) if a > 1 for q in range(0, a, 64)]
+    coarse = hkv * sum(-(-x // 8) for x in tiles)
+    assert tokens == 64 and merges > 0 and coarse < items <= 256, (items, coarse, merges)
     cases.assert_close(got, torch_reference(b), what="short prompt vs fp32 torch")
 
 
