@@ -690,7 +690,8 @@ constexpr uint32_t kLayerMaxWidth = 4;
 // columns), with the convolution folded in: per token the workgroup convolves the 288 channels it reads (the key head's
 // 128 q and 128 k channels and its 32 v channels; CausalConv1d's arithmetic: bias, then the taps oldest first with
 // fmaf, SiLU, rounded to bf16) into LDS, then runs RecurrentStep<4> (the recurrent kernel's arithmetic) and writes its
-// 32 output columns as the GDN op rounds them. Sequences sharing a state slot run in batch order, carried by the first one's workgroup, as in RecurrentUnit.
+// 32 output columns as the GDN op rounds them. Sequences sharing a state slot run in batch order, carried by the first
+// one's workgroup, as in RecurrentUnit.
 // Every workgroup reads the old convolution state (the four ops' convolution reads it before its state kernel runs), so
 // the state update and the gated norm run afterwards as their own launches. kW is the convolution's width and CS its
 // state's element type (uint16_t: bf16, or float).
@@ -2134,8 +2135,9 @@ RoostStatus AdmitLayer(const char* op, const RoostCausalConv1dParams& cp, const 
   return ROOST_STATUS_OK;
 }
 
-// Whether a layer call's convolution state update may wait for its last launch (one launch less, 4-5 us): nothing the calls between write lies over what the update reads or writes, and what they and the norm read
-// does not lie over the state. (The norm's output is refused there by AdmitLayer.)
+// Whether a layer call's convolution state update may wait for its last launch (one launch less, 4-5 us): nothing the
+// calls between write lies over what the update reads or writes, and what they and the norm read does not lie over the
+// state. (The norm's output is refused there by AdmitLayer.)
 bool ConvStateMayWait(const RoostCausalConv1dParams& cp, const RoostGatedDeltaRuleParams& p,
                       const RoostGatedRmsNormParams& np) {
   auto apart = [](const RoostDeviceSpan& a, uint64_t a_bytes, const RoostDeviceSpan& b, uint64_t b_bytes) {
@@ -2226,9 +2228,9 @@ extern "C" ROOST_API RoostStatus roost_amd_gdn_decode_layer_run(RoostContext* ct
 // One GDN layer over the recurrent variant for any step (no reference counterpart; the Qwen3.5 worker runs the four
 // ops one after another, Qwen35EagerModel.cs:89-92, and names the recurrent variant for every length): a step whose
 // sequences are all shorter than kRouteMinTokens, with the norm in its single-pass bf16 form, runs as the decode
-// layer (ConvRecurrentKernel, then the norm and the convolution's state); any other step runs the conv op, the recurrent variant with the gates computed where
-// they are read (its longer sequences on the chunk kernels, in `ws`), and the norm op. Either way the results equal
-// the four ops'.
+// layer (ConvRecurrentKernel, then the norm and the convolution's state); any other step runs the convolution, the
+// recurrent variant with the gates computed where they are read (its longer sequences on the chunk kernels, in `ws`), and
+// the norm with the convolution's state update. Either way the results equal the four ops'.
 extern "C" ROOST_API RoostStatus roost_amd_gdn_layer_run(RoostContext* ctx, const void* conv_params,
                                                          const void* gates_params, const void* gdn_params,
                                                          const void* norm_params, const RoostWorkspace* ws,

@@ -338,10 +338,13 @@ constexpr int kSub = 4;        // tokens of a boundary tile requested together
 // kW - 1 row halo per tile, and loads its kV x kW weights once. Narrow vectors (8 bytes for bf16) keep the register
 // count low enough for eight waves per SIMD. Weights, bias, halo and the first rows are requested before the tile's
 // sequence is looked up and unpacked after, as a request that waits for the lookup adds its round trip to the tile's.
-// A tile that crosses a sequence boundary takes its tokens kConvChunk at a time, every state entry they need requested
+// A tile that crosses a sequence boundary takes its tokens kSub at a time, every state entry they need requested
 // before any is used. (Taken token by token, each tap re-read, such a tile cost about 1.4 us a token, which set the time of
 // every batch with a length that is no multiple of the tile: at 32 tokens per tile 4 lengths around 3,940 took 136 us
-// against 79.5 now, 6 x 300 70 against 18, 4 x 40 46 against 9; 4 x 4,096 91 against 83. 6,144 channels, bf16.)
+// against 79.5 now, 6 x 300 70 against 18, 4 x 40 46 against 9. 6,144 channels, bf16.) The short tiles cost traffic: the 3
+// halo rows of 8 are read from memory again (267 MB fetched for 193 MB of rows, 4 lengths around 3,940). Batches of even
+// length gain where the rows come from memory (4 x 4,096 91 -> 83 us) and lose where the last-level cache holds them from
+// a call before (76 -> 79).
 template <typename T, int kW, int kBytes>
 __global__ void __launch_bounds__(256) ConvTileKernel(ConvArgs a, uint32_t cblocks, int32_t tile) {
   constexpr int kWords = kBytes / 4;
