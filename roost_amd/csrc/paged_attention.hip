@@ -438,6 +438,10 @@ DecodeDeal ChooseDeal(const RoostPagedAttentionParams& p, uint32_t cus, const st
   best.per_range = std::max<uint64_t>(1, roost::CeilDiv(total, std::max<uint64_t>(1, std::min(wanted, total))));
   // A row spans at most ceil(groups / per_range) + 1 pieces; keep that within what the merge kernel combines.
   best.per_range = std::max<uint64_t>(best.per_range, roost::CeilDiv(longest, kMaxMergeSplits - 2));
+  // In f32 the kernel spills at head dim 256 and a step takes many times kStepUs: cut row by row, 30 rows of 1,200 keys took
+  // 310 us (even: 122). At 64 and 128 the constants serve: one row of 1,500 13.5 -> 10.5 and 15.8 -> 13.8 us, 8 around 2,000
+  // 19.6 -> 12.0 and 27.4 -> 19.4, a prompt of 100 10.9 -> 7.5 and 14.9 -> 15.0.
+  if (p.q.dtype == ROOST_DTYPE_F32 && p.head_dim == 256) return best;
   if (!may_align || groups.size() > slots || best.per_range > kAlignMost) return best;
   const uint64_t ranges = roost::CeilDiv(total, best.per_range);
   double best_us = cost(ranges * (heads / most), most, best.per_range,

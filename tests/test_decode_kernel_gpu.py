@@ -147,6 +147,18 @@ def test_decode_reads_nothing_that_nobody_wrote(session, hq, hkv, d, bf16, ps, h
         cases.assert_close(got, ref, 1e-5, 1e-5, what="f32 decode")
 
 
+@pytest.mark.parametrize("kv_lens", [[16000], [300, 17, 120, 250], [1200] * 30])
+def test_f32_decode_deal_at_head_dim_256(session, kv_lens):
+    """The f32 kernel spills there and its steps are long: few rows are dealt out evenly all the same."""
+    rng = np.random.default_rng(len(kv_lens))
+    dev = Dev(cases.make_paged_batch(rng, kv_lens, [1] * len(kv_lens), bf16=False))
+    ws = session.prepare(session.lib.entry(roost_amd.ATTENTION_VARIANT), dev.params(), ("f32 deal", len(kv_lens)))
+    words = np.frombuffer(C.string_at(ws.plan, ws.plan_bytes), np.uint64)
+    groups = sum(-(-n // 16) for n in kv_lens)
+    per_range = -(-groups // (2 * torch().cuda.get_device_properties(0).multi_processor_count))
+    assert int(words[5]) >> 32 == 2 and int(words[8]) == -(-groups // per_range)
+
+
 @pytest.mark.parametrize("kv_lens,hq,hkv,d,by_row", [
     ([1500], 8, 2, 256, True), ([2400, 2500, 2600], 8, 2, 256, True), ([3000] * 10, 8, 2, 256, True),
     ([9000], 32, 8, 128, True), ([512 + 120 * i for i in range(64)], 8, 2, 256, False), ([6960] * 17, 8, 2, 256, False),
