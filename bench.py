@@ -690,7 +690,8 @@ def bench_attention_input(torch, roost_amd, session, steps, warmup):
     p = roost_amd.qk_norm_params(q, k, qw, kw, tokens=T, q_heads=HQ, kv_heads=HK, head_dim=D, eps=1e-6)
     timed("qk_norm_8192", roost_amd.QK_NORM_VARIANT, p, 2 * T * (HQ + HK) * D * 2)
     p = roost_amd.rope_params(q, k, pos, tokens=T, q_heads=HQ, kv_heads=HK, head_dim=D, theta=1e7, rotary_dim=64)
-    timed("rope_partial64_8192", roost_amd.ROPE_VARIANT, p, 2 * T * (HQ + HK) * D * 2)
+    # only the rotated 64 of a head's 256 elements are read and written, and a position for each token
+    timed("rope_partial64_8192", roost_amd.ROPE_VARIANT, p, 2 * T * (HQ + HK) * 64 * 2 + T * 4)
     return res
 
 
@@ -933,7 +934,7 @@ def main():
                  "note": "median of 10 launches, each after reading a 512 MiB buffer (evicts the 256 MB MALL)"},
         "roofline": {"bound": "hbm", "achieved": round(dec_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(dec_gbs / HBM_PEAK_GBS, 4), "traffic": measured_traffic(),
-                     "algorithmic_bytes": dec_bytes, "kernel": "DecodeKernel + DecodeMergeKernel (one run())"},
+                     "algorithmic_bytes": dec_bytes, "kernel": "DecodeMfmaKernel + DecodeMergeKernel (one run())"},
         "plan_ms": {"decode": round(dec_plan_ms, 3), "prefill": round(pre_plan_ms, 3)},
         "prefill": {"workload": "BASELINE config 3: 8 seqs, chunk U(256, 2048) on prefix U(0, 6144), causal",
                     "ms": round(pre_ms, 4), "tflops": round(pre_tflops, 1), "peak": MFMA_BF16_PEAK_TFLOPS,
