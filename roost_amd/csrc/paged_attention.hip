@@ -183,7 +183,7 @@ struct Layout {
   uint64_t merges_two = 0;  // prefill: leading merge entries of two pieces
   uint32_t item_tokens = kPfTokens;  // prefill: query tokens per work item
   uint64_t splits_bf16 = 0;          // prefill: leading partial slots in bf16
-  uint32_t overlap = 0;     // prefill: tile and decode kernels on two streams (ChooseOverlap)
+  uint32_t overlap = 0;     // prefill: tile pieces and decode ranges side by side in one launch (ChooseOverlap)
   uint64_t range_offset = 0;
   uint64_t merge_offset = 0;
   uint64_t counter_offset = 0;
@@ -1739,8 +1739,9 @@ __global__ void __launch_bounds__(256, kDecodeWgsPerCu)
   __shared__ float m_lds[4][NH];
   __shared__ float l_lds[4][NH];
   __shared__ __attribute__((aligned(16))) float o_lds[4][NH][D];
-  DecodeMfmaBody<D, NH, kFastPage, 4>(q, out, lse, kv, kv_indices, work, range_ptr, part_o, part_ml, q_rows, q_heads, heads_per_wg,
-                           scale_log2, window, causal, cap, blockIdx.x, &m_lds[0][0], &l_lds[0][0], &o_lds[0][0][0]);
+  DecodeMfmaBody<D, NH, kFastPage, 4>(q, out, lse, kv, kv_indices, work, range_ptr, part_o, part_ml, q_rows, q_heads,
+                                      heads_per_wg, scale_log2, window, causal, cap, blockIdx.x, &m_lds[0][0],
+                                      &l_lds[0][0], &o_lds[0][0][0]);
 }
 
 // Combines the pieces of each split sequence: one workgroup per (sequence, query head) of D threads, four slices of D / 4
@@ -2148,8 +2149,8 @@ __device__ __forceinline__ void PrefillTileBody(const uint16_t* __restrict__ q, 
                                                 const int32_t* __restrict__ q_indptr,
                                                 const PrefillWork* __restrict__ work, uint16_t* __restrict__ part_o,
                                                 float* __restrict__ part_ml, uint32_t splits_bf16, uint32_t q_heads,
-                                                uint32_t causal, uint32_t ps_shift, float scale_log2, int32_t window, SoftCap cap,
-                                                uint32_t item, unsigned char (*tiles)[2][kPfTileBytes<D>]) {
+                                                uint32_t causal, uint32_t ps_shift, float scale_log2, int32_t window,
+                                                SoftCap cap, uint32_t item, unsigned char (*tiles)[2][kPfTileBytes<D>]) {
   static_assert(D == 64 || D == 128 || D == 256, "the tile kernel is built for head dims 64, 128 and 256");
   constexpr int kRowB = 2 * D;                  // bytes of one K or V row in LDS
   constexpr int kPieces = D / 8;                // 16-byte pieces per row
@@ -2792,8 +2793,8 @@ RoostStatus LaunchMixed(const RoostPagedAttentionParams& p, const PlanRecord& re
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, q16, outp, lsep, kv, kv.kv_indices, q_indptr, items,
                        PrefillPartO(p, rec, dev), PrefillPartMl(p, rec, dev), static_cast<uint32_t>(rec.splits_bf16),
-                       p.q_heads, p.causal, ps_shift, scale_log2, WindowOf(p), raw, n_items, dec_items, dec_ranges, dec_o, dec_ml, hpw, dkv.vheads,
-                       dkv.head_shift, cap);
+                       p.q_heads, p.causal, ps_shift, scale_log2, WindowOf(p), raw, n_items,
+                       dec_items, dec_ranges, dec_o, dec_ml, hpw, dkv.vheads, dkv.head_shift, cap);
   };
   auto of_group = [&](auto d, auto capped_c) {
     constexpr int kD = decltype(d)::value;
@@ -2918,8 +2919,8 @@ PlanRecord MakeRecord(const RoostPagedAttentionParams& p, const Layout& l) {
 bool RecordFits(const PlanRecord& r, const RoostPagedAttentionParams& p) {
   const bool dtype = r.dtype == p.q.dtype || (r.dtype == ROOST_DTYPE_UNDEFINED &&
                                               (p.mode == ROOST_ATTENTION_DECODE || p.q.dtype == ROOST_DTYPE_BF16));
-  return dtype && r.q_heads == p.q_heads && r.mode == p.mode && r.batch == p.batch && r.tokens == p.tokens && r.page_size == p.page_size &&
-         r.kv_layout == p.kv_layout && r.head_dim == p.head_dim && r.kv_heads == p.kv_heads && r.window == WindowOf(p);
+  return dtype && r.q_heads == p.q_heads && r.mode == p.mode && r.batch == p.batch && r.tokens == p.tokens &&
+         r.page_size == p.page_size && r.kv_layout == p.kv_layout && r.head_dim == p.head_dim && r.kv_heads == p.kv_heads && r.window == WindowOf(p);
 }
 
 }  // namespace
